@@ -159,6 +159,35 @@ __device__ __forceinline__ void otx_exp_n(float (&v)[N], const double* tab) {
   }
 }
 
+// v[j] = exp(v[j]) correctly rounded, in place, for arguments of either sign
+// (NaN is not carried through: see otx_exp_any_t), stage by stage like otx_exp_n.
+template <int N>
+__device__ __forceinline__ void otx_exp_any_n(float (&v)[N], const double* tab) {
+  double xd[N], d[N], tv[N];
+  uint32_t kb[N];
+#pragma unroll
+  for (int j = 0; j < N; j++) d[j] = otx_exp_any_t(v[j], &xd[j]);
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    kb[j] = (uint32_t)otx_d2u(d[j]);
+    tv[j] = *reinterpret_cast<const double*>(reinterpret_cast<const unsigned char*>(tab) + otx_tab_off(kb[j]));
+  }
+#pragma unroll
+  for (int j = 0; j < N; j++) v[j] = otx_exp_le0_y(otx_exp_le0_p(otx_exp_le0_r(d[j], xd[j])), tv[j], kb[j]);
+}
+
+// 1/d to about one unit of binary64 for d >= 1 (NaN for d = inf): the hardware
+// reciprocal (about 24 bits) and two Newton steps, six instructions where the
+// correctly rounded binary64 division takes a dozen more.  RN32(RN64(a * r)) is
+// the correctly rounded a/d in the normal range for any r within 2^-51 of 1/d
+// (the argument of otx_div_by_recip).
+__device__ __forceinline__ double otx_recip64_newton(float d) {
+  const double dd = (double)d;
+  double r = __builtin_amdgcn_rcp(dd);
+  r = __builtin_fma(__builtin_fma(-dd, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-dd, r, 1.0), r, r);
+}
+
 __device__ __forceinline__ float otx_exp1(float x, const double* tab) {
   float v[1] = {x};
   otx_exp_n<1>(v, tab);

@@ -366,6 +366,21 @@ OTX_HD float otx_exp_le0_y(double p, double tvb, uint32_t kb) {
   return (float)(scaled * p);
 }
 
+// The same evaluation for arguments of either sign: x is clamped to [-104, 89]
+// instead (exp(89) is above the binary32 range, so the last rounding gives +inf
+// from 88.73 on).  The binary32 rounding of y is the correctly rounded exp(x)
+// for every binary32 x >= 0 too, established like the other half by enumerating
+// all of them; |k| stays below 2^16, so the first fma of the reduction is still
+// exact.  NaN is mapped to an end of the range: callers carry it through x.
+OTX_HD double otx_exp_any_t(float x, double* xd) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  *xd = (double)__builtin_amdgcn_fmed3f(x, -104.0f, 89.0f);
+#else
+  *xd = (double)(x < -104.0f ? -104.0f : (x > 89.0f ? 89.0f : x));
+#endif
+  return __builtin_fma(*xd, 0x1.71547652b82fep+8, 0x1.8p52);
+}
+
 OTX_HD double otx_exp_le0_reduce(float x, const double* tab, double* tvb, uint32_t* kb) {
   double xd;
   const double t = otx_exp_le0_t(x, &xd);
@@ -384,6 +399,14 @@ OTX_HD float otx_expf_fast_le0(float x, const double* tab) {
   uint32_t kb;
   const double r = otx_exp_le0_reduce(x, tab, &tvb, &kb);
   return otx_exp_le0_finish(r, tvb, kb);
+}
+
+// Correctly rounded exp of any binary32 x but NaN through the same table.
+OTX_HD float otx_expf_fast_any(float x, const double* tab) {
+  double xd;
+  const double t = otx_exp_any_t(x, &xd);
+  const uint32_t kb = (uint32_t)otx_d2u(t);
+  return otx_exp_le0_y(otx_exp_le0_p(otx_exp_le0_r(t, xd)), tab[kb & 255u], kb);
 }
 
 // Correctly rounded binary32 1/sqrt(x) (RMSNorm's rstd).  The binary64

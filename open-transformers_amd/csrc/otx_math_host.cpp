@@ -61,6 +61,19 @@ extern "C" void otx_host_exp_paths_check(uint64_t lo, uint64_t count, uint64_t* 
   out[0] = bf; out[1] = sf; out[2] = bl; out[3] = nl;
 }
 
+// otx_expf_fast_any over the bit patterns [lo, lo + count), NaN left out: the
+// number of inputs whose result is not the correctly rounded exp.
+extern "C" uint64_t otx_host_exp_any_check(uint64_t lo, uint64_t count) {
+  uint64_t bad = 0;
+#pragma omp parallel for schedule(dynamic, 65536) reduction(+ : bad) num_threads(omp_get_num_procs())
+  for (int64_t i = 0; i < (int64_t)count; i++) {
+    const float x = otx_u2f((uint32_t)(lo + (uint64_t)i));
+    if (x != x) continue;
+    if (otx_f2u(otx_expf_fast_any(x, tab256b.v)) != otx_f2u(x > 89.0f ? otx_expf(x) : exp_ref(x))) bad++;
+  }
+  return bad;
+}
+
 extern "C" float otx_host_rsqrtf(float x) { return otx_rsqrtf(x); }
 
 extern "C" float otx_host_div_by_recip(float a, float b) { return otx_div_by_recip(a, otx_recip64(b)); }

@@ -209,6 +209,17 @@ def test_kernel_exp_paths_exhaustive():
     assert bad_l == 0 and n_l == 1  # +0 (exp(0) = 1)
 
 
+def test_exp_of_either_sign_exhaustive():
+    """otx_expf_fast_any (SiLU's exp(-x): the softmax table and polynomial with the
+    argument clamped to [-104, 89]) equals the correctly rounded exp on every
+    binary32 input but NaN: overflow to +inf, the eight hard-to-round inputs and the
+    infinities included."""
+    host = _host_math()
+    host.otx_host_exp_any_check.restype = ctypes.c_uint64
+    host.otx_host_exp_any_check.argtypes = [ctypes.c_uint64, ctypes.c_uint64]
+    assert host.otx_host_exp_any_check(0, 1 << 32) == 0
+
+
 def test_log_rsqrt_tables_complete_exhaustive():
     """otx_logf (LSE) and otx_rsqrtf (RMSNorm's rstd) on every finite positive
     binary32 input: wherever the binary64 evaluation leaves the binary32
