@@ -55,3 +55,43 @@ def test_embedding_out_of_range_ids():
     assert torch.isnan(o[0, 1]).all() and torch.isnan(o[0, 2]).all() and not torch.isnan(o[0, 0]).any()
     gw = w.grad.float().cpu()
     assert (gw[3] == 2.0).all() and (gw[torch.arange(16) != 3] == 0).all()
+
+
+@pytest.mark.parametrize("npos,V,D,bf16,distinct,shift", [
+    (1, 1, 8, True, 1, 0),          # one position, one row
+    (64, 7, 2048, True, 2, 0),      # a wave of positions; 32-row segments
+    (65, 300, 2056, True, 300, 1),  # two column blocks; an unaligned gradient
+    (1024, 5, 64, False, 5, 0),     # one round of the LDS sort, segments over the 16-row batch
+    (1025, 5, 1028, False, 4, 1),   # one position past it
+    (257, 9, 128, True, 1, 0),      # one segment past the 256-position list
+    (16384, 262143, 16, True, 262143, 0),  # the largest LDS sort: 14 bits of position, 18 of id
+    (16384, 262144, 16, True, 262144, 0),  # an id bit more: the device-wide sort
+    (16385, 1000, 16, False, 1000, 0),     # a position more: the device-wide sort
+])
+def test_embedding_backward_edges(npos, V, D, bf16, distinct, shift):
+    """Sizes at the edges of the sorts, the position lists and the column blocks, ids outside the vocabulary among
+    them, through the C ABI (the gradient ``shift`` elements past an aligned address)."""
+    from open_transformers_amd import _lib
+
+    print(f"embedding backward npos={npos} V={V} D={D} bf16={bf16} distinct={distinct} shift={shift}", flush=True)
+    rng = np.random.default_rng(npos * 31 + V)
+    ids = rng.integers(0, distinct, npos).astype(np.int64)
+    if npos > 8:
+        ids[rng.integers(0, npos, 3)] = [-1, V, V + 5]
+    g = rng.standard_normal((npos, D)).astype(np.float32)
+    if bf16:
+        g = synthetic.round_to_bf16(g)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    buf = torch.zeros(npos * D + 8, dtype=dt, device=DEV)
+    buf[shift:shift + npos * D] = torch.from_numpy(g).reshape(-1).to(dt).to(DEV)
+    gw = torch.full((V, D), 7.0, dtype=dt, device=DEV)
+    it = torch.from_numpy(ids).to(DEV)
+    lib = _lib.load()
+    n = int(lib.otx_embedding_bwd_workspace_bytes(npos, V))
+    ws = torch.empty(n + 256, dtype=torch.uint8, device=DEV)
+    _lib.check(lib.otx_embedding_bwd(it.data_ptr(), buf.data_ptr() + shift * buf.element_size(), gw.data_ptr(), npos, V,
+                                     D, _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_F32, (ws.data_ptr() + 255) & ~255, n,
+                                     torch.cuda.current_stream().cuda_stream), "otx_embedding_bwd")
+    torch.cuda.synchronize()
+    ref = orc.embedding_bwd(ids, g, V, out_bf16=bf16)
+    assert_bits_equal(gw.float().cpu().numpy(), ref, "weight gradient")
