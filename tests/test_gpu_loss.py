@@ -118,3 +118,57 @@ def test_open1b_lm_head_shape():
     rows = slice(4000, 4064)
     g_r = orc.ce_zloss_bwd(x[rows], lab[rows], st_r[:, rows], 1e-4, n_total=N, nthreads=16)
     assert_bits_equal(logits.grad[rows].float().cpu().numpy(), g_r, "logit gradient rows 4000..4063")
+
+
+def _edge_rows(x, rng):
+    """Rows that leave the window of the table form: zeros, subnormals, infinities, NaN, huge and tiny values, a row
+    without a positive value, one of -inf alone, one of equal values."""
+    V = x.shape[1]
+    x[1, ::7] = 0.0
+    x[2, V // 2] = -0.0
+    x[3] *= 2.0 ** -20
+    x[4] = -np.abs(x[4]) - 2.0 ** -10
+    x[5, 5], x[5, V - 1] = np.inf, 300.0
+    x[6, rng.integers(0, V, 3)] = -np.inf
+    x[7, V - 2] = np.nan
+    x[8] = -np.inf
+    x[9] = 1.5
+    x[10, :40] = 1e-40
+    x[11] = rng.standard_normal(V) * 400
+    x[12] = -0.0
+    return x
+
+
+@pytest.mark.parametrize("N,V,dtype", [
+    (300, 16384, "bf16"),  # the table form's shortest row; more rows than CUs
+    (17, 16408, "bf16"),   # a last chunk of 24
+    (14, 131072, "bf16"),  # the longest row
+    (17, 16376, "bf16"),   # just under the table form
+    (17, 20001, "bf16"),   # unaligned rows, sixteen waves
+    (15, 2048, "f32"),     # one wave per row, whole tiles
+    (15, 2049, "bf16"),    # four waves, one logit past a tile
+    (15, 16388, "f32"),    # sixteen waves
+    (33000, 40, "f32"),    # more rows than workgroups
+])
+def test_loss_forms_and_edge_rows(N, V, dtype):
+    """Every form of the kernels at the edges of its range, with rows that hold values outside the table's window:
+    statistics, scalars and gradient against the oracle (NaN where the oracle has NaN)."""
+    from attn_util import assert_bits_equal_nan_class as eq
+
+    print(f"loss forms N={N} V={V} {dtype}", flush=True)
+    x, lab = _inputs(N, V, dtype, seed=N + V, scale=2.0)
+    x = _edge_rows(x, np.random.default_rng(V))
+    if dtype == "bf16":
+        x = synthetic.round_to_bf16(x)
+    lab[5], lab[7] = 5, V - 2
+    labels = torch.from_numpy(lab).to(DEV)
+    logits = _gpu(x, dtype)
+    with np.errstate(all="ignore"):
+        ce_r, z_r, st_r = orc.ce_zloss_fwd(x, lab, 1e-4, nthreads=8)
+        g_r = orc.ce_zloss_bwd(x, lab, st_r, 1e-4, gce=2.0, gz=3.0, out_bf16=dtype == "bf16", nthreads=8)
+    ce, z, st = L.ce_zloss_forward(logits, labels, 1e-4)
+    g = L.ce_zloss_backward(logits, labels, st, torch.tensor(2.0, device=DEV), torch.tensor(3.0, device=DEV), 1e-4)
+    torch.cuda.synchronize()
+    eq(st.cpu().numpy(), st_r, "row statistics")
+    eq(np.array([ce.item(), z.item()], np.float32), np.array([ce_r, z_r], np.float32), "ce, z")
+    eq(g.float().cpu().numpy(), g_r, "logit gradient")
