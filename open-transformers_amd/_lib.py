@@ -9,10 +9,11 @@ library is an error, never a silent fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import json
 import pathlib
 
-from .build import LIB_NAME, PKG_DIR
+from .build import AUTOGRAD_LIB, LIB_NAME, PKG_DIR
 
 OTX_OK = 0
 OTX_EINVAL = 1
@@ -22,6 +23,7 @@ DTYPE_BF16 = 1
 NOALLOC_SCRATCH_BYTES = 32 << 20  # OTX_NOALLOC_SCRATCH_BYTES of include/otx_attn.h
 
 _LIB = None
+_AUTOGRAD = None
 
 _vp = ctypes.c_void_p
 _i = ctypes.c_int
@@ -96,6 +98,22 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
     _LIB = lib
     return lib
+
+
+def autograd():
+    """The native autograd nodes (csrc/otx_autograd.cpp), imported once; raises
+    RuntimeError if they have not been built."""
+    global _AUTOGRAD
+    if _AUTOGRAD is None:
+        load()
+        path = PKG_DIR / AUTOGRAD_LIB
+        if not path.exists():
+            raise RuntimeError(f"{path} is missing: run `python -c 'import __graft_entry__ as g; g.build()'` first")
+        spec = importlib.util.spec_from_file_location("_otx_autograd", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _AUTOGRAD = mod
+    return _AUTOGRAD
 
 
 def check(rc: int, what: str) -> None:

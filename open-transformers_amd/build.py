@@ -164,6 +164,30 @@ def build(verbose: bool = False) -> pathlib.Path:
     if verbose:
         print(out, tree_stamp(), sources_digest())
     build_host_math()
+    build_autograd()
+    return out
+
+
+AUTOGRAD_LIB = "_otx_autograd.so"
+
+
+def build_autograd() -> pathlib.Path:
+    """The autograd nodes of the Python operators (csrc/otx_autograd.cpp): host code
+    against torch's C++ API, linked with the libotx_attn.so beside it."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    out = PKG_DIR / AUTOGRAD_LIB
+    tmp = out.with_suffix(".so.tmp")
+    cxx = shutil.which("g++") or "g++"
+    includes = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"]]
+    _run([cxx, "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-DTORCH_API_INCLUDE_EXTENSION_H", f"-I{INCLUDE}", *(f"-isystem{p}" for p in includes),
+          str(CSRC / "otx_autograd.cpp"), "-o", str(tmp), f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN",
+          *(f"-L{p}" for p in cpp_extension.library_paths("cuda")), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch",
+          "-ltorch_python"])
+    os.replace(tmp, out)
     return out
 
 

@@ -1,0 +1,371 @@
+// The operators' autograd nodes, over the C ABI of include/otx_attn.h.
+//
+// Each node is one of the operators of nn/ (which check their arguments first):
+// it allocates outputs and workspaces, launches on the current stream and saves what
+// its backward reads.  Native because a pass over small tensors is bound by the host: a
+// Python node's backward runs on the engine's device thread, where the interpreter and
+// the foreign-function calls cost several times what the launches do.  Measured on one
+// host (issue time of one forward and backward, Python nodes against these): linear 113
+// against 33 us, RMSNorm 112 / 39, attention 146 / 46, SwiGLU 81 / 25, the loss 143 / 47,
+// the embedding 117 / 29.
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/extension.h>
+
+#include "otx_attn.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+
+void check(int rc, const char* what) {
+  if (rc == OTX_OK) return;
+  TORCH_CHECK_VALUE(rc != OTX_EINVAL, what, ": ", otx_last_error());
+  TORCH_CHECK(false, what, ": ", otx_last_error());
+}
+
+int dtype_code(const Tensor& t) {
+  TORCH_CHECK_VALUE(t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat, "dtype ", t.scalar_type(),
+                    " not supported (bfloat16 or float32)");
+  return t.scalar_type() == at::kBFloat16 ? OTX_DTYPE_BF16 : OTX_DTYPE_F32;
+}
+
+// The stream that work on t's device is queued on, with that device made current.
+struct Launch {
+  c10::DeviceGuard guard;
+  void* stream;
+  explicit Launch(const Tensor& t)
+      : guard(t.device()), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+};
+
+// nbytes of device memory at a 256-byte aligned address.
+struct Workspace {
+  Tensor mem;
+  void* ptr;
+  Workspace(const Tensor& like, size_t nbytes)
+      : mem(at::empty({(int64_t)nbytes + 256}, like.options().dtype(at::kByte))),
+        ptr((void*)(((uintptr_t)mem.data_ptr() + 255) & ~(uintptr_t)255)) {}
+};
+
+// C[M, N] = serial fold over r of A(i, r) * B(j, r), bf16 (strides in elements).
+Tensor gemm(const Tensor& a, long a_i, long a_r, const Tensor& b, long b_j, long b_r, int64_t M, int64_t N, int64_t R) {
+  TORCH_CHECK_VALUE(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16,
+                    "gemm_bf16 takes bfloat16 operands");
+  TORCH_CHECK_VALUE(M <= INT_MAX && N <= INT_MAX && R <= INT_MAX, "GEMM shape ", M, " x ", N, " x ", R, " too large");
+  Tensor c = at::empty({M, N}, a.options());
+  Launch at(a);
+  check(otx_gemm_bf16(a.data_ptr(), a_i, a_r, b.data_ptr(), b_j, b_r, c.data_ptr(), N, (int)M, (int)N, (int)R,
+                      OTX_DTYPE_BF16, at.stream),
+        "otx_gemm_bf16");
+  return c;
+}
+
+struct Linear : Function<Linear> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+    const int64_t K = x.size(-1), N = w.size(0);
+    const Tensor x2 = x.reshape({-1, K}).contiguous(), wc = w.contiguous();
+    const Tensor y = gemm(x2, K, 1, wc, K, 1, x2.size(0), N, K);  // y = x w^T
+    ctx->save_for_backward({x2, wc});
+    std::vector<int64_t> shape = x.sizes().vec();
+    ctx->saved_data["shape"] = shape;
+    shape.back() = N;
+    return y.view(shape);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w = saved[1];
+    const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+    const Tensor dy = grads[0].reshape({M, N}).contiguous();
+    Tensor dx, dw;
+    if (ctx->needs_input_grad(0))  // dx[m][k] = sum_n dy[m][n] w[n][k]
+      dx = gemm(dy, N, 1, w, 1, K, M, K, N).view(ctx->saved_data["shape"].toIntVector());
+    if (ctx->needs_input_grad(1))  // dw[n][k] = sum_m dy[m][n] x[m][k]
+      dw = gemm(dy, 1, N, x, 1, K, N, K, M);
+    return {dx, dw};
+  }
+};
+
+struct RMSNorm : Function<RMSNorm> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
+    const int64_t D = x.size(-1);
+    const Tensor xc = x.contiguous(), wc = w.to(x.scalar_type()).contiguous();
+    const int64_t rows = xc.numel() / D;
+    const Tensor y = at::empty_like(xc), rstd = at::empty({rows}, x.options().dtype(at::kFloat));
+    {
+      Launch at(x);
+      check(otx_rmsnorm_fwd(xc.data_ptr(), wc.data_ptr(), y.data_ptr(), rstd.data_ptr<float>(), rows, (int)D,
+                            (float)eps, dtype_code(x), at.stream),
+            "otx_rmsnorm_fwd");
+    }
+    ctx->save_for_backward({xc, wc, rstd});
+    ctx->saved_data["wdtype"] = (int64_t)w.scalar_type();
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w = saved[1], &rstd = saved[2];
+    const int64_t D = x.size(-1), rows = x.numel() / D;
+    const Tensor dy = grads[0].contiguous();
+    const Tensor dx = at::empty_like(x), dw = at::empty({D}, x.options().dtype(at::kFloat));
+    {
+      Launch at(x);
+      const size_t nbytes = otx_rmsnorm_bwd_workspace_bytes(rows, (int)D);
+      const Workspace ws(x, nbytes);
+      check(otx_rmsnorm_bwd(x.data_ptr(), w.data_ptr(), rstd.data_ptr<float>(), dy.data_ptr(), dx.data_ptr(),
+                            dw.data_ptr<float>(), rows, (int)D, dtype_code(x), ws.ptr, nbytes, at.stream),
+            "otx_rmsnorm_bwd");
+    }
+    return {dx, dw.to((at::ScalarType)ctx->saved_data["wdtype"].toInt()), Tensor()};
+  }
+};
+
+struct SiLU : Function<SiLU> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x) {
+    const Tensor xc = x.contiguous(), y = at::empty_like(xc);
+    Launch at(x);
+    check(otx_silu_fwd(xc.data_ptr(), y.data_ptr(), xc.numel(), dtype_code(x), at.stream), "otx_silu_fwd");
+    ctx->save_for_backward({xc});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const Tensor x = ctx->get_saved_variables()[0], dy = grads[0].contiguous(), dx = at::empty_like(x);
+    Launch at(x);
+    check(otx_silu_bwd(x.data_ptr(), dy.data_ptr(), dx.data_ptr(), x.numel(), dtype_code(x), at.stream),
+          "otx_silu_bwd");
+    return {dx};
+  }
+};
+
+struct SwiGLU : Function<SwiGLU> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& gu) {
+    const int64_t F = gu.size(-1) / 2;
+    const Tensor guc = gu.contiguous();
+    std::vector<int64_t> shape = gu.sizes().vec();
+    shape.back() = F;
+    const Tensor h = at::empty(shape, gu.options());
+    Launch at(gu);
+    check(otx_swiglu_fwd(guc.data_ptr(), h.data_ptr(), guc.numel() / (2 * F), (int)F, dtype_code(gu), at.stream),
+          "otx_swiglu_fwd");
+    ctx->save_for_backward({guc});
+    return h;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const Tensor gu = ctx->get_saved_variables()[0], dh = grads[0].contiguous(), dgu = at::empty_like(gu);
+    const int64_t F = gu.size(-1) / 2;
+    Launch at(gu);
+    check(otx_swiglu_bwd(gu.data_ptr(), dh.data_ptr(), dgu.data_ptr(), gu.numel() / (2 * F), (int)F, dtype_code(gu),
+                         at.stream),
+          "otx_swiglu_bwd");
+    return {dgu};
+  }
+};
+
+struct RopeHeads : Function<RopeHeads> {  // [B, T, H, D] -> [B, H, T, D]
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& cos, const Tensor& sin) {
+    const int64_t B = x.size(0), T = x.size(1), H = x.size(2), D = x.size(3);
+    const Tensor xc = x.contiguous(), y = at::empty({B, H, T, D}, x.options());
+    Launch at(x);
+    check(otx_rope_heads_fwd(xc.data_ptr(), cos.data_ptr<float>(), sin.data_ptr<float>(), y.data_ptr(), (int)B, (int)T,
+                             (int)H, (int)D, dtype_code(x), at.stream),
+          "otx_rope_heads_fwd");
+    ctx->save_for_backward({cos, sin});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor dy = grads[0].contiguous();
+    const int64_t B = dy.size(0), H = dy.size(1), T = dy.size(2), D = dy.size(3);
+    const Tensor dx = at::empty({B, T, H, D}, dy.options());
+    Launch at(dy);
+    check(otx_rope_heads_bwd(dy.data_ptr(), saved[0].data_ptr<float>(), saved[1].data_ptr<float>(), dx.data_ptr(),
+                             (int)B, (int)T, (int)H, (int)D, dtype_code(dy), at.stream),
+          "otx_rope_heads_bwd");
+    return {dx, Tensor(), Tensor()};
+  }
+};
+
+Tensor swap12(const Tensor& x) {
+  const Tensor xc = x.contiguous(), y = at::empty({x.size(0), x.size(2), x.size(1), x.size(3)}, x.options());
+  Launch at(x);
+  check(otx_swap_heads(xc.data_ptr(), y.data_ptr(), (int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3),
+                       dtype_code(x), at.stream),
+        "otx_swap_heads");
+  return y;
+}
+
+struct SwapHeads : Function<SwapHeads> {  // [B, X, Y, D] -> [B, Y, X, D]
+  static Tensor forward(AutogradContext*, const Tensor& x) { return swap12(x); }
+  static variable_list backward(AutogradContext*, variable_list grads) { return {swap12(grads[0])}; }
+};
+
+struct Embedding : Function<Embedding> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& ids, const Tensor& weight) {
+    const Tensor flat = ids.reshape({-1}).to(at::kLong).contiguous();
+    const int64_t V = weight.size(0), D = weight.size(1), n = flat.numel();
+    const Tensor out = at::empty({n, D}, weight.options());
+    {
+      Launch at(weight);
+      check(otx_embedding_fwd(flat.data_ptr<int64_t>(), weight.data_ptr(), out.data_ptr(), n, (int)V, (int)D,
+                              dtype_code(weight), at.stream),
+            "otx_embedding_fwd");
+    }
+    ctx->save_for_backward({flat});
+    ctx->saved_data["V"] = V;
+    ctx->saved_data["D"] = D;
+    ctx->saved_data["dtype"] = (int64_t)weight.scalar_type();
+    std::vector<int64_t> shape = ids.sizes().vec();
+    shape.push_back(D);
+    return out.view(shape);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const Tensor flat = ctx->get_saved_variables()[0];
+    const int64_t V = ctx->saved_data["V"].toInt(), D = ctx->saved_data["D"].toInt(), n = flat.numel();
+    TORCH_CHECK(grads[0].device() == flat.device(), "grad_output is on ", grads[0].device(), " but the ids are on ",
+                flat.device());
+    const Tensor g = grads[0].reshape({-1, D}).to((at::ScalarType)ctx->saved_data["dtype"].toInt()).contiguous();
+    const Tensor gw = at::empty({V, D}, g.options());
+    Launch at(g);
+    const size_t nbytes = otx_embedding_bwd_workspace_bytes(n, (int)V);
+    const Workspace ws(g, nbytes);
+    check(otx_embedding_bwd(flat.data_ptr<int64_t>(), g.data_ptr(), gw.data_ptr(), n, (int)V, (int)D, dtype_code(g),
+                            ws.ptr, nbytes, at.stream),
+          "otx_embedding_bwd");
+    return {Tensor(), gw};
+  }
+};
+
+struct Loss : Function<Loss> {  // logits [N, V], labels [N] -> (ce, z)
+  static variable_list forward(AutogradContext* ctx, const Tensor& logits, const Tensor& labels, double coeff) {
+    const Tensor x = logits.contiguous(), lab = labels.contiguous();
+    const int64_t N = x.size(0), V = x.size(1);
+    TORCH_CHECK_VALUE(V <= INT_MAX, "vocabulary ", V, " too large");
+    const auto f32 = x.options().dtype(at::kFloat);
+    const Tensor stats = at::empty({5, N}, f32), loss = at::empty({2}, f32);
+    {
+      Launch at(x);
+      check(otx_ce_zloss_fwd(x.data_ptr(), lab.data_ptr<int64_t>(), N, (int)V, dtype_code(x), coeff,
+                             stats.data_ptr<float>(), loss.data_ptr<float>(), at.stream),
+            "otx_ce_zloss_fwd");
+    }
+    ctx->save_for_backward({logits, labels, stats});
+    ctx->saved_data["coeff"] = coeff;
+    return {loss.select(0, 0), loss.select(0, 1)};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor x = saved[0].contiguous(), lab = saved[1].contiguous();
+    const Tensor g = at::stack({grads[0].reshape({}).to(at::kFloat), grads[1].reshape({}).to(at::kFloat)});
+    const Tensor dx = at::empty_like(x);
+    Launch at(x);
+    check(otx_ce_zloss_bwd(x.data_ptr(), lab.data_ptr<int64_t>(), saved[2].data_ptr<float>(), g.data_ptr<float>(),
+                           x.size(0), (int)x.size(1), dtype_code(x), ctx->saved_data["coeff"].toDouble(), dx.data_ptr(),
+                           at.stream),
+          "otx_ce_zloss_bwd");
+    return {dx, Tensor(), Tensor()};
+  }
+};
+
+// q [B, H, S, D], k and v [B, Hkv, S, D], checked and contiguous; sc: the score cache
+// to fill for the backward, or none.  int8pv: the int8-PV forward, whose backward is the
+// same binary32 one (straight-through).
+struct Attention : Function<Attention> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
+                        const std::optional<Tensor>& sc, int64_t window, bool int8pv) {
+    const int B = (int)q.size(0), H = (int)q.size(1), Hkv = (int)k.size(1), S = (int)q.size(2), D = (int)q.size(3);
+    const Tensor o = at::empty_like(q), lse = at::empty({B, H, S}, q.options().dtype(at::kFloat));
+    {
+      Launch at(q);
+      const int dt = dtype_code(q), w = (int)window;
+      float* l = lse.data_ptr<float>();
+      float* c = sc ? sc->data_ptr<float>() : nullptr;
+      const size_t nc = sc ? (size_t)sc->numel() * 4 : 0;
+      if (int8pv) {
+        const size_t nbytes = otx_attn_fwd_int8pv_workspace_bytes(B, H, Hkv, S, D);
+        const Workspace ws(q, nbytes);
+        check(sc ? otx_attn_fwd_int8pv_sc(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), l, c, nc, B, H, Hkv,
+                                          S, D, w, dt, ws.ptr, nbytes, 0, at.stream)
+                 : otx_attn_fwd_int8pv(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), l, B, H, Hkv, S, D, w,
+                                       dt, ws.ptr, nbytes, at.stream),
+              "otx_attn_fwd_int8pv");
+      } else {
+        check(sc ? otx_attn_fwd_sc(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), l, c, nc, B, H, Hkv, S, D, w,
+                                   dt, 0, at.stream)
+                 : otx_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), l, B, H, Hkv, S, D, w, dt,
+                                at.stream),
+              "otx_attn_fwd");
+      }
+    }
+    // in the order of the Python node of nn/flash_attention.py, whose first checkpointed
+    // forward this one may be the recompute of
+    variable_list save = {q, k, v, o, lse};
+    if (sc) save.push_back(*sc);
+    ctx->save_for_backward(save);
+    ctx->saved_data["window"] = window;
+    return o;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor q = saved[0].contiguous(), k = saved[1].contiguous(), v = saved[2].contiguous(),
+                 o = saved[3].contiguous(), lse = saved[4].contiguous(), dout = grads[0].contiguous();
+    const int B = (int)q.size(0), H = (int)q.size(1), Hkv = (int)k.size(1), S = (int)q.size(2), D = (int)q.size(3);
+    const int w = (int)ctx->saved_data["window"].toInt(), dt = dtype_code(q);
+    for (const Tensor& t : {k, v, o, dout})
+      TORCH_CHECK_VALUE(t.device() == q.device() && t.scalar_type() == q.scalar_type(),
+                        "saved tensors and grad_output must match q in dtype and device");
+    TORCH_CHECK_VALUE(dout.sizes() == q.sizes() && o.sizes() == q.sizes(), "o and grad_output must match q in shape");
+    TORCH_CHECK_VALUE(lse.device() == q.device() && lse.scalar_type() == at::kFloat && lse.numel() == (int64_t)B * H * S,
+                      "lse must be float32 [B, H, T] on q's device");
+    const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    Launch at(q);
+    const size_t nbytes = otx_attn_bwd_workspace_bytes(B, H, Hkv, S, D, w);
+    const Workspace ws(q, nbytes);
+    if (saved.size() > 5) {
+      const Tensor sc = saved[5].contiguous();
+      TORCH_CHECK_VALUE(sc.device() == q.device() && sc.scalar_type() == at::kFloat,
+                        "score_cache must be a float32 tensor on q's device");
+      check(otx_attn_bwd_sc(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(),
+                            dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), sc.data_ptr<float>(),
+                            (size_t)sc.numel() * 4, B, H, Hkv, S, D, w, dt, ws.ptr, nbytes, 0, 7, at.stream),
+            "otx_attn_bwd");
+    } else {
+      check(otx_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(),
+                         dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, H, Hkv, S, D, w, dt, ws.ptr,
+                         nbytes, at.stream),
+            "otx_attn_bwd");
+    }
+    return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
+  }
+};
+
+Tensor linear(const Tensor& x, const Tensor& w) { return Linear::apply(x, w); }
+Tensor rms_norm(const Tensor& x, const Tensor& w, double eps) { return RMSNorm::apply(x, w, eps); }
+Tensor silu(const Tensor& x) { return SiLU::apply(x); }
+Tensor swiglu(const Tensor& gu) { return SwiGLU::apply(gu); }
+Tensor rope_heads(const Tensor& x, const Tensor& cos, const Tensor& sin) { return RopeHeads::apply(x, cos, sin); }
+Tensor swap_heads(const Tensor& x) { return SwapHeads::apply(x); }
+Tensor embedding(const Tensor& ids, const Tensor& w) { return Embedding::apply(ids, w); }
+std::tuple<Tensor, Tensor> loss(const Tensor& logits, const Tensor& labels, double coeff) {
+  const variable_list r = Loss::apply(logits, labels, coeff);
+  return {r[0], r[1]};
+}
+Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const std::optional<Tensor>& sc, int64_t window,
+                 bool int8pv) {
+  return Attention::apply(q, k, v, sc, window, int8pv);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_otx_autograd, m) {
+  m.def("linear", torch::wrap_pybind_function(linear));
+  m.def("rms_norm", torch::wrap_pybind_function(rms_norm));
+  m.def("silu", torch::wrap_pybind_function(silu));
+  m.def("swiglu", torch::wrap_pybind_function(swiglu));
+  m.def("rope_heads", torch::wrap_pybind_function(rope_heads));
+  m.def("swap_heads", torch::wrap_pybind_function(swap_heads));
+  m.def("embedding", torch::wrap_pybind_function(embedding));
+  m.def("loss", torch::wrap_pybind_function(loss));
+  m.def("attention", torch::wrap_pybind_function(attention));
+}

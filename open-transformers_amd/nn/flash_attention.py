@@ -327,6 +327,18 @@ class _CausalFlashAttention(torch.autograd.Function):
         return dq, dk, dv, None, None
 
 
+def _native_attention(q, k, v, window, int8pv, mode):
+    """The native node, for every call but those under activation checkpointing's
+    modes, which record, replay or leave out what the forward saves (the Python
+    nodes above).  It saves the same tensors in the same order as they do, so it
+    serves as the recompute of a first forward that they ran."""
+    sc = None
+    if mode == _SC_KEEP:
+        B, H, S, _ = q.shape
+        sc = _new_score_cache(B, H, S, window, q.device)
+    return _lib.autograd().attention(q, k, v, sc, window, int8pv)
+
+
 def causal_flash_attention(
     q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, dropout: float = 0.0, window: int = 0
 ) -> torch.Tensor:
@@ -334,7 +346,10 @@ def causal_flash_attention(
     if dropout != 0.0:
         raise ValueError("causal_flash_attention is deterministic: dropout must be 0.0")
     _check_inputs(q, k, v, window)
-    return _CausalFlashAttention.apply(q, k, v, window, _score_cache_mode(q, k, v))
+    mode = _score_cache_mode(q, k, v)
+    if mode == _SC_PLACEHOLDER or getattr(_ckpt, "state", None) is not None:
+        return _CausalFlashAttention.apply(q, k, v, window, mode)
+    return _native_attention(q, k, v, window, False, mode)
 
 
 def int8pv_workspace_bytes(B: int, H: int, Hkv: int, S: int, D: int) -> int:
@@ -414,4 +429,7 @@ def int8pv_causal_flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Ten
     _check_inputs(q, k, v, window)
     if q.dtype != torch.bfloat16:
         raise ValueError(f"int8pv_causal_flash_attention takes bfloat16 inputs, got {q.dtype}")
-    return _Int8PVFlashAttention.apply(q, k, v, window, _score_cache_mode(q, k, v))
+    mode = _score_cache_mode(q, k, v)
+    if mode == _SC_PLACEHOLDER or getattr(_ckpt, "state", None) is not None:
+        return _Int8PVFlashAttention.apply(q, k, v, window, mode)
+    return _native_attention(q, k, v, window, True, mode)

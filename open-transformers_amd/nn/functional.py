@@ -10,7 +10,7 @@ and the torch compositions around them, each fused into one pass:
                         (rope.py:103-125, attention_repop.py:143-149)
   heads(x)              x.transpose(1, 2).contiguous() (attention_repop.py:150)
   merge_heads(o)        o.transpose(1, 2).contiguous().view(B, T, H * D) (attention_repop.py:155)
-Each is a torch.autograd.Function over the C ABI of libotx_attn.so: bf16 in,
+Each is an autograd node of csrc/otx_autograd.cpp over the C ABI of libotx_attn.so: bf16 in,
 binary32 arithmetic in a fixed order, bf16 out, and for the compositions the
 bytes torch's own forward and autograd backward give; weight gradients come
 back in the weight's dtype.  GPU tensors only; there is no CPU fallback.
@@ -52,70 +52,10 @@ def gemm_bf16(a: torch.Tensor, a_strides: tuple[int, int], b: torch.Tensor, b_st
     return c
 
 
-class _Linear(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, w):
-        K = x.shape[-1]
-        N = w.shape[0]
-        x2 = x.reshape(-1, K).contiguous()
-        wc = w.contiguous()
-        M = x2.shape[0]
-        y = gemm_bf16(x2, (K, 1), wc, (K, 1), M, N, K)  # y = x @ w^T
-        ctx.save_for_backward(x2, wc)
-        ctx.xshape = x.shape
-        return y.view(*x.shape[:-1], N)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x2, w = ctx.saved_tensors
-        M, K = x2.shape
-        N = w.shape[0]
-        dy2 = dy.reshape(M, N).contiguous()
-        dx = dw = None
-        if ctx.needs_input_grad[0]:  # dx[m][k] = sum_n dy[m][n] w[n][k]
-            dx = gemm_bf16(dy2, (N, 1), w, (1, K), M, K, N).view(ctx.xshape)
-        if ctx.needs_input_grad[1]:  # dw[n][k] = sum_m dy[m][n] x[m][k]
-            dw = gemm_bf16(dy2, (1, N), x2, (1, K), N, K, M)
-        return dx, dw
-
-
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w^T (no bias), bf16 operands, serial binary32 fold, bf16 result."""
     _need_gpu(x, w)
-    return _Linear.apply(x, w)
-
-
-class _RMSNorm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, w, eps):
-        D = x.shape[-1]
-        xc = x.contiguous()
-        wc = w.to(x.dtype).contiguous()
-        rows = xc.numel() // D
-        y = torch.empty_like(xc)
-        rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
-        rc = _lib.load().otx_rmsnorm_fwd(xc.data_ptr(), wc.data_ptr(), y.data_ptr(), rstd.data_ptr(), rows, D, eps,
-                                         _DT[x.dtype], _stream(x))
-        _lib.check(rc, "otx_rmsnorm_fwd")
-        ctx.save_for_backward(xc, wc, rstd)
-        ctx.wdtype = w.dtype
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, w, rstd = ctx.saved_tensors
-        D = x.shape[-1]
-        rows = x.numel() // D
-        dyc = dy.contiguous()
-        dx = torch.empty_like(x)
-        dw = torch.empty(D, dtype=torch.float32, device=x.device)
-        lib = _lib.load()
-        nbytes = int(lib.otx_rmsnorm_bwd_workspace_bytes(rows, D))
-        ws = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=x.device)
-        rc = lib.otx_rmsnorm_bwd(x.data_ptr(), w.data_ptr(), rstd.data_ptr(), dyc.data_ptr(), dx.data_ptr(),
-                                 dw.data_ptr(), rows, D, _DT[x.dtype], ws.data_ptr(), nbytes, _stream(x))
-        _lib.check(rc, "otx_rmsnorm_bwd")
-        return dx, dw.to(ctx.wdtype), None
+    return _lib.autograd().linear(x, w)
 
 
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -123,28 +63,7 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     _need_gpu(x, w)
     if x.dtype not in _DT:
         raise ValueError(f"dtype {x.dtype} not supported")
-    return _RMSNorm.apply(x, w, float(eps))
-
-
-class _SiLU(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x):
-        xc = x.contiguous()
-        y = torch.empty_like(xc)
-        rc = _lib.load().otx_silu_fwd(xc.data_ptr(), y.data_ptr(), xc.numel(), _DT[x.dtype], _stream(x))
-        _lib.check(rc, "otx_silu_fwd")
-        ctx.save_for_backward(xc)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        (x,) = ctx.saved_tensors
-        dyc = dy.contiguous()
-        dx = torch.empty_like(x)
-        rc = _lib.load().otx_silu_bwd(x.data_ptr(), dyc.data_ptr(), dx.data_ptr(), x.numel(), _DT[x.dtype],
-                                      _stream(x))
-        _lib.check(rc, "otx_silu_bwd")
-        return dx
+    return _lib.autograd().rms_norm(x, w, float(eps))
 
 
 def silu(x: torch.Tensor) -> torch.Tensor:
@@ -152,32 +71,7 @@ def silu(x: torch.Tensor) -> torch.Tensor:
     _need_gpu(x)
     if x.dtype not in _DT:
         raise ValueError(f"dtype {x.dtype} not supported")
-    return _SiLU.apply(x)
-
-
-class _SwiGLU(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, gu):
-        F = gu.shape[-1] // 2
-        guc = gu.contiguous()
-        rows = guc.numel() // (2 * F)
-        h = torch.empty(*gu.shape[:-1], F, dtype=gu.dtype, device=gu.device)
-        rc = _lib.load().otx_swiglu_fwd(guc.data_ptr(), h.data_ptr(), rows, F, _DT[gu.dtype], _stream(gu))
-        _lib.check(rc, "otx_swiglu_fwd")
-        ctx.save_for_backward(guc)
-        return h
-
-    @staticmethod
-    def backward(ctx, dh):
-        (gu,) = ctx.saved_tensors
-        F = gu.shape[-1] // 2
-        rows = gu.numel() // (2 * F)
-        dhc = dh.contiguous()
-        dgu = torch.empty_like(gu)
-        rc = _lib.load().otx_swiglu_bwd(gu.data_ptr(), dhc.data_ptr(), dgu.data_ptr(), rows, F, _DT[gu.dtype],
-                                        _stream(gu))
-        _lib.check(rc, "otx_swiglu_bwd")
-        return dgu
+    return _lib.autograd().silu(x)
 
 
 def swiglu(gu: torch.Tensor) -> torch.Tensor:
@@ -188,31 +82,7 @@ def swiglu(gu: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"dtype {gu.dtype} not supported")
     if gu.shape[-1] % 16:
         raise ValueError(f"swiglu: last dimension {gu.shape[-1]} is not a multiple of 16")
-    return _SwiGLU.apply(gu)
-
-
-class _RopeHeads(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, cos, sin):
-        B, T, H, D = x.shape
-        xc = x.contiguous()
-        y = torch.empty((B, H, T, D), dtype=x.dtype, device=x.device)
-        rc = _lib.load().otx_rope_heads_fwd(xc.data_ptr(), cos.data_ptr(), sin.data_ptr(), y.data_ptr(), B, T, H, D,
-                                            _DT[x.dtype], _stream(x))
-        _lib.check(rc, "otx_rope_heads_fwd")
-        ctx.save_for_backward(cos, sin)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        cos, sin = ctx.saved_tensors
-        B, H, T, D = dy.shape
-        dyc = dy.contiguous()
-        dx = torch.empty((B, T, H, D), dtype=dy.dtype, device=dy.device)
-        rc = _lib.load().otx_rope_heads_bwd(dyc.data_ptr(), cos.data_ptr(), sin.data_ptr(), dx.data_ptr(), B, T, H, D,
-                                            _DT[dy.dtype], _stream(dy))
-        _lib.check(rc, "otx_rope_heads_bwd")
-        return dx, None, None
+    return _lib.autograd().swiglu(gu)
 
 
 def rope_heads(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
@@ -227,26 +97,7 @@ def rope_heads(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     for name, t in (("cos", cos), ("sin", sin)):
         if t.dtype != torch.float32 or tuple(t.shape) != (T, D // 2):
             raise ValueError(f"rope_heads: {name} must be binary32 [{T}, {D // 2}], got {t.dtype} {tuple(t.shape)}")
-    return _RopeHeads.apply(x, cos.contiguous(), sin.contiguous())
-
-
-def _swap12(x: torch.Tensor) -> torch.Tensor:
-    B, X, Y, D = x.shape
-    xc = x.contiguous()
-    y = torch.empty((B, Y, X, D), dtype=x.dtype, device=x.device)
-    rc = _lib.load().otx_swap_heads(xc.data_ptr(), y.data_ptr(), B, X, Y, D, _DT[x.dtype], _stream(x))
-    _lib.check(rc, "otx_swap_heads")
-    return y
-
-
-class _SwapHeads(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x):
-        return _swap12(x)
-
-    @staticmethod
-    def backward(ctx, dy):
-        return _swap12(dy)
+    return _lib.autograd().rope_heads(x, cos.contiguous(), sin.contiguous())
 
 
 def heads(x: torch.Tensor) -> torch.Tensor:
@@ -255,7 +106,7 @@ def heads(x: torch.Tensor) -> torch.Tensor:
     if x.dtype not in _DT or x.dim() != 4 or x.shape[-1] % 8:
         raise ValueError(f"heads takes a bf16/binary32 [B, T, H, D] tensor with D a multiple of 8, got {x.dtype} "
                          f"{tuple(x.shape)}")
-    return _SwapHeads.apply(x)
+    return _lib.autograd().swap_heads(x)
 
 
 def merge_heads(o: torch.Tensor) -> torch.Tensor:
@@ -265,4 +116,4 @@ def merge_heads(o: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"merge_heads takes a bf16/binary32 [B, H, T, D] tensor with D a multiple of 8, got "
                          f"{o.dtype} {tuple(o.shape)}")
     B, H, T, D = o.shape
-    return _SwapHeads.apply(o).view(B, T, H * D)
+    return _lib.autograd().swap_heads(o).view(B, T, H * D)

@@ -61,24 +61,13 @@ def ce_zloss_backward(logits, labels, stats, grad_ce, grad_z, coeff: float) -> t
     return grad
 
 
-class _FusedCEZLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logits, labels, coeff):
-        ce, z, stats = ce_zloss_forward(logits, labels, coeff)
-        ctx.save_for_backward(logits, labels, stats)
-        ctx.coeff = coeff
-        return ce, z
-
-    @staticmethod
-    def backward(ctx, grad_ce, grad_z):
-        logits, labels, stats = ctx.saved_tensors
-        return ce_zloss_backward(logits, labels, stats, grad_ce, grad_z, ctx.coeff), None, None
-
-
 def fused_ce_z_loss(logits: torch.Tensor, labels: torch.Tensor, coeff: float, *, chunk_rows: int = 2048):
     """Fused ``(ce, z_loss)`` over ``[..., V]`` logits and matching labels;
     ``coeff == 0`` gives ``z_loss == 0`` and no z gradient."""
     del chunk_rows  # row chunking is a memory device of the reference; the kernels need none
-    flat_logits = logits.reshape(-1, logits.shape[-1])
-    flat_labels = labels.reshape(-1)
-    return _FusedCEZLoss.apply(flat_logits, flat_labels, float(coeff))
+    if logits.dim() != 2:
+        logits = logits.reshape(-1, logits.shape[-1])
+    if labels.dim() != 1:
+        labels = labels.reshape(-1)
+    _check(logits, labels)
+    return _lib.autograd().loss(logits, labels, float(coeff))

@@ -1,0 +1,97 @@
+"""The native autograd nodes as autograd sees them: saved-tensor hooks reach every saved tensor, a saved input changed
+in place is refused, a gradient that nobody asks for is not computed, an unused output counts as a zero gradient, and
+non-contiguous and expanded upstream gradients give the bytes of contiguous ones."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from open_transformers_amd.nn import functional as F
+from open_transformers_amd.nn.embedding import embedding
+from open_transformers_amd.nn.flash_attention import causal_flash_attention, int8pv_causal_flash_attention
+from open_transformers_amd.nn.layer import rope_tables
+from open_transformers_amd.nn.loss import fused_ce_z_loss
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _rand(*shape, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + sum(shape))
+    return torch.randn(shape, device=DEV, generator=g).bfloat16().requires_grad_()
+
+
+def _cases():
+    cos, sin = (t.to(DEV) for t in rope_tables(64, 64, 10000.0))
+    q, k, v = _rand(1, 4, 64, 64), _rand(1, 2, 64, 64, seed=1), _rand(1, 2, 64, 64, seed=2)
+    ids = torch.arange(64, device=DEV) % 16
+    return {  # name: (call, inputs, tensors the node saves)
+        "linear": (F.linear, (_rand(128, 128), _rand(256, 128)), 2),
+        "rms_norm": (lambda x, w: F.rms_norm(x, w, 1e-5), (_rand(64, 128), _rand(128)), 3),
+        "silu": (F.silu, (_rand(33, 7),), 1),
+        "swiglu": (F.swiglu, (_rand(8, 64),), 1),
+        "rope_heads": (lambda x: F.rope_heads(x, cos, sin), (_rand(2, 64, 4, 64),), 2),
+        "heads": (F.heads, (_rand(2, 64, 4, 64),), 0),
+        "embedding": (lambda w: embedding(ids, w), (_rand(16, 64),), 1),
+        "attention": (causal_flash_attention, (q, k, v), 6),
+        "attention_int8pv": (int8pv_causal_flash_attention, (q, k, v), 6),
+        "loss": (lambda x: fused_ce_z_loss(x, ids, 1e-4)[0], (_rand(64, 100),), 3),
+    }
+
+
+NAMES = ["linear", "rms_norm", "silu", "swiglu", "rope_heads", "heads", "embedding", "attention", "attention_int8pv",
+         "loss"]
+
+
+def _bits(t):
+    return t.contiguous().view(torch.int16 if t.dtype == torch.bfloat16 else torch.int32)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_hooks_partial_and_strided_gradients(name):
+    print(f"autograd node {name}", flush=True)
+    call, inputs, nsaved = _cases()[name]
+    y = call(*inputs)
+    dy = torch.randn(y.shape, device=DEV).to(y.dtype)
+    ref = torch.autograd.grad(y, inputs, dy)
+
+    packed = []
+
+    def pack(t):
+        packed.append(t)
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(DEV)):
+        y2 = call(*inputs)
+    assert len(packed) == nsaved
+    for a, b in zip(torch.autograd.grad(y2, inputs, dy), ref):
+        assert torch.equal(_bits(a), _bits(b))
+
+    for i in range(len(inputs)):  # one input at a time
+        args = [t if j == i else t.detach() for j, t in enumerate(inputs)]
+        (g,) = torch.autograd.grad(call(*args), [inputs[i]], dy)
+        assert torch.equal(_bits(g), _bits(ref[i]))
+
+    if y.dim() >= 2:  # a transposed upstream gradient of the same values
+        strided = dy.transpose(-1, -2).contiguous().transpose(-1, -2)
+        for a, b in zip(torch.autograd.grad(call(*inputs), inputs, strided), ref):
+            assert torch.equal(_bits(a), _bits(b))
+        expanded = torch.ones(1, device=DEV, dtype=y.dtype).expand(y.shape)
+        for a, b in zip(torch.autograd.grad(call(*inputs), inputs, expanded),
+                        torch.autograd.grad(call(*inputs), inputs, torch.ones_like(y))):
+            assert torch.equal(_bits(a), _bits(b))
+    with torch.no_grad():
+        assert torch.equal(_bits(call(*inputs)), _bits(y.detach()))
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("name", ["linear", "rms_norm", "silu", "swiglu", "attention", "loss"])
+def test_saved_input_changed_in_place_is_refused(name):
+    call, inputs, _ = _cases()[name]
+    x = inputs[0].detach().clone().requires_grad_()
+    y = call(x, *inputs[1:])
+    with torch.no_grad():
+        x.add_(1.0)
+    with pytest.raises(RuntimeError, match="inplace"):
+        torch.autograd.grad(y.sum(), [x])
