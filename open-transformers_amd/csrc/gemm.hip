@@ -17,30 +17,23 @@
 // Tiling: a workgroup of 4 waves owns a 128 x 128 block of C, each wave a
 // 64 x 64 quarter (two MFMAs per r: i-blocks {0,1} x j-block 0, then x
 // j-block 1), or, in the narrow form, a 128 x 64 block with 64 x 32 per wave
-// (one MFMA per r), or, in the small form, a 64 x 64 block with 32 x 32 per
-// wave (one v_mfma_f32_16x16x1_4b_f32 per r, also one fma per output).  r
-// advances in chunks of 32.  The wide and narrow forms (gemm_bf16_v2_kernel)
-// keep each chunk in LDS as bf16 in two slots, one barrier per chunk: an
-// i-contiguous operand is copied straight from global memory into LDS, an
+// (one MFMA per r), or, in the small forms, a 64 x 64 or 32 x 32 block with
+// 32 x 32 or 16 x 16 per wave, on v_mfma_f32_16x16x4_f32 (four serial fmas per
+// output; see there).  The wide and narrow forms (gemm_bf16_v2_kernel)
+// advance r in chunks of 32 kept in LDS as bf16 in two slots, one barrier per chunk:
+// an i-contiguous operand is copied straight from global memory into LDS, an
 // r-contiguous one loaded into registers and stored transposed, and the MFMA
 // operands are read with ds_read_u16_d16_hi, which yields the binary32 value of
-// a bf16 with no conversion instruction (see GemmTile16).  The narrow form of
-// dx = dy w and the small form stage their chunks as binary32 (GemmOperand),
-// converted once per element, with the next chunk's global loads issued before
-// the current chunk's MFMAs.  Either operand may be r-contiguous (a_r == 1) or
-// i-contiguous (a_i == 1); the loads are 16-byte vectors along the contiguous
-// axis.  Every output is one lane's serial chain whatever the tile, so every
-// form gives the same bytes.
+// a bf16 with no conversion instruction (see GemmTile16).  Either operand may be
+// r-contiguous (a_r == 1) or i-contiguous (a_i == 1); the loads are 16-byte
+// vectors along the contiguous axis.  Every output is one lane's serial chain
+// whatever the tile, so every form gives the same bytes.
 #include "otx_common.h"
 
 namespace otx {
 
 constexpr int GT = 128;   // workgroup tile (i and j)
 constexpr int GRC = 32;   // r chunk
-constexpr int GP = GT + 4;  // LDS pitch (floats) of one r row of a staged tile
-#ifndef OTX_GEMM_SMALL_PF
-#define OTX_GEMM_SMALL_PF 3  // chunks of global loads in flight in the small form
-#endif
 
 // Tile of workgroup `bid` among ntiles = tiles_i x tiles_j.  Workgroups are
 // dealt to the 8 XCDs round-robin (workgroup b runs on XCD b % 8, each XCD with
@@ -60,123 +53,6 @@ __device__ __forceinline__ void gemm_tile(int bid, int ntiles, int tiles_j, int*
   const int within = s - first * tiles_j;
   *ti = first + within % gm;
   *tj = within / gm;
-}
-
-// One operand's chunk: ROWS rows (i; 128, or 64 for the narrow form's B) x 32 r
-// = ROWS * 4 vectors of 8 bf16, NV per thread.  An r-contiguous operand is
-// staged [i][r] (pitch GRC + 4 floats: the 16-byte reads of 16 consecutive rows
-// start in 16 distinct 4-bank groups), so both its commit and its reads are
-// 16-byte vectors along r; an i-contiguous operand is staged [r][i] (pitch
-// ROWS + 4), read one r at a time with the lanes on consecutive i.
-template <bool RCONT, int ROWS>
-struct GemmOperand {
-  static constexpr int NV = ROWS * GRC / 8 / 256;  // 16-byte vectors per thread
-  static constexpr int IV = ROWS / 8;              // vectors per r of an i-contiguous operand
-  static constexpr int PITCH = RCONT ? GRC + 4 : ROWS + 4;
-  static constexpr int FLOATS = RCONT ? ROWS * (GRC + 4) : GRC * (ROWS + 4);
-  static_assert(NV >= 1 && NV * 256 * 8 == ROWS * GRC, "the chunk must split evenly over 256 threads");
-  uint4 v[NV];
-  __device__ __forceinline__ void issue(const uint16_t* base, long s_i, long s_r, int i0, int r0) {
-#pragma unroll
-    for (int x = 0; x < NV; x++) {
-      const int idx = threadIdx.x + 256 * x;
-      if constexpr (RCONT) {  // 8 consecutive r of one row i
-        const int i = idx >> 2, rv = (idx & 3) * 8;
-        v[x] = *reinterpret_cast<const uint4*>(base + (long)(i0 + i) * s_i + (r0 + rv));
-      } else {  // 8 consecutive i of one r
-        const int r = idx / IV, iv = (idx % IV) * 8;
-        v[x] = *reinterpret_cast<const uint4*>(base + (long)(r0 + r) * s_r + (i0 + iv));
-      }
-    }
-  }
-  __device__ __forceinline__ void commit(float* tile) const {
-#pragma unroll
-    for (int x = 0; x < NV; x++) {
-      const int idx = threadIdx.x + 256 * x;
-      float* d;
-      if constexpr (RCONT) {
-        const int i = idx >> 2, rv = (idx & 3) * 8;
-        d = tile + i * PITCH + rv;
-      } else {
-        const int r = idx / IV, iv = (idx % IV) * 8;
-        d = tile + r * PITCH + iv;
-      }
-      *reinterpret_cast<float4*>(d) = make_float4(Elem<uint16_t>::get(v[x], 0), Elem<uint16_t>::get(v[x], 1),
-                                                  Elem<uint16_t>::get(v[x], 2), Elem<uint16_t>::get(v[x], 3));
-      *reinterpret_cast<float4*>(d + 4) = make_float4(Elem<uint16_t>::get(v[x], 4), Elem<uint16_t>::get(v[x], 5),
-                                                      Elem<uint16_t>::get(v[x], 6), Elem<uint16_t>::get(v[x], 7));
-    }
-  }
-  // Staged values (i, r0 .. r0 + 3).
-  __device__ __forceinline__ static void load4(const float* tile, int i, int r0, float (&o)[4]) {
-    if constexpr (RCONT) {
-      const float4 t = *reinterpret_cast<const float4*>(tile + i * PITCH + r0);
-      o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; e++) o[e] = tile[(r0 + e) * PITCH + i];
-    }
-  }
-};
-
-// WJ: the columns of C per wave (64, or 32 in the narrow form); the workgroup
-// tile is 128 x 2 WJ.
-template <bool ARC, bool BRC, bool OUT_F32, int WJ>
-__global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(const uint16_t* __restrict__ A, long a_i, long a_r,
-                                                            const uint16_t* __restrict__ B, long b_j, long b_r,
-                                                            void* __restrict__ C, long ldc, int M, int N, int R) {
-  constexpr int GTJ = 2 * WJ;
-  __shared__ __align__(16) float As[GemmOperand<ARC, GT>::FLOATS];
-  __shared__ __align__(16) float Bs[GemmOperand<BRC, GTJ>::FLOATS];
-  const int tiles_j = N / GTJ;
-  int ti, tj;
-  gemm_tile(blockIdx.x, (M / GT) * tiles_j, tiles_j, &ti, &tj);
-  const int i0 = ti * GT, j0 = tj * GTJ;
-  const int wave = threadIdx.x >> 6, L = threadIdx.x & 63, hh = L >> 5, c = L & 31;
-  const int wi = (wave >> 1) * 64, wj = (wave & 1) * WJ;  // wave quarter inside the tile
-
-  GemmOperand<ARC, GT> ga;
-  GemmOperand<BRC, GTJ> gb;
-  f32x32 acc0 = f32x32{}, acc1 = f32x32{};
-  const int nch = R / GRC;
-  ga.issue(A, a_i, a_r, i0, 0);
-  gb.issue(B, b_j, b_r, j0, 0);
-  for (int ch = 0; ch < nch; ++ch) {
-    __syncthreads();  // previous chunk fully consumed
-    ga.commit(As);
-    gb.commit(Bs);
-    __syncthreads();
-    if (ch + 1 < nch) {
-      ga.issue(A, a_i, a_r, i0, (ch + 1) * GRC);
-      gb.issue(B, b_j, b_r, j0, (ch + 1) * GRC);
-    }
-    const int ai = wi + hh * 32 + c, bj = wj + c;
-#pragma unroll
-    for (int r0 = 0; r0 < GRC; r0 += 4) {
-      float a[4], b0[4], b1[4];
-      GemmOperand<ARC, GT>::load4(As, ai, r0, a);
-      GemmOperand<BRC, GTJ>::load4(Bs, bj, r0, b0);
-      if constexpr (WJ == 64) GemmOperand<BRC, GTJ>::load4(Bs, bj + 32, r0, b1);
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        acc0 = otx_mfma(a[e], b0[e], acc0);
-        if constexpr (WJ == 64) acc1 = otx_mfma(a[e], b1[e], acc1);
-      }
-    }
-  }
-  // acc0: rows wi + blk*32 + R(r%16, hh), column wj + c; acc1: column wj + 32 + c.
-#pragma unroll
-  for (int r = 0; r < 32; r++) {
-    const int i = i0 + wi + 32 * (r >> 4) + otx_row(r, hh);
-    const long o0 = (long)i * ldc + j0 + wj + c;
-    if constexpr (OUT_F32) {
-      static_cast<float*>(C)[o0] = acc0[r];
-      if constexpr (WJ == 64) static_cast<float*>(C)[o0 + 32] = acc1[r];
-    } else {
-      static_cast<uint16_t*>(C)[o0] = otx_f32_to_bf16(acc0[r]);
-      if constexpr (WJ == 64) static_cast<uint16_t*>(C)[o0 + 32] = otx_f32_to_bf16(acc1[r]);
-    }
-  }
 }
 
 // One operand's chunk of 32 r held in LDS as bf16, [r][row] with a pitch of PB
@@ -341,154 +217,293 @@ __global__ __launch_bounds__(256, 4) void gemm_bf16_v2_kernel(const uint16_t* __
   }
 }
 
-// Small form: a workgroup of 4 waves owns a 64 x 64 block of C, each wave a
-// 32 x 32 quarter as the four 16 x 16 blocks of one v_mfma_f32_16x16x1_4b_f32
-// per r (lane L supplies A row wi + 16 (b & 1) + L % 16 and B column
-// wj + 16 (b >> 1) + L % 16 of block b = L / 16).  For grids of far fewer
-// 128 x 128 tiles than CUs, where the other forms would leave CUs idle.
-template <bool ARC, bool BRC, bool OUT_F32>
-__global__ __launch_bounds__(256, 2) void gemm_bf16_small_kernel(const uint16_t* __restrict__ A, long a_i, long a_r,
-                                                                  const uint16_t* __restrict__ B, long b_j, long b_r,
-                                                                  void* __restrict__ C, long ldc, int M, int N,
-                                                                  int R) {
-  constexpr int GS = 64;
-  __shared__ __align__(16) float As[GemmOperand<ARC, GS>::FLOATS];
-  __shared__ __align__(16) float Bs[GemmOperand<BRC, GS>::FLOATS];
+// ---- the small forms: v_mfma_f32_16x16x4_f32 ----
+// One instruction is four steps of the fold: D = fma(a3, b3, fma(a2, b2, fma(a1, b1,
+// fma(a0, b0, C)))), each rounded (tests/test_gpu_selftest.py compares it with fmaf), in
+// 32 cycles.  Its rate is that of the K = 1 forms, but a 16 x 16 block advances one r in 8
+// cycles where they take 32 (or 64): a product with few tiles is bound by the chain
+// of one wave, so the smaller block per wave is worth its operand traffic.  Lane
+// L = 16 g + c supplies A row c and B column c of the block at r = 4 s + g, step s; result
+// register q of lane L holds row 4 g + q, column c.
+//
+// A workgroup of 4 waves owns a 32 NB x 32 NB tile of C, each wave NB x NB blocks.  r
+// advances in stages of 32 SUBS, kept in LDS as bf16 and copied straight from global
+// memory (global_load_lds_dwordx4) three stages ahead into four slots, one barrier per
+// stage.  An i-contiguous operand lies as [r][row]; an r-contiguous one as SUBS
+// sub-chunks of [row][32 r], the four 16-byte units of a row swizzled by row / 4, so that
+// the 16 rows that a step reads fall in distinct banks.  Either way a step reads its
+// operands with ds_read_u16_d16_hi (no conversion, and no commit through registers),
+// two groups ahead under hand-kept lgkmcnt accounting; no read is in flight across a
+// branch, where the compiler could copy its register.
+template <bool RC, int ROWS, int SUBS>
+struct GemmStage {
+  static constexpr int SUB = 32 * ROWS * 2;      // bytes of 32 r
+  static constexpr int BYTES = SUBS * SUB;
+  static constexpr int NI = BYTES / 1024 / 4;    // copy instructions per wave
+  static constexpr int NA = RC ? 4 : 1;          // lane addresses
+  static_assert(NI >= 1, "stage shape");
+  // The stage of r0 on; r past the end of the product (a last stage that is not whole) copy its
+  // first 32 again and are not read.
+  __device__ __forceinline__ static void issue(const uint16_t* base, long s_i, long s_r, int i0, int r0, int R,
+                                               unsigned char* lds, int wave_u, int L) {
+#pragma unroll
+    for (int x = 0; x < NI; x++) {
+      const int n = wave_u + 4 * x;
+      if constexpr (RC) {
+        const int sub = n / (ROWS / 16), row = n % (ROWS / 16) * 16 + (L >> 2);
+        const int unit = (L & 3) ^ ((row >> 2) & 3);
+        const int r = r0 + (r0 + 32 * sub < R ? 32 * sub : 0) + 8 * unit;
+        otx_dma16(base + (long)(i0 + row) * s_i + r, lds + n * 1024);
+      } else {
+        constexpr int VPR = ROWS / 8;  // vectors per r
+        const int k = n * (64 / VPR) + L / VPR;
+        const int r = r0 + k < R ? r0 + k : r0 + (k & 31);
+        otx_dma16(base + (long)r * s_r + (i0 + L % VPR * 8), lds + n * 1024);
+      }
+    }
+  }
+  // Lane addresses (row0: the wave's first row), and the offset of block b at step s from address which(s).
+  __device__ __forceinline__ static void lanes(uint32_t lds, int row0, int g, int c, uint32_t (&a)[NA]) {
+    if constexpr (RC) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) a[u] = lds + (row0 + c) * 64 + ((u ^ ((c >> 2) & 3)) << 4) + 2 * g;
+    } else {
+      a[0] = lds + g * ROWS * 2 + (row0 + c) * 2;
+    }
+  }
+  static constexpr int which(int s) { return RC ? (s & 7) >> 1 : 0; }
+  static constexpr int off(int s, int b) {
+    return RC ? (s >> 3) * SUB + b * 16 * 64 + (s & 1) * 8 : 4 * s * ROWS * 2 + b * 32;
+  }
+};
+
+template <int N>
+__device__ __forceinline__ void gemm_vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// f(0), f(1), ... f(E - 1) as long as they are true; whether all were.
+template <int B, int E>
+struct OtxAll {
+  template <class F>
+  __device__ __forceinline__ static bool run(F&& f) {
+    if constexpr (B < E) {
+      if (!f(std::integral_constant<int, B>{})) return false;
+      return OtxAll<B + 1, E>::run(f);
+    }
+    return true;
+  }
+};
+
+template <bool ARC, bool BRC, bool OUT_F32, int NB>
+__global__ __launch_bounds__(256, 2) void gemm_bf16_k4_kernel(const uint16_t* __restrict__ A, long a_i, long a_r,
+                                                               const uint16_t* __restrict__ B, long b_j, long b_r,
+                                                               void* __restrict__ C, long ldc, int M, int N, int R) {
+  constexpr int GS = 32 * NB;
+  constexpr int NS = 4, P = NS - 1;
+  constexpr int SUBS = NB == 1 ? 4 : 2, SR = 32 * SUBS;  // r per stage
+  constexpr int SPG = NB == 1 ? 2 : 1;      // steps per read group
+  using TA = GemmStage<ARC, GS, SUBS>;
+  using TB = GemmStage<BRC, GS, SUBS>;
+  constexpr int SLOT = TA::BYTES + TB::BYTES;
+  constexpr int NDMA = TA::NI + TB::NI;     // copy instructions of a stage and wave
+  static_assert(NS * SLOT <= 65536, "slot offsets are 16-bit immediates");
+  static_assert(2 * NB * SPG == 4, "read group of 4");
+  __shared__ __align__(16) unsigned char smem[NS * SLOT];
   const int tiles_j = N / GS;
   int ti, tj;
   gemm_tile(blockIdx.x, (M / GS) * tiles_j, tiles_j, &ti, &tj);
   const int i0 = ti * GS, j0 = tj * GS;
-  const int wave = threadIdx.x >> 6, L = threadIdx.x & 63, blk = L >> 4, c = L & 15;
-  const int wi = (wave >> 1) * 32, wj = (wave & 1) * 32;
+  const int wave = threadIdx.x >> 6, L = threadIdx.x & 63, g = L >> 4, c = L & 15;
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  const int wi = (wave >> 1) * 16 * NB, wj = (wave & 1) * 16 * NB;
+  const int nst = (R + SR - 1) / SR;
+  const auto issue = [&](int st, unsigned char* slot) {
+    TA::issue(A, a_i, a_r, i0, SR * st, R, slot, wave_u, L);
+    TB::issue(B, b_j, b_r, j0, SR * st, R, slot + TA::BYTES, wave_u, L);
+  };
+#pragma unroll
+  for (int k = 0; k < P; k++)
+    if (k < nst) issue(k, smem + k * SLOT);
+  uint32_t la[TA::NA], lb[TB::NA];
+  TA::lanes(otx_lds_addr(smem), wi, g, c, la);
+  TB::lanes(otx_lds_addr(smem) + TA::BYTES, wj, g, c, lb);
+  f32x4 acc[NB][NB];
+#pragma unroll
+  for (int x = 0; x < NB; x++)
+#pragma unroll
+    for (int y = 0; y < NB; y++) acc[x][y] = f32x4{};
+  float opr[3][4];  // read banks, low halves zero
+#pragma unroll
+  for (int x = 0; x < 4; x++) { opr[0][x] = 0.0f; opr[1][x] = 0.0f; opr[2][x] = 0.0f; }
+  // every scalar load of an argument has returned before the counted LDS reads begin (they share lgkmcnt)
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(ldc), "+s"(C));
 
-  // A chunk's MFMAs take a quarter of the wide form's time, less than a global
-  // load's latency, so the loads run PF chunks ahead (a ring of PF register
-  // sets, indexed statically by unrolling over the ring).
-  constexpr int PF = OTX_GEMM_SMALL_PF;
-  GemmOperand<ARC, GS> ga[PF];
-  GemmOperand<BRC, GS> gb[PF];
-  f32x16 acc = f32x16{};
-  const int nch = R / GRC;
-#pragma unroll
-  for (int k = 0; k < PF; k++)
-    if (k < nch) {
-      ga[k].issue(A, a_i, a_r, i0, k * GRC);
-      gb[k].issue(B, b_j, b_r, j0, k * GRC);
-    }
-  const int ai = wi + 16 * (blk & 1) + c, bj = wj + 16 * (blk >> 1) + c;
-  for (int ch0 = 0; ch0 < nch; ch0 += PF) {
-#pragma unroll
-    for (int k = 0; k < PF; k++) {
-      const int ch = ch0 + k;
-      if (ch < nch) {
-        __syncthreads();  // previous chunk fully consumed
-        ga[k].commit(As);
-        gb[k].commit(Bs);
-        __syncthreads();
-        if (ch + PF < nch) {
-          ga[k].issue(A, a_i, a_r, i0, (ch + PF) * GRC);
-          gb[k].issue(B, b_j, b_r, j0, (ch + PF) * GRC);
-        }
-#pragma unroll
-        for (int r0 = 0; r0 < GRC; r0 += 4) {
-          float a[4], b[4];
-          GemmOperand<ARC, GS>::load4(As, ai, r0, a);
-          GemmOperand<BRC, GS>::load4(Bs, bj, r0, b);
-#pragma unroll
-          for (int e = 0; e < 4; e++) acc = otx_mfma16(a[e], b[e], acc);
-        }
+  // The steps of SN sub-chunks from byte OFF of the addresses on.
+  const auto steps = [&](auto offc, auto subc, const uint32_t (&pa)[TA::NA], const uint32_t (&pb)[TB::NA]) {
+    constexpr int OFF = decltype(offc)::value, NG = decltype(subc)::value * 8 / SPG;
+    const auto rd = [&](auto gc) {
+      constexpr int G = decltype(gc)::value, BK = G % 3;
+      OtxUnroll<0, SPG>::run([&](auto ec) {
+        constexpr int E = decltype(ec)::value, ST = G * SPG + E;
+        OtxUnroll<0, NB>::run([&](auto xc) {
+          constexpr int X = decltype(xc)::value;
+          otx_lds_bf16<OFF + TA::off(ST, X)>(opr[BK][E * 2 * NB + X], pa[TA::which(ST)]);
+          otx_lds_bf16<OFF + TB::off(ST, X)>(opr[BK][E * 2 * NB + NB + X], pb[TB::which(ST)]);
+        });
+      });
+    };
+    rd(std::integral_constant<int, 0>{});
+    rd(std::integral_constant<int, 1>{});
+    OtxUnroll<0, NG>::run([&](auto gc) {
+      constexpr int G = decltype(gc)::value, BK = G % 3;
+      if constexpr (G + 2 < NG) {
+        rd(std::integral_constant<int, G + 2>{});
+        otx_lds_wait<8>(opr[BK]);
+      } else if constexpr (G + 1 < NG) {
+        otx_lds_wait<4>(opr[BK]);
+      } else {
+        otx_lds_wait<0>(opr[BK]);
       }
-    }
-  }
-  // acc[r]: block r / 4 (i-block (r / 4) & 1, j-block (r / 4) >> 1), row 4 (L / 16) + r % 4, column L % 16.
+      OtxUnroll<0, SPG>::run([&](auto ec) {
+        constexpr int E = decltype(ec)::value;
 #pragma unroll
-  for (int r = 0; r < 16; r++) {
-    const int bb = r >> 2;
-    const int i = i0 + wi + 16 * (bb & 1) + 4 * blk + (r & 3);
-    const long o = (long)i * ldc + j0 + wj + 16 * (bb >> 1) + c;
-    if constexpr (OUT_F32)
-      static_cast<float*>(C)[o] = acc[r];
-    else
-      static_cast<uint16_t*>(C)[o] = otx_f32_to_bf16(acc[r]);
+        for (int x = 0; x < NB; x++)
+#pragma unroll
+          for (int y = 0; y < NB; y++)
+            acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(opr[BK][E * 2 * NB + x], opr[BK][E * 2 * NB + NB + y],
+                                                             acc[x][y], 0, 0, 0);
+      });
+      // bank BK is consumed before it is read again
+#pragma unroll
+      for (int x = 0; x < NB; x++)
+#pragma unroll
+        for (int y = 0; y < NB; y++) asm volatile("" : "+v"(acc[x][y]));
+    });
+  };
+  int st = 0;
+  const auto stage = [&](auto sc) {
+    constexpr int S = decltype(sc)::value;
+    if (st == nst) return false;
+    // stage st has landed for every wave (the copies of at most P - 1 later ones stay in
+    // flight), and stage st - 1 is no longer read
+    if (nst - st > 2) gemm_vm_wait<2 * NDMA>();
+    else if (nst - st == 2) gemm_vm_wait<NDMA>();
+    else gemm_vm_wait<0>();
+    asm volatile("s_barrier" ::: "memory");
+    if (st + P < nst) issue(st + P, smem + ((S + P) % NS) * SLOT);
+    if (SR * st + SR <= R) {
+      steps(std::integral_constant<int, S * SLOT>{}, std::integral_constant<int, SUBS>{}, la, lb);
+      st++;
+      return true;
+    }
+    // a last stage that is not whole: its sub-chunks one by one (R is a multiple of 32)
+    uint32_t pa[TA::NA], pb[TB::NA];
+    for (int sub = 0; SR * st + 32 * sub < R; sub++) {
+#pragma unroll
+      for (int u = 0; u < TA::NA; u++) pa[u] = la[u] + S * SLOT + sub * TA::SUB;
+#pragma unroll
+      for (int u = 0; u < TB::NA; u++) pb[u] = lb[u] + S * SLOT + sub * TB::SUB;
+      steps(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, pa, pb);
+    }
+    return false;
+  };
+  while (OtxAll<0, NS>::run(stage)) {
   }
+#pragma unroll
+  for (int x = 0; x < NB; x++)
+#pragma unroll
+    for (int y = 0; y < NB; y++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const long o = (long)(i0 + wi + 16 * x + 4 * g + q) * ldc + j0 + wj + 16 * y + c;
+        if constexpr (OUT_F32)
+          static_cast<float*>(C)[o] = acc[x][y][q];
+        else
+          static_cast<uint16_t*>(C)[o] = otx_f32_to_bf16(acc[x][y][q]);
+      }
 }
 
-// The bf16-tile kernel serves both forms, except the narrow form of an
-// r-contiguous A with an i-contiguous B (dx = dy w), where the binary32-tile
-// kernel measured 11-14 % faster (its A commit is shared by half as many
-// MFMAs there as in the wide form).
 template <bool ARC, bool BRC, int WJ>
 static hipError_t launch_gemm_w(const void* A, long a_i, long a_r, const void* B, long b_j, long b_r, void* C,
                                 long ldc, int M, int N, int R, bool out_f32, hipStream_t st) {
   const dim3 grid((unsigned)((M / GT) * (N / (2 * WJ)))), block(256);
-  if constexpr (!(WJ == 32 && ARC && !BRC)) {
-    if (out_f32)
-      hipLaunchKernelGGL((gemm_bf16_v2_kernel<ARC, BRC, true, WJ>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
-                         (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
-    else
-      hipLaunchKernelGGL((gemm_bf16_v2_kernel<ARC, BRC, false, WJ>), grid, block, 0, st, (const uint16_t*)A, a_i,
-                         a_r, (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
-  } else {
-    if (out_f32)
-      hipLaunchKernelGGL((gemm_bf16_kernel<ARC, BRC, true, WJ>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
-                         (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
-    else
-      hipLaunchKernelGGL((gemm_bf16_kernel<ARC, BRC, false, WJ>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
-                         (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
-  }
-  return hipGetLastError();
-}
-
-template <bool ARC, bool BRC>
-static hipError_t launch_gemm_small(const void* A, long a_i, long a_r, const void* B, long b_j, long b_r, void* C,
-                                    long ldc, int M, int N, int R, bool out_f32, hipStream_t st) {
-  const dim3 grid((unsigned)((M / 64) * (N / 64))), block(256);
   if (out_f32)
-    hipLaunchKernelGGL((gemm_bf16_small_kernel<ARC, BRC, true>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
+    hipLaunchKernelGGL((gemm_bf16_v2_kernel<ARC, BRC, true, WJ>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
                        (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
   else
-    hipLaunchKernelGGL((gemm_bf16_small_kernel<ARC, BRC, false>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
+    hipLaunchKernelGGL((gemm_bf16_v2_kernel<ARC, BRC, false, WJ>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
                        (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
   return hipGetLastError();
 }
 
-// form: 0 wide (128 x 128), 1 narrow (128 x 64), 2 small (64 x 64).
+template <bool ARC, bool BRC, int NB>
+static hipError_t launch_gemm_k4(const void* A, long a_i, long a_r, const void* B, long b_j, long b_r, void* C,
+                                 long ldc, int M, int N, int R, bool out_f32, hipStream_t st) {
+  const dim3 grid((unsigned)((M / (32 * NB)) * (N / (32 * NB)))), block(256);
+  if (out_f32)
+    hipLaunchKernelGGL((gemm_bf16_k4_kernel<ARC, BRC, true, NB>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
+                       (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
+  else
+    hipLaunchKernelGGL((gemm_bf16_k4_kernel<ARC, BRC, false, NB>), grid, block, 0, st, (const uint16_t*)A, a_i, a_r,
+                       (const uint16_t*)B, b_j, b_r, C, ldc, M, N, R);
+  return hipGetLastError();
+}
+
+// form: 0 wide (128 x 128), 1 narrow (128 x 64), 2 small (64 x 64), 3 smallest (32 x 32).
 template <bool ARC, bool BRC>
 static hipError_t launch_gemm_t(const void* A, long a_i, long a_r, const void* B, long b_j, long b_r, void* C,
                                 long ldc, int M, int N, int R, bool out_f32, int form, hipStream_t st) {
-  if (form == 2) return launch_gemm_small<ARC, BRC>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
+  if (form == 3) return launch_gemm_k4<ARC, BRC, 1>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
+  if (form == 2) return launch_gemm_k4<ARC, BRC, 2>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
   if (form == 1) return launch_gemm_w<ARC, BRC, 32>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
   return launch_gemm_w<ARC, BRC, 64>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
 }
 
-// Tile choice (every form gives the same bytes).  With t tiles of 128 x 128 on
-// n CUs, the busiest CU works through ceil(t / n) wide tiles, ceil(2t / n)
-// narrow ones (half the work each) or ceil(4t / n) small ones (a quarter).
-// Per unit of work the narrow form costs 2-6 % more than the wide one (one
-// MFMA per operand read of A instead of two) and the small form about 10 %
-// more (a quarter of the work per chunk for the same barriers and staging), so
-// the launcher takes the form whose busiest CU does the least weighted work:
-// t = 5.5 n (the OPEN-1B gate/up weight gradient, 1408 tiles) gives six wide,
-// eleven narrow or 22 small tiles (5.5 wide tiles' work), and the narrow form
-// wins (-3.2 % with binary32 tiles, -6 to -9 % with bf16 tiles); t = n / 4 (the
-// k and v weight gradients, 64 tiles) leaves three quarters of the CUs idle in
-// the wide form, half of them in the narrow one and none in the small one (-23 %
-// against narrow with binary32 tiles, -10 % against the bf16-tile narrow form).  At t = n (one tile per
-// CU) the wide and narrow forms are equal.  variant 1, 2, 3 force the wide,
-// narrow and small form.
-static int gemm_form(int M, int N, int variant) {
+// Tile choice (every form gives the same bytes): the form whose busiest CU has the least to
+// do.  With t tiles of 128 x 128 on n CUs that CU works through m = ceil(t / n) wide tiles,
+// ceil(2t / n) narrow, ceil(4t / n) 64 x 64 or ceil(16t / n) 32 x 32 ones.  What a tile takes
+// over its matrix instructions (fitted to products of R 512 to 8192 and 16 to 5632 tiles,
+// 4 us of launch taken off) is, for m = 1, 2 and more:
+//                        y = x w^T          dx = dy w          dw = dy^T x
+//   wide               1.24 1.17 1.12     1.19 1.14 1.10     1.09 1.10 1.085
+//   narrow             1.43 1.26 1.16     1.40 1.27 1.18     1.19 1.11 1.10
+//   64 x 64            1.25 1.17 1.15     1.25 1.17 1.18     1.25 1.17 1.18
+//   32 x 32            1.41 throughout
+// (few waves per SIMD expose a wide tile's waits; an r-contiguous operand costs the wide and
+// narrow forms their commits, where the small forms copy it as it is).  Measured, before
+// and now: 256 x 512 over 2048 (the k projection of a short batch) 46.7 -> 13.8 us, 32 x 32
+// tiles; 1024 x 1024 over 1024 27 -> 21 us and 1280 x 5632 over 2048 267 -> 229 us, 64 x 64;
+// 8192 x 11264 over 2048 stays with the wide form's 2.71 ms.  The narrow form is left to
+// products with both operands i-contiguous (11264 x 2048 over 8192, 5.5 wide tiles per CU:
+// 2.66 ms against 2.84 and 2.86); elsewhere the 64 x 64 form is as fast or faster.
+// variant 1, 2 and 3 force the wide, the narrow and the 64 x 64 form.
+static int gemm_form(int M, int N, bool arc, bool brc, int variant) {
   if (variant >= 1) return variant - 1;
   const long t = (long)(M / GT) * (N / GT), n = otx_cu_count();
-  const long wide = 400 * ((t + n - 1) / n), narrow = 208 * ((2 * t + n - 1) / n),
-             small = 110 * ((4 * t + n - 1) / n);  // in 1/400 of a wide tile's work
-  if (small < wide && small < narrow) return 2;
-  return narrow < wide ? 1 : 0;
+  const int lay = arc && brc ? 0 : arc || brc ? 1 : 2;
+  static const long over[3][3][3] = {{{1240, 1170, 1120}, {1190, 1140, 1100}, {1090, 1100, 1085}},
+                                     {{1430, 1260, 1160}, {1400, 1270, 1180}, {1190, 1110, 1100}},
+                                     {{1250, 1170, 1150}, {1250, 1170, 1180}, {1250, 1170, 1180}}};
+  long best = 1410 * ((16 * t + n - 1) / n);  // in 1/16000 of a wide tile's matrix instructions
+  int form = 3;
+  for (int f = 2; f >= 0; f--) {
+    if (f == 1 && lay != 2) continue;
+    const long m = ((t << f) + n - 1) / n, cost = m * (16 >> f) * over[f][lay][m < 3 ? m - 1 : 2];
+    if (cost <= best) {
+      best = cost;
+      form = f;
+    }
+  }
+  return form;
 }
 
 hipError_t launch_gemm(const void* A, long a_i, long a_r, const void* B, long b_j, long b_r, void* C, long ldc, int M,
                        int N, int R, bool out_f32, int variant, hipStream_t st) {
   const bool arc = a_r == 1, brc = b_r == 1;
-  const int f = gemm_form(M, N, variant);
+  const int f = gemm_form(M, N, arc, brc, variant);
   if (arc && brc) return launch_gemm_t<true, true>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, f, st);
   if (arc) return launch_gemm_t<true, false>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, f, st);
   if (brc) return launch_gemm_t<false, true>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, f, st);
