@@ -21,6 +21,9 @@
 //          the device only once (its long chunks would then set the time).
 //   dq   : one wave per 32-query block; dQ^T chain over the processed keys
 //          reading the stored dS tiles, scaled by sigma at the end.
+// The dkdv of binary32 inputs, and dkdv and dq of grids too small for one wave
+// per block, are in attn_tile.hip (four waves per block); the rules stand at the
+// launcher below.
 // Every output element is produced by a single lane in a single fixed order.
 #include "otx_common.h"
 
@@ -92,227 +95,6 @@ __device__ __forceinline__ void load_dpair(const T* row, int L, float* a0, float
   }
 }
 
-template <typename T, int D, int NWK>
-__global__ __launch_bounds__(64 * NWK) void attn_dkdv_kernel(
-    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ dO,
-    const float* __restrict__ lse, const float* __restrict__ dsum, T* __restrict__ dk, T* __restrict__ dv,
-    float* __restrict__ ws_ds, int B, int H, int Hkv, int S, int window, float sigma, int order) {
-  constexpr int ES = sizeof(T);
-  constexpr int VEC = Elem<T>::VEC;
-  constexpr int PADE = 16 / ES;
-  constexpr int KP = D + PADE;
-  constexpr int CH = D * ES / 16;
-  constexpr int NI = D / 64;
-  constexpr int KV_ELEMS = 2 * NWK * 32 * KP;
-  constexpr int QD_ELEMS = 2 * 64 * KP;
-  __shared__ __align__(16) T smem_t[KV_ELEMS + QD_ELEMS];
-  __shared__ float Ls[64], Ds[64];
-  __shared__ double tab[OTX_EXP_LE0_TAB_N];
-  T* Ks = smem_t;
-  T* Vs = Ks + NWK * 32 * KP;
-  T* Qs = Vs + NWK * 32 * KP;
-  T* dOs = Qs + 64 * KP;
-
-  const int nkt = S / OTX_BLK;
-  const int nchunk = (nkt + NWK - 1) / NWK;
-  const int BG = B * Hkv;
-  const int G = H / Hkv;
-  const int bid = blockIdx.x;
-  int chunk, bg;
-  if (order == 0) {  // low key chunks see the most query blocks: launch them first
-    chunk = bid / BG;
-    bg = bid % BG;
-  } else {
-    chunk = nchunk - 1 - bid % nchunk;
-    bg = bid / nchunk;
-  }
-  const int b = bg / Hkv, g = bg % Hkv;
-  const int wave = threadIdx.x >> 6, L = threadIdx.x & 63, hh = L >> 5, c = L & 31;
-  const int kt = chunk * NWK + wave;
-  const bool wactive = kt < nkt;
-  const int kt0 = chunk * NWK;
-  const int ktl = (kt0 + NWK < nkt ? kt0 + NWK : nkt) - 1;
-  const T* kg = k + (size_t)bg * S * D;
-  const T* vg = v + (size_t)bg * S * D;
-  const long tiles_per_head = otx_tile_offset(nkt, window);
-
-  otx_load_exp_table(tab);
-  // K and V rows of the workgroup's key blocks.
-  for (int idx = threadIdx.x; idx < NWK * 32 * CH; idx += 64 * NWK) {
-    const int row = idx / CH, ch = idx % CH;
-    const int key = kt0 * OTX_BLK + row;
-    if (key < S) {
-      *reinterpret_cast<uint4*>(Ks + row * KP + ch * VEC) =
-          *reinterpret_cast<const uint4*>(kg + (size_t)key * D + ch * VEC);
-      *reinterpret_cast<uint4*>(Vs + row * KP + ch * VEC) =
-          *reinterpret_cast<const uint4*>(vg + (size_t)key * D + ch * VEC);
-    }
-  }
-
-  f32x32 accV[NI], accK[NI];
-#pragma unroll
-  for (int n = 0; n < NI; n++) { accV[n] = f32x32{}; accK[n] = f32x32{}; }
-
-  const int qhi = wactive ? otx_qblock_hi(kt, window, nkt) : -1;
-  const int u_begin = kt0 >> 1;
-  const int u_end = otx_qblock_hi(ktl, window, nkt) >> 1;
-  const int key = kt * OTX_BLK + c;
-  const T* krow = Ks + (wave * 32 + c) * KP;
-  const T* vrow = Vs + (wave * 32 + c) * KP;
-
-  for (int r = 0; r < G; r++) {
-    const int h = g * G + r;
-    const size_t bh = (size_t)b * H + h;
-    const T* qg = q + bh * S * D;
-    const T* dog = dO + bh * S * D;
-    for (int u = u_begin; u <= u_end; u++) {
-      __syncthreads();
-      for (int idx = threadIdx.x; idx < 64 * CH; idx += 64 * NWK) {
-        const int row = idx / CH, ch = idx % CH;
-        const int qrow = 64 * u + row;
-        if (qrow < S) {
-          *reinterpret_cast<uint4*>(Qs + row * KP + ch * VEC) =
-              *reinterpret_cast<const uint4*>(qg + (size_t)qrow * D + ch * VEC);
-          *reinterpret_cast<uint4*>(dOs + row * KP + ch * VEC) =
-              *reinterpret_cast<const uint4*>(dog + (size_t)qrow * D + ch * VEC);
-        }
-      }
-      for (int idx = threadIdx.x; idx < 64; idx += 64 * NWK) {
-        const int qrow = 64 * u + idx;
-        if (qrow < S) {
-          Ls[idx] = lse[bh * S + qrow];
-          Ds[idx] = dsum[bh * S + qrow];
-        }
-      }
-      __syncthreads();
-      const int qa = 2 * u, qb = 2 * u + 1;
-      const bool doA = wactive && qa >= kt && qa <= qhi;
-      const bool doB = wactive && qb >= kt && qb <= qhi;
-      if (!(doA || doB)) continue;
-
-      // ---- S = Q K^T and dP = dO V^T (two interleaved chains over d) ----
-      f32x32 sacc = f32x32{}, pacc = f32x32{};
-      const T* qrow = Qs + (hh * 32 + c) * KP;
-      const T* drow = dOs + (hh * 32 + c) * KP;
-#pragma unroll
-      for (int d0 = 0; d0 < D; d0 += VEC) {
-        const uint4 qv = *reinterpret_cast<const uint4*>(qrow + d0);
-        const uint4 kv = *reinterpret_cast<const uint4*>(krow + d0);
-        const uint4 dv4 = *reinterpret_cast<const uint4*>(drow + d0);
-        const uint4 vv = *reinterpret_cast<const uint4*>(vrow + d0);
-#pragma unroll
-        for (int e = 0; e < VEC; e++) {
-          sacc = otx_mfma(Elem<T>::get(qv, e), Elem<T>::get(kv, e), sacc);
-          pacc = otx_mfma(Elem<T>::get(dv4, e), Elem<T>::get(vv, e), pacc);
-        }
-      }
-      float P[32], dS[32];
-#pragma unroll
-      for (int rr = 0; rr < 16; rr++) {
-        float x = sacc[rr], y = sacc[16 + rr];
-        otx_swap_halves(x, y);
-        P[otx_row(rr, 0)] = x;
-        P[otx_row(rr, 1)] = y;
-        float x2 = pacc[rr], y2 = pacc[16 + rr];
-        otx_swap_halves(x2, y2);
-        dS[otx_row(rr, 0)] = x2;
-        dS[otx_row(rr, 1)] = y2;
-      }
-      // lane (hh, c): key `key`, queries (qa + hh) * 32 + i for i = 0..31
-      const int qbase = (qa + hh) * OTX_BLK;
-      const bool hact = hh ? doB : doA;
-      float ex[32];
-#pragma unroll
-      for (int i = 0; i < 32; i++) {
-        const bool msk = !hact || otx_masked(qbase + i, key, window);
-        const float sv = P[i] * sigma;
-        ex[i] = msk ? -__builtin_inff() : sv - Ls[hh * 32 + i];  // exp(-inf) = +0 for masked pairs
-      }
-      otx_exp_n<32, true, 16>(ex, tab);
-#pragma unroll
-      for (int i = 0; i < 32; i++) {
-        P[i] = ex[i];
-        dS[i] = P[i] * (dS[i] - Ds[hh * 32 + i]);
-      }
-      // ---- export dS for the dQ kernel: tile (query block, key block), row-major ----
-      if ((hh == 0 && doA) || (hh == 1 && doB)) {
-        const int qblk = qa + hh;
-        float* tile = ws_ds + ((long)bh * tiles_per_head + otx_tile_offset(qblk, window) +
-                               (kt - otx_kblock_lo(qblk, window))) * (OTX_BLK * OTX_BLK);
-#pragma unroll
-        for (int i = 0; i < 32; i++) tile[i * 32 + c] = dS[i];
-      }
-      // ---- dV^T += dO^T P, dK^T += Q^T dS (serial over queries) ----
-      if (doA) {
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-          float plo, phi, slo, shi;
-          otx_bcast_halves(P[i], &plo, &phi);
-          otx_bcast_halves(dS[i], &slo, &shi);
-          P[i] = phi;
-          dS[i] = shi;
-          float a0, a1, b0, b1;
-          load_dpair<T, D>(dOs + i * KP, L, &a0, &a1);
-          load_dpair<T, D>(Qs + i * KP, L, &b0, &b1);
-          accV[0] = otx_mfma(a0, plo, accV[0]);
-          accK[0] = otx_mfma(b0, slo, accK[0]);
-          if constexpr (NI == 2) {
-            accV[1] = otx_mfma(a1, plo, accV[1]);
-            accK[1] = otx_mfma(b1, slo, accK[1]);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-          float plo, phi, slo, shi;
-          otx_bcast_halves(P[i], &plo, &phi);
-          otx_bcast_halves(dS[i], &slo, &shi);
-          P[i] = phi;
-          dS[i] = shi;
-        }
-      }
-      if (doB) {
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-          float a0, a1, b0, b1;
-          load_dpair<T, D>(dOs + (32 + i) * KP, L, &a0, &a1);
-          load_dpair<T, D>(Qs + (32 + i) * KP, L, &b0, &b1);
-          accV[0] = otx_mfma(a0, P[i], accV[0]);
-          accK[0] = otx_mfma(b0, dS[i], accK[0]);
-          if constexpr (NI == 2) {
-            accV[1] = otx_mfma(a1, P[i], accV[1]);
-            accK[1] = otx_mfma(b1, dS[i], accK[1]);
-          }
-        }
-      }
-    }
-  }
-
-  // ---- epilogue: dV as is, dK = RN(acc * sigma); transpose through LDS ----
-  __syncthreads();
-  T* Vo = smem_t + wave * 2 * 32 * KP;
-  T* Ko = Vo + 32 * KP;
-  if (wactive) {
-#pragma unroll
-    for (int n = 0; n < NI; n++)
-#pragma unroll
-      for (int r = 0; r < 32; r++) {
-        const int d = dpair_row<D>(n, r, hh);
-        Vo[c * KP + d] = Elem<T>::put(accV[n][r]);
-        Ko[c * KP + d] = Elem<T>::put(accK[n][r] * sigma);
-      }
-  }
-  __syncthreads();
-  if (wactive) {
-    for (int idx = L; idx < 32 * CH; idx += 64) {
-      const int row = idx / CH, ch = idx % CH;
-      const size_t off = ((size_t)bg * S + kt * OTX_BLK + row) * D + ch * VEC;
-      *reinterpret_cast<uint4*>(dv + off) = *reinterpret_cast<const uint4*>(Vo + row * KP + ch * VEC);
-      *reinterpret_cast<uint4*>(dk + off) = *reinterpret_cast<const uint4*>(Ko + row * KP + ch * VEC);
-    }
-  }
-}
-
 // bf16 dK/dV kernel.  One wave (and one SIMD) per 32-key block, NWK waves
 // per workgroup, one workgroup per CU.  LDS holds the workgroup's own K and V
 // rows for the whole kernel and two slots of the streamed query side: 64-row
@@ -321,7 +103,7 @@ __global__ __launch_bounds__(64 * NWK) void attn_dkdv_kernel(
 // bf16, padded to 2D + 16 bytes.  Every chain operand is read with
 // ds_read_u16_d16_hi (binary32 value of a bf16, no conversion instruction)
 // under hand-kept lgkmcnt accounting: groups of 4 reads, two groups ahead (at
-// most 12 outstanding).  Arithmetic order is the same as in attn_dkdv_kernel.
+// most 12 outstanding).
 template <int D, int NWK, bool SC>
 __global__ __launch_bounds__(64 * NWK, 1) void attn_dkdv_bf16_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
@@ -1276,6 +1058,12 @@ __global__ __launch_bounds__(64 * NWQ) void attn_dq_kernel(const T* __restrict__
   }
 }
 
+hipError_t launch_dkdv_tile(int dtype, int D, int n16, const void* q, const void* k, const void* v, const void* dO,
+                            const float* lse, const float* dsum, void* dk, void* dv, float* ds, int B, int H, int Hkv,
+                            int S, int window, float sigma, int order, const float* scache, hipStream_t st);
+hipError_t launch_dq_tile(int dtype, int D, int n16, const void* k, const float* ds, void* dq, int B, int H, int Hkv,
+                          int S, int window, float sigma, int order, hipStream_t st);
+
 template <typename T, int D>
 static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void* v, const void* o, const float* lse,
                                const void* dO, void* dq, void* dk, void* dv, float* dsum, float* ds, int B, int H,
@@ -1291,10 +1079,8 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
     if (e != hipSuccess) return e;
   }
   const int nt = S / OTX_BLK;
-#define OTX_LAUNCH_DKDV(NW)                                                                                      \
-  hipLaunchKernelGGL((attn_dkdv_kernel<T, D, NW>), dim3((unsigned)(((nt + NW - 1) / NW) * B * Hkv)),            \
-                     dim3(64 * NW), 0, st, (const T*)q, (const T*)k, (const T*)v, (const T*)dO, lse, dsum,      \
-                     (T*)dk, (T*)dv, ds, B, H, Hkv, S, window, sigma, order)
+  const long cus = otx_cu_count();
+  const long nkb = (long)nt * B * Hkv, nqb = (long)nt * B * H;  // key and query blocks of all heads
   // dQ workgroups: head-grouped (see attn_dq_kernel) for GQA in the default launch order.
   auto dq_hg = [&](int nw) { return (nw > 1 && (H / Hkv) % nw == 0 && order == 0) ? 1 : 0; };
   auto dq_nu = [&](int nw) { return (long)(dq_hg(nw) ? nt : (nt + nw - 1) / nw); };
@@ -1306,7 +1092,22 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
                                      dq_bu(NW))),                                                                \
                      dim3(64 * NW), 0, st, (const T*)k, ds, (T*)dq, B, H, Hkv, S, window, sigma, dq_order(NW),     \
                      dq_hg(NW))
+  // dK/dV on the tile kernel (every choice gives the same bits).  binary32 always: it replaced a form with
+  // one wave per key block, one wave per SIMD (4 heads x 256, D 64: 71 -> 12 us; 8 heads, 2 KV heads x 1024,
+  // D 128: 1457 -> 222; 16 heads, 4 KV heads x 2 x 4096: 6410 -> 2520).  bf16 in the default launch while the
+  // key blocks are at most two per CU (with the score cache, 16 heads x 1024, D 128: 118 -> 95 us; 16 heads,
+  // 4 KV heads x 2048: 886 -> 492; at nkb 1024, 32 heads x 1024: 137 against 139, D 64: 87 against 89), or
+  // eight when the scores are recomputed, where the other forms have more to do in one wave (nkb 1024: 188 ->
+  // 181; nkb 2048, window 256: 216 -> 171; nkb 4096: 1158 against 1234).  Sixteen keys per workgroup rather
+  // than 32 up to two key blocks per CU (nkb 512: 95 against 106 us; nkb 1024: 165 against 139), half a block
+  // under a window (nkb 128: 20 against 29; nkb 256: 29.2 against 29.1; nkb 512: 51 against 46).
+  const bool tile_dkdv = sizeof(T) == 4 || (nw == 4 && nkb <= (scache != nullptr ? 2 : 8) * cus);
   if (!(stages & 2)) {
+  } else if (tile_dkdv) {
+    const int n16 = nw == 4 ? (2 * nkb <= (window > 0 ? 1 : 4) * cus ? 1 : 2) : nw;
+    e = launch_dkdv_tile(sizeof(T) == 2, D, n16, q, k, v, dO, lse, dsum, dk, dv, ds, B, H, Hkv, S, window, sigma, order,
+                         scache, st);
+    if (e != hipSuccess) return e;
   } else if constexpr (sizeof(T) == 2) {
 #define OTX_LAUNCH_DKDV_BF16(NW, SC)                                                                         \
   hipLaunchKernelGGL((attn_dkdv_bf16_kernel<D, NW, SC>), dim3((unsigned)(((nt + NW - 1) / NW) * B * Hkv)),    \
@@ -1336,20 +1137,18 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
     }
 #undef OTX_LAUNCH_DKDV_BF16
 #undef OTX_LAUNCH_DKDV_KB2
-  } else {
-    if (scache != nullptr) return hipErrorInvalidValue;  // the score cache is a bf16-path feature
-    // fp32 with D = 128 holds twice the LDS per key block: at most 2 key blocks per workgroup.
-    constexpr bool kWide = D != 128;
-    switch (nw) {
-      case 4:
-        if constexpr (kWide) OTX_LAUNCH_DKDV(4); else OTX_LAUNCH_DKDV(2);
-        break;
-      case 2: OTX_LAUNCH_DKDV(2); break;
-      default: OTX_LAUNCH_DKDV(1); break;
-    }
   }
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  // dQ on the tile kernel (the same bits): in the default launch up to four query blocks per CU, two under a
+  // window; with bf16 K two at D 64, and eight or four at D 128.  Beyond, its loads (a K row for 32 queries
+  // where the other form shares it among 128) set its time.  bf16, D 128, nqb 512: 69 -> 30 us; 1024: 137 ->
+  // 93; 2048: 98 -> 83; 4096: 302 against 318; window 256, nqb 1024: 30 -> 25 (four heads a group: 25 against
+  // 27); D 64, nqb 512: 39 -> 26, nqb 1024: 40 against 44.  binary32, D 128, nqb 1024: 85 -> 69, 2048: 113
+  // against 117; window 256, nqb 512: 32 -> 19, 1024: 30 against 34.
+  const long dq_lim = sizeof(T) == 4 ? (window > 0 ? 2 : 4) : D == 64 ? 2 : (window > 0 ? 4 : 8);
+  if ((stages & 4) && nw == 4 && nqb <= dq_lim * cus)
+    return launch_dq_tile(sizeof(T) == 2, D, nqb <= 2 * cus ? 1 : 2, k, ds, dq, B, H, Hkv, S, window, sigma, order, st);
   if (stages & 4) {
     switch (nw) {
       case 4: OTX_LAUNCH_DQ(4); break;
@@ -1357,7 +1156,6 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
       default: OTX_LAUNCH_DQ(1); break;
     }
   }
-#undef OTX_LAUNCH_DKDV
 #undef OTX_LAUNCH_DQ
   return hipGetLastError();
 }

@@ -1,0 +1,69 @@
+"""The four-waves-per-block attention kernels (forward, dK/dV, dQ) against the
+CPU oracle and against the one-wave-per-block kernels, byte for byte, at the
+edges of their tiles and on both sides of every limit of the launcher's choice.
+
+In the default launch the choice goes by the number of 32-row blocks over all
+heads (256 compute units: forward 256, 512 and 1024 blocks, dK/dV 128, 512 and
+2048 key blocks, dQ 512, 1024 and 2048); variants 1 and 2 keep one form each.
+The comparison is exact: both forms are the same serial folds.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from attn_util import assert_bits_equal, gpu_fwd_bwd, make, oracle_fwd_bwd
+from open_transformers_amd.nn import flash_attention as fa
+
+pytestmark = pytest.mark.gpu
+NAMES = ("o", "lse", "dq", "dk", "dv")
+
+# (B, H, Hkv, S, D, window): one block; odd block counts (the last pair of key or query blocks is half empty); a window
+# of one block, of an odd number of blocks and longer than the sequence; query groups
+SMALL = [(1, 1, 1, 32, 64, 0), (1, 2, 1, 64, 128, 0), (2, 3, 1, 96, 128, 32), (1, 2, 2, 160, 64, 96),
+         (1, 4, 2, 224, 128, 64), (1, 2, 1, 96, 64, 320), (1, 1, 1, 288, 128, 0)]
+
+
+@pytest.mark.parametrize("shape", SMALL, ids=[f"s{i}" for i in range(len(SMALL))])
+@pytest.mark.parametrize("form", ["f32-0", "f32-1", "f32-2", "bf16", "bf16-cache"])
+def test_gpu_tile_small(shape, form):
+    B, H, Hkv, S, D, window = shape
+    bf16 = form.startswith("bf16")
+    variant = 0 if bf16 else int(form[-1])
+    print(form, shape, flush=True)
+    inp = make(B, H, Hkv, S, D, dtype="bf16" if bf16 else "f32", seed=S + D, qk_scale=3.0)
+    got = gpu_fwd_bwd(inp, window, bf16, variant=variant, score_cache=form == "bf16-cache")
+    ref = oracle_fwd_bwd(inp, window, bf16)
+    for n in NAMES:
+        assert_bits_equal(got[n], ref[n], n)
+
+
+# block counts over all heads on either side of a limit: (B, H, Hkv, S, D, window)
+LIMITS = [(1, 16, 8, 512, 128, 64), (1, 16, 8, 544, 128, 64), (1, 16, 16, 1024, 64, 0), (1, 16, 16, 1056, 64, 0),
+          (1, 16, 16, 1024, 128, 96), (1, 16, 16, 1056, 128, 96), (1, 32, 32, 1024, 128, 0), (1, 32, 32, 1056, 128, 0),
+          (2, 32, 16, 1024, 64, 64), (2, 32, 32, 1024, 128, 64), (2, 33, 33, 1024, 128, 64), (1, 32, 2, 1024, 128, 256)]
+
+
+@pytest.mark.parametrize("shape", LIMITS, ids=[f"l{i}" for i in range(len(LIMITS))])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_gpu_tile_choice(shape, dtype):
+    """Variants 0, 1 and 2, with the scores recomputed and (bf16) read from the cache of another variant's forward."""
+    B, H, Hkv, S, D, window = shape
+    print(dtype, shape, flush=True)
+    T = torch.float32 if dtype == "f32" else torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(S + H)
+    q, k, v, do = (torch.randn(B, h, S, D, device="cuda", generator=g).to(T) for h in (H, Hkv, Hkv, H))
+    o, lse = fa.flash_attention_forward(q, k, v, window, variant=2)
+    ref = fa.flash_attention_backward(q, k, v, o, lse, do, window, variant=2)
+    for variant in (0, 1):
+        o2, lse2 = fa.flash_attention_forward(q, k, v, window, variant=variant)
+        assert torch.equal(o, o2) and torch.equal(lse, lse2), variant
+        for a, b, n in zip(ref, fa.flash_attention_backward(q, k, v, o, lse, do, window, variant=variant), NAMES[2:]):
+            assert torch.equal(a, b), (n, variant)
+    if dtype == "bf16":
+        sc = [fa.flash_attention_forward_sc(q, k, v, window, variant=x) for x in (0, 2)]
+        for a, b in zip(*sc):
+            assert torch.equal(a, b)
+        for a, b, n in zip(ref, fa.flash_attention_backward(q, k, v, o, lse, do, window, score_cache=sc[1][2]),
+                           NAMES[2:]):
+            assert torch.equal(a, b), (n, "cache")
