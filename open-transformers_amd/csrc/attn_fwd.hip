@@ -601,6 +601,32 @@ static hipError_t launch_fwd_t(const void* q, const void* k, const void* v, void
   return hipGetLastError();
 }
 
+// Whether a forward takes attn_fwd_tile_kernel and with how many 16-query tiles
+// per workgroup (0: the one-wave-per-block kernel); every choice gives the same
+// bits.  nb: the query blocks of all heads.  In the default launch the tile
+// kernel serves up to four blocks per CU under a full causal mask and two under
+// a window, where the one-wave-per-block kernel has at most one wave per SIMD and
+// waits for the longest rows.  256 CUs, bf16, D 128: 16 heads x 1024 (nb 512)
+// 166 -> 76 us, int8-PV 134 -> 69; 16 x 2048 (nb 1024) 322 -> 226, int8-PV, four
+// heads a group, 255 -> 184; window 256, nb 512: 67 -> 39, int8-PV 59 -> 39.
+// Beyond it is no faster: nb 2048 228 against 220 and 119 against 126, int8-PV
+// 172 against 183; nb 4096 636 against 803; window 256, nb 1024, four heads a
+// group 58 against 72, int8-PV 53 against 66.  Sixteen queries per workgroup
+// rather than 32 up to two blocks per CU (nb 512: 76 against 81 us; nb 1024: 226
+// against 226), one under a window (nb 256: 26.6 against 25.4; nb 512: 42 against
+// 39).  binary32 always takes the tile kernel: it replaced a form with one wave
+// per block and per SIMD (4 heads x 256, D 64: 36 -> 14 us; 16 heads x 2 x 4096,
+// D 128: 1781 -> 1531).
+static int fwd_tile_rows16(int nwq, long nb, int window) {
+  const long cus = otx_cu_count();
+  if (nwq != 4 || nb > (window > 0 ? 2 : 4) * cus) return 0;
+  return nb <= (window > 0 ? 1 : 2) * cus ? 1 : 2;
+}
+
+hipError_t launch_fwd_tile_i8(int D, int n16, const void* q, const void* k, void* o, float* lse, int B, int H, int Hkv,
+                              int S, int window, float sigma, int order, const int8_t* qvt, const float* vstep,
+                              float* scache, hipStream_t st);
+
 template <int D>
 static hipError_t launch_fwd_i8_d(int nwq, const void* q, const void* k, const void* v, void* o, float* lse, int B,
                                   int H, int Hkv, int S, int window, float sigma, int order, int8_t* qvt,
@@ -611,6 +637,8 @@ static hipError_t launch_fwd_i8_d(int nwq, const void* q, const void* k, const v
                      (const uint16_t*)v, qvt, vstep, nblk);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (const int n16 = fwd_tile_rows16(nwq, (long)(S / OTX_BLK) * B * H, window))
+    return launch_fwd_tile_i8(D, n16, q, k, o, lse, B, H, Hkv, S, window, sigma, order, qvt, vstep, scache, st);
   switch (nwq) {
     case 4: return launch_fwd_t<D, 4, true>(q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, st, qvt, vstep, scache);
     case 2: return launch_fwd_t<D, 2, true>(q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, st, qvt, vstep, scache);
@@ -643,32 +671,16 @@ hipError_t launch_fwd_tile(int dtype, int D, int n16, const void* q, const void*
                            hipStream_t st);
 
 // scache (bf16 only, may be null): also write the score cache.
-//
-// Kernel choice (every choice gives the same bits; CUs = 256, nb = the query
-// blocks of all heads).  binary32 always takes the tile kernel: it replaced a
-// form with one wave per block that needed 4 times as long on a small grid and
-// 1.2 times as long on the largest (4 heads x 256, D 64: 36 -> 14 us; 16 heads
-// x 2 x 4096, D 128: 1781 -> 1531 us).  bf16 takes it in the default launch up
-// to four blocks per CU under a full causal mask and two under a window, where
-// the one-wave-per-block kernel has at most one wave per SIMD and waits for the
-// longest rows: 16 heads x 1024, D 128 (nb 512): 166 -> 76 us; 16 x 2048 (nb
-// 1024): 322 -> 226; window 256 at nb 512: 67 -> 39; beyond it is no faster (nb
-// 2048: 228 against 220 and 119 against 126; nb 4096: 636 against 803; window
-// 256 at nb 1024, four query heads a group: 58 against 72).  Sixteen queries per
-// workgroup rather than 32 up to two blocks per CU (nb 512: 76 against 81 us; nb
-// 1024: 226 against 226), one under a window (nb 256: 26.6 against 25.4; nb 512:
-// 42 against 39).
 hipError_t launch_fwd(int dtype, int D, int nwq, const void* q, const void* k, const void* v, void* o, float* lse,
                       int B, int H, int Hkv, int S, int window, float sigma, int order, float* scache,
                       hipStream_t st) {
   const long nb = (long)(S / OTX_BLK) * B * H;
-  const long cus = otx_cu_count();
   const bool bf16 = dtype == 1;
   if (!bf16 && scache != nullptr) return hipErrorInvalidValue;  // the score cache is a bf16-path feature
-  if (!bf16 || (nwq == 4 && nb <= (window > 0 ? 2 : 4) * cus)) {
-    const int n16 = nwq == 4 ? (nb <= (window > 0 ? 1 : 2) * cus ? 1 : 2) : nwq;  // nwq 1, 2: the variant's own
+  int n16 = fwd_tile_rows16(nwq, nb, window);
+  if (!bf16 && n16 == 0) n16 = nwq == 1 ? 1 : 2;  // binary32 has no other form
+  if (n16)
     return launch_fwd_tile(dtype, D, n16, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, scache, st);
-  }
   if (D == 128) return launch_fwd_d<128>(nwq, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, scache, st);
   return launch_fwd_d<64>(nwq, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, scache, st);
 }

@@ -29,6 +29,7 @@
 namespace otx {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4 otx_mfma_k4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -108,11 +109,18 @@ __device__ __attribute__((noinline)) float otx_logf_tile_call(float x) { return 
 //        before the scores; B = the probabilities of all four waves, from LDS);
 //   the running sum l (a serial fold over the 64 keys) is kept in LDS and
 //   advanced by one wave per pair, the four waves in turn.
-template <typename T, int D, int NQ>
+// The fp32 matrix instructions and the vector unit take turns, so what is left
+// beside 32 cycles per product is vector work: K's transposes (one per product
+// pair), 4 NQ exps per lane, the sums.  4 heads x 256 x 64 in binary32: 36 -> 14
+// us; 16 heads x 1024 x 128 in bf16: 166 -> 76 us (its products alone: 14 us).
+// I8 (int8-PV): the probabilities also go to LDS as bytes with their block's step
+// and O^T += dequant(V^T P^T) takes one v_mfma_i32_16x16x32_i8 per 16 columns and
+// key block (integer sums, so the order of its keys does not matter): 134 -> 69 us.
+template <typename T, int D, int NQ, bool I8 = false>
 __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ o,
     float* __restrict__ lse, int B, int H, int Hkv, int S, int window, float sigma, int order,
-    float* __restrict__ scache) {
+    float* __restrict__ scache, const int8_t* __restrict__ qvt, const float* __restrict__ vstep) {
   constexpr int KS = D / 4;   // four-term steps of a score
   constexpr int NT = D / 64;  // 16-wide output tiles per wave
   constexpr int UPB = 2 / NQ; // workgroups per query block
@@ -120,6 +128,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
   __shared__ float4 Pb[NQ][4][64];
   __shared__ float Mx[4][16 * NQ];
   __shared__ float Ls[16 * NQ];
+  __shared__ uint2 Pq[I8 ? 2 : 1][NQ][16][4];  // int8 probabilities [key block][.][query][8 keys]
+  __shared__ float Sp[2][16 * NQ];             // and their steps
 
   const int nqt = S / OTX_BLK, units = nqt * UPB, BH = B * H;
   const int bid = blockIdx.x;
@@ -183,8 +193,22 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
   for (int ka = lo; ka <= qt; ka += 2, turn = (turn + 1) & 3) {
     const bool doB = ka + 1 <= qt;
     const bool wact = w < 2 || doB;
-    RN vraw[16];
-    {
+    RN vraw[I8 ? 1 : 16];
+    uint2 vq[2][NT];
+    float4 vst[2][NT];
+    if constexpr (I8) {  // d = w D/4 + 16 j + row; a block past the diagonal is not used
+#pragma unroll
+      for (int x = 0; x < 2; x++) {
+        const size_t blk = ((size_t)b * Hkv + gk) * nqt + (ka + x < qt ? ka + x : qt);
+        const uint2* qp = reinterpret_cast<const uint2*>(qvt + (blk * D + w * (D / 4) + c) * 32 + 8 * g);
+        const float4* sp = reinterpret_cast<const float4*>(vstep + blk * D + w * (D / 4) + 4 * g);
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+          vq[x][j] = qp[64 * j];
+          vst[x][j] = sp[4 * j];
+        }
+      }
+    } else {
       const T* p = vsrc + (size_t)ka * OTX_BLK * D;
 #pragma unroll
       for (int t = 0; t < 8; t++) vraw[t] = tile_load<T, NT>(p + (size_t)4 * t * D);
@@ -193,7 +217,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
         for (int t = 8; t < 16; t++) vraw[t] = tile_load<T, NT>(p + (size_t)4 * t * D);
       }
     }
-    float s[4 * NQ];
+    float s[(I8 ? 5 : 4) * NQ];  // with I8 the last NQ become the largest probability of this wave's block
     if (wact) {
       f32x4 sa[NQ];
 #pragma unroll
@@ -246,9 +270,11 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
       bool moved = false;
 #pragma unroll
       for (int n = 0; n < NQ; n++) {
-        ma[n] = otx_max_update(otx_max2p(Mx[0][16 * n + c], Mx[1][16 * n + c]), m[n]);
-        const float mb = otx_max2p(Mx[2][16 * n + c], Mx[3][16 * n + c]);
-        mbn[n] = doB ? otx_max_update(mb, ma[n]) : ma[n];
+        const float mba = otx_max2p(Mx[0][16 * n + c], Mx[1][16 * n + c]);
+        const float mbb = otx_max2p(Mx[2][16 * n + c], Mx[3][16 * n + c]);
+        ma[n] = otx_max_update(mba, m[n]);
+        mbn[n] = doB ? otx_max_update(mbb, ma[n]) : ma[n];
+        if constexpr (I8) s[4 * NQ + n] = w < 2 ? mba : mbb;
         al[2 * n] = ma[n] == m[n] ? 0.0f : m[n] - ma[n];
         al[2 * n + 1] = mbn[n] == ma[n] ? 0.0f : ma[n] - mbn[n];
         moved = moved || ma[n] != m[n] || mbn[n] != ma[n];
@@ -262,10 +288,30 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
         const float moff = mref != -__builtin_inff() ? mref : __builtin_inff();
 #pragma unroll
         for (int r = 0; r < 4; r++) s[4 * n + r] = s[4 * n + r] - moff;
+        if constexpr (I8) s[4 * NQ + n] = s[4 * NQ + n] - moff;
         m[n] = mbn[n];
       }
     }
-    otx_exp_n<4 * NQ, false, 4>(s, tab);
+    otx_exp_n<(I8 ? 5 : 4) * NQ, false, I8 ? 5 : 4>(s, tab);
+    if constexpr (I8) {
+      // The block's largest probability is the exp of its largest score: the difference and the correctly
+      // rounded exp are both monotone (a NaN score makes every probability of the row +0, as in the other form).
+      // Step and bytes as in attn_fwd_bf16_kernel, four keys per lane.
+#pragma unroll
+      for (int n = 0; n < NQ; n++) {
+        const float pmax = s[4 * NQ + n];
+        float inv = 0.0f, sp = 0.0f;
+        if (pmax > 0.0f) {
+          inv = otx_div_rn(127.0f, pmax);
+          sp = otx_div_by_recip(pmax, OTX_RECIP64_127);
+        }
+        uint32_t word = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) word = __builtin_amdgcn_cvt_pk_u8_f32(s[4 * n + e] * inv, e, word);
+        reinterpret_cast<uint32_t*>(&Pq[w >> 1][n][c][0])[4 * (w & 1) + g] = word & 0x7f7f7f7fu;
+        if (!(w & 1) && g == n) Sp[w >> 1][16 * n + c] = sp;
+      }
+    }
 #pragma unroll
     for (int n = 0; n < NQ; n++)
 #pragma unroll
@@ -301,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
             for (int r = 0; r < 4; r++) acc[n][j][r] = acc[n][j][r] * al[n];
       }
     };
-    auto fold = [&](int t4) {
+    auto fold = [&](int t4) {  // 16 keys
       float p[NQ][4];
 #pragma unroll
       for (int n = 0; n < NQ; n++) tile_get(Pb[n][t4][L], p[n]);
@@ -315,13 +361,38 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
           for (int n = 0; n < NQ; n++) acc[n][j] = otx_mfma_k4(x[j], p[n][e], acc[n][j]);
       }
     };
-    scale(al_a);
-    fold(0);
-    fold(1);
-    if (doB) {
-      scale(al_b);
-      fold(2);
-      fold(3);
+    if constexpr (I8) {
+      auto fold8 = [&](int x) {
+#pragma unroll
+        for (int n = 0; n < NQ; n++) {
+          const uint2 pb = Pq[x][n][c][g];
+          const float sp = Sp[x][16 * n + c];
+#pragma unroll
+          for (int j = 0; j < NT; j++) {
+            const i32x4 pv = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, vq[x][j]),
+                                                                   __builtin_bit_cast(long, pb), i32x4{}, 0, 0, 0);
+            float st[4];
+            tile_get(vst[x][j], st);
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[n][j][r] = __builtin_fmaf((float)pv[r] * st[r], sp, acc[n][j][r]);
+          }
+        }
+      };
+      scale(al_a);
+      fold8(0);
+      if (doB) {
+        scale(al_b);
+        fold8(1);
+      }
+    } else {
+      scale(al_a);
+      fold(0);
+      fold(1);
+      if (doB) {
+        scale(al_b);
+        fold(2);
+        fold(3);
+      }
     }
   }
 
@@ -331,22 +402,32 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
     const float l = Ls[16 * n + c];
     // RN(acc / l) through one binary64 reciprocal, as in attn_fwd_bf16_kernel
     const double rl = otx_recip64(l);
-    float x[4 * NT];
+    float x[4 * NT];  // output row r, tile j at X(r, j)
+    auto X = [](int r, int j) { return I8 ? 4 * j + r : NT * r + j; };
     bool low = false;
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
       for (int j = 0; j < NT; j++) {
-        x[NT * r + j] = otx_div_by_recip(acc[n][j][r], rl);
-        low = low || !(__builtin_fabsf(x[NT * r + j]) >= 0x1p-126f);
+        x[X(r, j)] = otx_div_by_recip(acc[n][j][r], rl);
+        low = low || !(__builtin_fabsf(x[X(r, j)]) >= 0x1p-126f);
       }
     if (__builtin_expect(__ballot(low) != 0, 0)) {
 #pragma unroll
       for (int r = 0; r < 4; r++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) x[NT * r + j] = otx_div_by_recip_checked(acc[n][j][r], rl, l);
+        for (int j = 0; j < NT; j++) x[X(r, j)] = otx_div_by_recip_checked(acc[n][j][r], rl, l);
     }
-    tile_store(o + ((size_t)bh * S + q0 + 16 * n + c) * D + w * (D / 4) + NT * 4 * g, x);
+    T* dst = o + ((size_t)bh * S + q0 + 16 * n + c) * D + w * (D / 4);
+    if constexpr (I8) {
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        const float y[4] = {x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]};
+        tile_store(dst + 16 * j + 4 * g, y);
+      }
+    } else {
+      tile_store(dst + NT * 4 * g, x);
+    }
     if (w == 0 && g == n) lse[(size_t)bh * S + q0 + 16 * n + c] = m[n] + otx_logf_tile_call(l);
   }
 }
@@ -363,7 +444,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
 //        from LDS across rows; B = P, dS).
 // Rows are D + 20 floats apart: the score reads (16 rows, four terms) then fall
 // into 64 different banks and the fold reads (four rows, 16 columns) share a
-// bank two at a time at most.
+// bank two at a time at most.  (D 128 with 64-query steps keeps D + 4, four at a
+// time: then two workgroups fit a CU's LDS; 16 heads x 2048, nkb 1024, 428 -> 361
+// us.)  8 heads, 2 KV heads x 1024 x 128, binary32: 1457 -> 222 us; 16 heads x 1024
+// x 128, bf16 with the score cache: 118 -> 95 us.
 template <typename T, int D, int NK, bool SC>
 __global__ __launch_bounds__(256, 2) void attn_dkdv_tile_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ dO,
@@ -572,7 +656,8 @@ __global__ __launch_bounds__(256, 2) void attn_dkdv_tile_kernel(
 
 // dQ.  A workgroup owns 16 NQ consecutive queries of one head, wave w the
 // columns d = w D/4 ..: no LDS and no barrier, K and the dS tiles come straight
-// from global memory one key block ahead.
+// from global memory one key block ahead.  Beside the products its time is those
+// loads (a K row per 32 queries and wave).  16 heads x 1024 x 128, bf16: 69 -> 30 us.
 template <typename T, int D, int NQ>
 __global__ __launch_bounds__(256, 2) void attn_dq_tile_kernel(const T* __restrict__ k,
                                                               const float* __restrict__ ws_ds, T* __restrict__ dq,
@@ -665,7 +750,22 @@ static hipError_t launch_fwd_tile_d(int nq, const void* q, const void* k, const 
   const unsigned grid = (unsigned)((long)(S / OTX_BLK) * (2 / nq) * B * H);
 #define OTX_FWD_TILE(NQ)                                                                                        \
   hipLaunchKernelGGL((attn_fwd_tile_kernel<T, D, NQ>), dim3(grid), dim3(256), 0, st, (const T*)q, (const T*)k, \
-                     (const T*)v, (T*)o, lse, B, H, Hkv, S, window, sigma, order, scache)
+                     (const T*)v, (T*)o, lse, B, H, Hkv, S, window, sigma, order, scache, nullptr, nullptr)
+  if (nq == 1) OTX_FWD_TILE(1); else OTX_FWD_TILE(2);
+#undef OTX_FWD_TILE
+  return hipGetLastError();
+}
+
+// int8-PV on the quantized V of attn_quant_v_kernel (qvt, vstep).
+template <int D>
+static hipError_t launch_fwd_tile_i8_d(int nq, const void* q, const void* k, void* o, float* lse, int B, int H, int Hkv,
+                                       int S, int window, float sigma, int order, const int8_t* qvt,
+                                       const float* vstep, float* scache, hipStream_t st) {
+  const unsigned grid = (unsigned)((long)(S / OTX_BLK) * (2 / nq) * B * H);
+#define OTX_FWD_TILE(NQ)                                                                                    \
+  hipLaunchKernelGGL((attn_fwd_tile_kernel<uint16_t, D, NQ, true>), dim3(grid), dim3(256), 0, st,           \
+                     (const uint16_t*)q, (const uint16_t*)k, nullptr, (uint16_t*)o, lse, B, H, Hkv, S, window, \
+                     sigma, order, scache, qvt, vstep)
   if (nq == 1) OTX_FWD_TILE(1); else OTX_FWD_TILE(2);
 #undef OTX_FWD_TILE
   return hipGetLastError();
@@ -714,6 +814,13 @@ hipError_t launch_fwd_tile(int dtype, int D, int n16, const void* q, const void*
                            int B, int H, int Hkv, int S, int window, float sigma, int order, float* scache,
                            hipStream_t st) {
   return OTX_TILE_DISPATCH(launch_fwd_tile_d, n16, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, scache, st);
+}
+hipError_t launch_fwd_tile_i8(int D, int n16, const void* q, const void* k, void* o, float* lse, int B, int H, int Hkv,
+                              int S, int window, float sigma, int order, const int8_t* qvt, const float* vstep,
+                              float* scache, hipStream_t st) {
+  if (D == 128)
+    return launch_fwd_tile_i8_d<128>(n16, q, k, o, lse, B, H, Hkv, S, window, sigma, order, qvt, vstep, scache, st);
+  return launch_fwd_tile_i8_d<64>(n16, q, k, o, lse, B, H, Hkv, S, window, sigma, order, qvt, vstep, scache, st);
 }
 hipError_t launch_dkdv_tile(int dtype, int D, int n16, const void* q, const void* k, const void* v, const void* dO,
                             const float* lse, const float* dsum, void* dk, void* dv, float* ds, int B, int H, int Hkv,

@@ -67,3 +67,18 @@ def test_gpu_tile_choice(shape, dtype):
         for a, b, n in zip(ref, fa.flash_attention_backward(q, k, v, o, lse, do, window, score_cache=sc[1][2]),
                            NAMES[2:]):
             assert torch.equal(a, b), (n, "cache")
+
+
+@pytest.mark.parametrize("shape", LIMITS, ids=[f"l{i}" for i in range(len(LIMITS))])
+def test_gpu_tile_choice_int8pv(shape):
+    """The int8-PV forward with its score cache, variants 0, 1 and 2.  Some rows have scores so far apart that a
+    block's probabilities are all +0 or below the step's normal range."""
+    B, H, Hkv, S, D, window = shape
+    print(shape, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    q, k, v = (torch.randn(B, h, S, D, device="cuda", generator=g).to(torch.bfloat16) for h in (H, Hkv, Hkv))
+    q[:, :, 5::7] *= 12.0
+    ref = fa.int8pv_flash_attention_forward_sc(q, k, v, window, variant=2)
+    for variant in (0, 1):
+        for a, b in zip(ref, fa.int8pv_flash_attention_forward_sc(q, k, v, window, variant=variant)):
+            assert torch.equal(a, b), variant
