@@ -31,90 +31,36 @@
 
 namespace otx {
 
-// Partials of fold32 over one row, term(d, acc) = fma(f_d..., acc): chunk c is
-// computed by lane c % 64 into slot c / 64.
-template <int SLOTS, typename F>
-__device__ __forceinline__ void row_partials(int D, F&& term, float (&part)[SLOTS]) {
-  const int L = threadIdx.x & 63;
+// 16 bytes of a T tensor: 8 bf16 or 4 binary32 elements.
+template <typename T>
+struct Act16 {
+  static constexpr int N = 16 / sizeof(T);
+  __device__ __forceinline__ static void load(const T* p, float (&v)[N]) {
+    const uint4 w = *(const uint4*)p;
 #pragma unroll
-  for (int s = 0; s < SLOTS; s++) {
-    const int cidx = s * 64 + L;
-    float p = 0.0f;
-    if (cidx * 32 < D) {
-#pragma unroll 8
-      for (int i = 0; i < 32; i++) p = term(cidx * 32 + i, p);
+    for (int e = 0; e < N; e++) v[e] = Elem<T>::get(w, e);
+  }
+  __device__ __forceinline__ static void store(T* p, const float (&v)[N]) {
+    uint4 w;
+    uint32_t* wp = (uint32_t*)&w;
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        wp[k] = (uint32_t)Elem<T>::put(v[2 * k]) | ((uint32_t)Elem<T>::put(v[2 * k + 1]) << 16);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) wp[k] = __float_as_uint(v[k]);
     }
-    part[s] = p;
+    *(uint4*)p = w;
   }
-}
-
-// Ascending fold of the partials (chunk c in lane c % 64, slot c / 64); every
-// lane ends with the same value.
-template <int SLOTS>
-__device__ __forceinline__ float fold_all(const float (&part)[SLOTS], int nch) {
-  float acc = 0.0f;
-#pragma unroll
-  for (int s = 0; s < SLOTS; s++) {
-    const int n = nch - 64 * s < 64 ? nch - 64 * s : 64;
-    for (int l = 0; l < n; ++l) acc = acc + __shfl(part[s], l);
+  __device__ __forceinline__ static float round(float v) {
+    if constexpr (sizeof(T) == 2)
+      return otx_bf16_to_f32(otx_f32_to_bf16(v));
+    else
+      return v;
   }
-  return acc;
-}
+};
 
-template <typename T, int SLOTS>
-__global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                          T* __restrict__ y, float* __restrict__ rstd_out, long rows,
-                                                          int D, float eps) {
-  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int L = threadIdx.x & 63;
-  const T* xr = x + row * D;
-  float part[SLOTS];
-  row_partials<SLOTS>(D, [&](int d, float acc) {
-    const float v = Elem<T>::ld(xr + d);
-    return __builtin_fmaf(v, v, acc);
-  }, part);
-  const float ss = fold_all<SLOTS>(part, D / 32);
-  const float mean = otx_div_rn(ss, (float)D);
-  const float rstd = otx_rsqrtf(mean + eps);
-  T* yr = y + row * D;
-  for (int d = L; d < D; d += 64) {
-    const float xh = Elem<T>::ld(xr + d) * rstd;
-    yr[d] = Elem<T>::put(xh * Elem<T>::ld(w + d));
-  }
-  if (L == 0) rstd_out[row] = rstd;
-}
-
-template <typename T, int SLOTS>
-__global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                          const float* __restrict__ rstd_in,
-                                                          const T* __restrict__ dy, T* __restrict__ dx, long rows,
-                                                          int D) {
-  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int L = threadIdx.x & 63;
-  const T* xr = x + row * D;
-  const T* dyr = dy + row * D;
-  const float rstd = rstd_in[row];
-  float part[SLOTS];
-  row_partials<SLOTS>(D, [&](int d, float acc) {
-    const float xh = Elem<T>::ld(xr + d) * rstd;
-    const float g = Elem<T>::ld(dyr + d) * Elem<T>::ld(w + d);
-    return __builtin_fmaf(g, xh, acc);
-  }, part);
-  const float cc = otx_div_rn(fold_all<SLOTS>(part, D / 32), (float)D);
-  T* dxr = dx + row * D;
-  for (int d = L; d < D; d += 64) {
-    const float xh = Elem<T>::ld(xr + d) * rstd;
-    const float g = Elem<T>::ld(dyr + d) * Elem<T>::ld(w + d);
-    dxr[d] = Elem<T>::put(rstd * (g - xh * cc));
-  }
-}
-
-// Row-group form for D = 32 G with G a power of two up to 64: lane L of a wave
-// owns chunk c = L % G of row L / G (64 / G rows per wave) and reads its 32
-// elements with 16-byte loads; the partials are folded in order with G
-// shuffles inside the row's lane group.  Same arithmetic as the kernels above.
 template <typename T>
 struct Chunk32 {
   static constexpr int NV = 32 * (int)sizeof(T) / 16;  // 16-byte vectors per chunk
@@ -144,6 +90,144 @@ struct Chunk32 {
   }
 };
 
+// Partials of fold32 over one row, v(c, e) the 32 terms' factors of chunk c: chunk c
+// is computed by lane c % 64 into slot c / 64, +0 past the last chunk.
+template <int SLOTS, typename F>
+__device__ __forceinline__ void row_partials(int D, F&& chunk, float (&part)[SLOTS]) {
+  const int L = threadIdx.x & 63;
+#pragma unroll
+  for (int s = 0; s < SLOTS; s++) {
+    const int cidx = s * 64 + L;
+    part[s] = cidx * 32 < D ? chunk(cidx) : 0.0f;
+  }
+}
+
+// Ascending fold of the partials (chunk c in lane c % 64, slot c / 64); every
+// lane ends with the same value.  Called by whole waves.  Lanes are read sixteen at a
+// time, past the last chunk too: a partial there is +0, and the fold, begun at +0, is
+// never -0, so adding it changes nothing.
+template <int SLOTS>
+__device__ __forceinline__ float fold_all(const float (&part)[SLOTS], int nch) {
+  float acc = 0.0f;
+#pragma unroll
+  for (int s = 0; s < SLOTS; s++) {
+    const int n = nch - 64 * s < 64 ? nch - 64 * s : 64;
+    for (int l = 0; l < n; l += 16) {
+#pragma unroll
+      for (int u = 0; u < 16; u++)
+        acc = acc + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(part[s]), l + u));
+    }
+  }
+  return acc;
+}
+
+// Elements p[0 .. 31], 16 bytes at a time where VEC says that p is aligned.
+template <typename T, bool VEC>
+__device__ __forceinline__ void load_chunk(const T* p, float (&v)[32]) {
+  if constexpr (VEC) {
+    Chunk32<T>::load(p, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 32; i++) v[i] = Elem<T>::ld(p + i);
+  }
+}
+
+// One wave per row, any D = 32 n up to 64 * SLOTS chunks: the widths without a row-group
+// form (VEC), and rows that are not 16-byte aligned.  Bound by the loads: a lane reads
+// its chunk, and then the row again from the cache, 16 bytes at a time.  Measured at
+// 8192 x 3008 bf16: forward 37.9 -> 22.0 us (4.5 TB/s), dx 45.5 -> 35.4 (a lane's chunk and
+// the second pass were read 2 bytes at a time).
+template <typename T, int SLOTS, bool VEC>
+__global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ w,
+                                                          T* __restrict__ y, float* __restrict__ rstd_out, long rows,
+                                                          int D, float eps) {
+  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int L = threadIdx.x & 63;
+  const T* xr = x + row * D;
+  float part[SLOTS];
+  row_partials<SLOTS>(D, [&](int c) {
+    float v[32], p = 0.0f;
+    load_chunk<T, VEC>(xr + 32 * c, v);
+#pragma unroll
+    for (int i = 0; i < 32; i++) p = __builtin_fmaf(v[i], v[i], p);
+    return p;
+  }, part);
+  const float ss = fold_all<SLOTS>(part, D / 32);
+  const float mean = otx_div_rn(ss, (float)D);
+  const float rstd = otx_rsqrtf(mean + eps);
+  T* yr = y + row * D;
+  if constexpr (VEC) {
+    constexpr int N = Act16<T>::N;
+    for (int d = L * N; d < D; d += 64 * N) {
+      float v[N], wv[N];
+      Act16<T>::load(xr + d, v);
+      Act16<T>::load(w + d, wv);
+#pragma unroll
+      for (int e = 0; e < N; e++) v[e] = (v[e] * rstd) * wv[e];
+      Act16<T>::store(yr + d, v);
+    }
+  } else {
+    for (int d = L; d < D; d += 64) {
+      const float xh = Elem<T>::ld(xr + d) * rstd;
+      yr[d] = Elem<T>::put(xh * Elem<T>::ld(w + d));
+    }
+  }
+  if (L == 0) rstd_out[row] = rstd;
+}
+
+template <typename T, int SLOTS, bool VEC>
+__global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ x, const T* __restrict__ w,
+                                                          const float* __restrict__ rstd_in,
+                                                          const T* __restrict__ dy, T* __restrict__ dx, long rows,
+                                                          int D) {
+  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int L = threadIdx.x & 63;
+  const T* xr = x + row * D;
+  const T* dyr = dy + row * D;
+  const float rstd = rstd_in[row];
+  float part[SLOTS];
+  row_partials<SLOTS>(D, [&](int c) {
+    float xv[32], gv[32], wv[32], p = 0.0f;
+    load_chunk<T, VEC>(xr + 32 * c, xv);
+    load_chunk<T, VEC>(dyr + 32 * c, gv);
+    load_chunk<T, VEC>(w + 32 * c, wv);
+#pragma unroll
+    for (int i = 0; i < 32; i++) p = __builtin_fmaf(gv[i] * wv[i], xv[i] * rstd, p);
+    return p;
+  }, part);
+  const float cc = otx_div_rn(fold_all<SLOTS>(part, D / 32), (float)D);
+  T* dxr = dx + row * D;
+  if constexpr (VEC) {
+    constexpr int N = Act16<T>::N;
+    for (int d = L * N; d < D; d += 64 * N) {
+      float xv[N], gv[N], wv[N];
+      Act16<T>::load(xr + d, xv);
+      Act16<T>::load(dyr + d, gv);
+      Act16<T>::load(w + d, wv);
+#pragma unroll
+      for (int e = 0; e < N; e++) gv[e] = rstd * (gv[e] * wv[e] - (xv[e] * rstd) * cc);
+      Act16<T>::store(dxr + d, gv);
+    }
+  } else {
+    for (int d = L; d < D; d += 64) {
+      const float xh = Elem<T>::ld(xr + d) * rstd;
+      const float g = Elem<T>::ld(dyr + d) * Elem<T>::ld(w + d);
+      dxr[d] = Elem<T>::put(rstd * (g - xh * cc));
+    }
+  }
+}
+
+// Row-group form for D = 32 G with G a power of two up to 64: lane L of a wave
+// owns chunk c = L % G of row L / G (64 / G rows per wave) and reads its 32
+// elements with 16-byte loads; the partials are folded in order with G
+// shuffles inside the row's lane group.  Same arithmetic as the kernels above.
+// Bound by HBM.  The forward's second pass walks the wave's 2048 elements side by side
+// and reads x again from the cache: stores of a lane's own chunk left 64 bytes between
+// lanes.  Measured, bf16: 8192 x 2048 19.4 -> 14.7 us (4.6 TB/s), 131072 x 128 18.4 ->
+// 13.9.  The backward keeps its chunk (two tensors to read again: 21.8 us kept, 23.0
+// re-read at 8192 x 2048).
 // Ascending fold of the G partials of this lane's row group (every lane of the
 // group ends with the same value).
 template <int G>
@@ -159,27 +243,33 @@ template <typename T, int G>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_rows_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                                T* __restrict__ y, float* __restrict__ rstd_out,
                                                                long rows, float eps) {
-  constexpr int D = 32 * G, RPW = 64 / G;
+  constexpr int D = 32 * G, RPW = 64 / G, N = Act16<T>::N;
   const int L = threadIdx.x & 63, c = L % G;
-  const long row = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + L / G;
+  const long row0 = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW, row = row0 + L / G;
   const bool live = row < rows;
-  float v[32];
-  if (live) Chunk32<T>::load(x + row * D + 32 * c, v);
-  else
-#pragma unroll
-    for (int i = 0; i < 32; i++) v[i] = 0.0f;
   float p = 0.0f;
+  if (live) {
+    float v[32];
+    Chunk32<T>::load(x + row * D + 32 * c, v);
 #pragma unroll
-  for (int i = 0; i < 32; i++) p = __builtin_fmaf(v[i], v[i], p);
+    for (int i = 0; i < 32; i++) p = __builtin_fmaf(v[i], v[i], p);
+  }
   const float ss = fold_group<G>(p);
   const float rstd = otx_rsqrtf(otx_div_rn(ss, (float)D) + eps);
-  if (!live) return;
-  float wv[32];
-  Chunk32<T>::load(w + 32 * c, wv);
 #pragma unroll
-  for (int i = 0; i < 32; i++) v[i] = (v[i] * rstd) * wv[i];
-  Chunk32<T>::store(y + row * D + 32 * c, v);
-  if (c == 0) rstd_out[row] = rstd;
+  for (int k = 0; k < 32 / N; k++) {
+    const int i = (k * 64 + L) * N, r = i / D, d = i % D;  // element i of the wave's 2048
+    const float rs = __shfl(rstd, r * G);
+    if (row0 + r < rows) {
+      float v[N], wv[N];
+      Act16<T>::load(x + row0 * D + i, v);
+      Act16<T>::load(w + d, wv);
+#pragma unroll
+      for (int e = 0; e < N; e++) v[e] = (v[e] * rs) * wv[e];
+      Act16<T>::store(y + row0 * D + i, v);
+    }
+  }
+  if (live && c == 0) rstd_out[row] = rstd;
 }
 
 template <typename T, int G>
@@ -311,36 +401,6 @@ __device__ __forceinline__ void silu_terms(const float (&x)[N], float (&y)[N], f
     }
   }
 }
-
-// 16 bytes of a T tensor: 8 bf16 or 4 binary32 elements.
-template <typename T>
-struct Act16 {
-  static constexpr int N = 16 / sizeof(T);
-  __device__ __forceinline__ static void load(const T* p, float (&v)[N]) {
-    const uint4 w = *(const uint4*)p;
-#pragma unroll
-    for (int e = 0; e < N; e++) v[e] = Elem<T>::get(w, e);
-  }
-  __device__ __forceinline__ static void store(T* p, const float (&v)[N]) {
-    uint4 w;
-    uint32_t* wp = (uint32_t*)&w;
-    if constexpr (sizeof(T) == 2) {
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-        wp[k] = (uint32_t)Elem<T>::put(v[2 * k]) | ((uint32_t)Elem<T>::put(v[2 * k + 1]) << 16);
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; k++) wp[k] = __float_as_uint(v[k]);
-    }
-    *(uint4*)p = w;
-  }
-  __device__ __forceinline__ static float round(float v) {
-    if constexpr (sizeof(T) == 2)
-      return otx_bf16_to_f32(otx_f32_to_bf16(v));
-    else
-      return v;
-  }
-};
 
 // The activation kernels are bound by HBM once the exp and the quotients are
 // short (about 30 vector instructions per element forward): a workgroup loads
@@ -495,17 +555,46 @@ static bool launch_rows_bwd_any(int G, const void* x, const void* w, const float
   }
 }
 
+static bool all_aligned16(std::initializer_list<const void*> ptrs) {
+  for (const void* p : ptrs)
+    if (!aligned16p(p)) return false;
+  return true;
+}
+
+// One slot of chunks per lane up to 2048 columns, four up to the largest width; 16-byte
+// accesses where the base pointers are aligned (rows are: D is a multiple of 32).
+template <typename T, bool VEC>
+static void launch_wave_fwd(const void* x, const void* w, void* y, float* rstd, long rows, int D, float eps,
+                            hipStream_t st) {
+  const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+  if (D <= 2048)
+    hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, 1, VEC>), grid, block, 0, st, (const T*)x, (const T*)w, (T*)y, rstd,
+                       rows, D, eps);
+  else
+    hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, 4, VEC>), grid, block, 0, st, (const T*)x, (const T*)w, (T*)y, rstd,
+                       rows, D, eps);
+}
+
+template <typename T, bool VEC>
+static void launch_wave_bwd(const void* x, const void* w, const float* rstd, const void* dy, void* dx, long rows,
+                            int D, hipStream_t st) {
+  const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+  if (D <= 2048)
+    hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, 1, VEC>), grid, block, 0, st, (const T*)x, (const T*)w, rstd,
+                       (const T*)dy, (T*)dx, rows, D);
+  else
+    hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, 4, VEC>), grid, block, 0, st, (const T*)x, (const T*)w, rstd,
+                       (const T*)dy, (T*)dx, rows, D);
+}
+
 template <typename T>
 static hipError_t launch_rmsnorm_fwd_t(const void* x, const void* w, void* y, float* rstd, long rows, int D,
                                        float eps, hipStream_t st) {
   if (launch_rows_fwd_any<T>(row_group(D, {x, w, y}), x, w, y, rstd, rows, eps, st)) return hipGetLastError();
-  const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-  if (D <= 2048)
-    hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, 1>), grid, block, 0, st, (const T*)x, (const T*)w, (T*)y, rstd, rows,
-                       D, eps);
+  if (all_aligned16({x, w, y}))
+    launch_wave_fwd<T, true>(x, w, y, rstd, rows, D, eps, st);
   else
-    hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, 4>), grid, block, 0, st, (const T*)x, (const T*)w, (T*)y, rstd, rows,
-                       D, eps);
+    launch_wave_fwd<T, false>(x, w, y, rstd, rows, D, eps, st);
   return hipGetLastError();
 }
 
@@ -518,14 +607,11 @@ hipError_t launch_rmsnorm_fwd(int dtype, const void* x, const void* w, void* y, 
 template <typename T>
 static hipError_t launch_rmsnorm_bwd_t(const void* x, const void* w, const float* rstd, const void* dy, void* dx,
                                        float* dw, float* part, long rows, int D, hipStream_t st) {
-  const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
   if (!launch_rows_bwd_any<T>(row_group(D, {x, w, dy, dx}), x, w, rstd, dy, dx, rows, st)) {
-    if (D <= 2048)
-      hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, 1>), grid, block, 0, st, (const T*)x, (const T*)w, rstd,
-                         (const T*)dy, (T*)dx, rows, D);
+    if (all_aligned16({x, w, dy, dx}))
+      launch_wave_bwd<T, true>(x, w, rstd, dy, dx, rows, D, st);
     else
-      hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, 4>), grid, block, 0, st, (const T*)x, (const T*)w, rstd,
-                         (const T*)dy, (T*)dx, rows, D);
+      launch_wave_bwd<T, false>(x, w, rstd, dy, dx, rows, D, st);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

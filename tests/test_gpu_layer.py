@@ -145,6 +145,17 @@ def test_rmsnorm_widths_and_layouts(rows, D, bf16, offset):
     assert_bits_equal(host(gw.grad), rnd(rdw), "dw (weight dtype)")
 
 
+@pytest.mark.parametrize("rows,D,bf16,offset", [
+    (32, 8192, True, 0), (32, 8160, False, 0), (64, 2080, False, 0),  # four chunks a lane, the last slot part full
+    (64, 4128, True, 1), (64, 2016, False, 1),                        # the same kernels on unaligned rows
+    (32, 544, True, 0), (32, 96, False, 0),                           # a part of one slot
+    (32, 32, True, 0), (96, 64, False, 0), (32, 2048, False, 0),      # row groups: a wave past the last row
+])
+def test_rmsnorm_wide_loads(rows, D, bf16, offset):
+    """The 16-byte forms of the other widths and the row groups' side-by-side second pass, exactly."""
+    test_rmsnorm_widths_and_layouts(rows, D, bf16, offset)
+
+
 def test_silu_fwd_bwd():
     rng = np.random.default_rng(9)
     x = bf(np.concatenate([rng.standard_normal(50000) * 4, np.linspace(-120, 120, 4097),
