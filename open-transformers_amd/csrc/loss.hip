@@ -108,9 +108,10 @@ __device__ __forceinline__ void ce_store_stats(const T* row, long n, long N, int
   stats[4 * N + n] = lse * lse;
 }
 
-// v[j] = exp(v[j]) for v[j] = RN(x - m) <= 0, -inf or NaN (x or m not finite), by the
-// softmax path, with NaN put back where it was.
-template <int N, int NB = 8>
+// v[j] = exp(v[j]) for v[j] = RN(x - m), with NaN (x or m not finite) put back where it
+// was: the softmax path for m the row's maximum (v[j] <= 0), or, with ANY, the one for
+// either sign (the backward's m is the caller's, and a logit may lie above it).
+template <int N, int NB = 8, bool ANY = false>
 __device__ __forceinline__ void ce_exp_n(float (&v)[N], const double* tab) {
   float mx = v[0];
 #pragma unroll
@@ -121,7 +122,10 @@ __device__ __forceinline__ void ce_exp_n(float (&v)[N], const double* tab) {
 #pragma unroll
     for (int j = 0; j < N; j++) nan |= v[j] != v[j] ? 1u << j : 0u;
   }
-  otx_exp_n<N, false, NB>(v, tab);
+  if constexpr (ANY)
+    otx_exp_any_n<N, NB>(v, tab);
+  else
+    otx_exp_n<N, false, NB>(v, tab);
   if (__builtin_expect(__ballot(nan != 0) != 0, 0)) {
 #pragma unroll
     for (int j = 0; j < N; j++) v[j] = nan >> j & 1 ? __builtin_nanf("") : v[j];
@@ -530,7 +534,7 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(const T* __restrict__ logit
       }
 #pragma unroll
       for (int i = 0; i < 8; i++) e[i] = e[i] - row.m;
-      ce_exp_n<8>(e, tab);
+      ce_exp_n<8, 8, true>(e, tab);
       float g[8];
       ce_grad<8>(e, row, has_coeff, g);
 #pragma unroll
@@ -575,11 +579,8 @@ __global__ __launch_bounds__(256) void ce_bwd_table_kernel(const uint16_t* __res
   for (int i0 = t; i0 < CE_TAB_N; i0 += 8 * 256) {
     float e[8], g[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float x = ce_tab_x(i0 + 256 * j);
-      e[j] = x <= row.m ? x - row.m : -__builtin_inff();
-    }
-    otx_exp_n<8>(e, tab);
+    for (int j = 0; j < 8; j++) e[j] = ce_tab_x(i0 + 256 * j) - row.m;
+    ce_exp_n<8, 8, true>(e, tab);
     ce_grad<8>(e, row, has_coeff, g);
 #pragma unroll
     for (int j = 0; j < 8; j++)
@@ -616,7 +617,7 @@ __global__ __launch_bounds__(256) void ce_bwd_table_kernel(const uint16_t* __res
       float e[8], g[8];
 #pragma unroll
       for (int j = 0; j < 8; j++) e[j] = Elem<uint16_t>::get(u, j) - row.m;
-      ce_exp_n<8, 4>(e, tab);
+      ce_exp_n<8, 4, true>(e, tab);
       ce_grad<8>(e, row, has_coeff, g);
 #pragma unroll
       for (int j = 0; j < 8; j++)

@@ -160,20 +160,25 @@ __device__ __forceinline__ void otx_exp_n(float (&v)[N], const double* tab) {
 }
 
 // v[j] = exp(v[j]) correctly rounded, in place, for arguments of either sign
-// (NaN is not carried through: see otx_exp_any_t), stage by stage like otx_exp_n.
-template <int N>
+// (NaN is not carried through: see otx_exp_any_t), stage by stage like otx_exp_n,
+// NB values at a time.
+template <int N, int NB = N>
 __device__ __forceinline__ void otx_exp_any_n(float (&v)[N], const double* tab) {
-  double xd[N], d[N], tv[N];
-  uint32_t kb[N];
+  static_assert(N % NB == 0, "chunk size must divide the array");
 #pragma unroll
-  for (int j = 0; j < N; j++) d[j] = otx_exp_any_t(v[j], &xd[j]);
+  for (int c = 0; c < N; c += NB) {
+    double xd[NB], d[NB], tv[NB];
+    uint32_t kb[NB];
 #pragma unroll
-  for (int j = 0; j < N; j++) {
-    kb[j] = (uint32_t)otx_d2u(d[j]);
-    tv[j] = *reinterpret_cast<const double*>(reinterpret_cast<const unsigned char*>(tab) + otx_tab_off(kb[j]));
+    for (int j = 0; j < NB; j++) d[j] = otx_exp_any_t(v[c + j], &xd[j]);
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      kb[j] = (uint32_t)otx_d2u(d[j]);
+      tv[j] = *reinterpret_cast<const double*>(reinterpret_cast<const unsigned char*>(tab) + otx_tab_off(kb[j]));
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++) v[c + j] = otx_exp_le0_y(otx_exp_le0_p(otx_exp_le0_r(d[j], xd[j])), tv[j], kb[j]);
   }
-#pragma unroll
-  for (int j = 0; j < N; j++) v[j] = otx_exp_le0_y(otx_exp_le0_p(otx_exp_le0_r(d[j], xd[j])), tv[j], kb[j]);
 }
 
 // 1/d to about one unit of binary64 for d >= 1 (NaN for d = inf): the hardware

@@ -172,3 +172,30 @@ def test_loss_forms_and_edge_rows(N, V, dtype):
     eq(st.cpu().numpy(), st_r, "row statistics")
     eq(np.array([ce.item(), z.item()], np.float32), np.array([ce_r, z_r], np.float32), "ce, z")
     eq(g.float().cpu().numpy(), g_r, "logit gradient")
+
+
+@pytest.mark.parametrize("N,V,dtype", [
+    (24, 16384, "bf16"),  # the table form
+    (24, 4096, "bf16"),   # the general form, 16-byte vectors
+    (24, 4099, "f32"),    # element by element
+])
+def test_backward_from_a_maximum_below_the_logits(N, V, dtype):
+    """ce_zloss_backward takes the caller's statistics: with a stored maximum below some logits (or above all of them,
+    infinite or NaN) exp(x - m) is still the correctly rounded one, in every form of the kernel."""
+    from attn_util import assert_bits_equal_nan_class as eq
+
+    print(f"loss backward, maximum below the logits N={N} V={V} {dtype}", flush=True)
+    x, lab = _inputs(N, V, dtype, seed=N + V, scale=2.0)
+    x = _edge_rows(x, np.random.default_rng(V))
+    if dtype == "bf16":
+        x = synthetic.round_to_bf16(x)
+    with np.errstate(all="ignore"):
+        st = orc.ce_zloss_fwd(x, lab, 1e-4)[2]
+        st[0] -= np.resize(np.array([0.5, 3.0, 60.0, 100.0, -2.0], np.float32), N)
+        st[0, 13], st[0, 14], st[0, 15] = np.nan, np.inf, -np.inf
+        g_r = orc.ce_zloss_bwd(x, lab, st, 1e-4, gce=2.0, gz=3.0, out_bf16=dtype == "bf16")
+    assert np.isinf(g_r).any() and (st[0] < x.max(1)).any()
+    two, three = torch.tensor(2.0, device=DEV), torch.tensor(3.0, device=DEV)
+    g = L.ce_zloss_backward(_gpu(x, dtype), torch.from_numpy(lab).to(DEV), torch.from_numpy(st).to(DEV), two, three, 1e-4)
+    torch.cuda.synchronize()
+    eq(g.float().cpu().numpy(), g_r, "logit gradient")
