@@ -91,6 +91,7 @@ struct Linear : Function<Linear> {
 struct RMSNorm : Function<RMSNorm> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
     const int64_t D = x.size(-1);
+    TORCH_CHECK_VALUE(D > 0, "rms_norm: empty last dimension");
     const Tensor xc = x.contiguous(), wc = w.to(x.scalar_type()).contiguous();
     const int64_t rows = xc.numel() / D;
     const Tensor y = at::empty_like(xc), rstd = at::empty({rows}, x.options().dtype(at::kFloat));
@@ -142,6 +143,7 @@ struct SiLU : Function<SiLU> {
 struct SwiGLU : Function<SwiGLU> {
   static Tensor forward(AutogradContext* ctx, const Tensor& gu) {
     const int64_t F = gu.size(-1) / 2;
+    TORCH_CHECK_VALUE(F > 0, "swiglu: empty last dimension");
     const Tensor guc = gu.contiguous();
     std::vector<int64_t> shape = gu.sizes().vec();
     shape.back() = F;
