@@ -1,8 +1,8 @@
 // The operators' autograd nodes, over the C ABI of include/otx_attn.h.
 //
-// Each node is one of the operators of nn/ (which check their arguments first):
-// it allocates outputs and workspaces, launches on the current stream and saves what
-// its backward reads.  Native because a pass over small tensors is bound by the host: a
+// Each node is one of the operators of nn/ (which check device and dtype first; sizes that
+// the C ABI cannot see are checked here): it allocates outputs and workspaces, launches on
+// the current stream and saves what its backward reads.  Native because a pass over small tensors is bound by the host: a
 // Python node's backward runs on the engine's device thread, where the interpreter and
 // the foreign-function calls cost several times what the launches do.  Measured on one
 // host (issue time of one forward and backward, Python nodes against these): linear 113
@@ -31,6 +31,11 @@ int dtype_code(const Tensor& t) {
   TORCH_CHECK_VALUE(t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat, "dtype ", t.scalar_type(),
                     " not supported (bfloat16 or float32)");
   return t.scalar_type() == at::kBFloat16 ? OTX_DTYPE_BF16 : OTX_DTYPE_F32;
+}
+
+void check_device(const Tensor& t, const Tensor& like, const char* what) {
+  TORCH_CHECK(t.device() == like.device(), what, " is on ", t.device(), ", the input on ", like.device(),
+              ": Expected all tensors to be on the same device");
 }
 
 // The stream that work on t's device is queued on, with that device made current.
@@ -66,6 +71,8 @@ Tensor gemm(const Tensor& a, long a_i, long a_r, const Tensor& b, long b_j, long
 struct Linear : Function<Linear> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
     const int64_t K = x.size(-1), N = w.size(0);
+    check_device(w, x, "linear: the weight");
+    TORCH_CHECK_VALUE(w.numel() == N * K, "linear: weight ", w.sizes(), " for an input of width ", K);
     const Tensor x2 = x.reshape({-1, K}).contiguous(), wc = w.contiguous();
     const Tensor y = gemm(x2, K, 1, wc, K, 1, x2.size(0), N, K);  // y = x w^T
     ctx->save_for_backward({x2, wc});
@@ -91,7 +98,9 @@ struct Linear : Function<Linear> {
 struct RMSNorm : Function<RMSNorm> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
     const int64_t D = x.size(-1);
+    check_device(w, x, "rms_norm: the weight");
     TORCH_CHECK_VALUE(D > 0, "rms_norm: empty last dimension");
+    TORCH_CHECK_VALUE(w.numel() == D, "rms_norm: weight ", w.sizes(), " for an input of width ", D);
     const Tensor xc = x.contiguous(), wc = w.to(x.scalar_type()).contiguous();
     const int64_t rows = xc.numel() / D;
     const Tensor y = at::empty_like(xc), rstd = at::empty({rows}, x.options().dtype(at::kFloat));
@@ -168,6 +177,8 @@ struct SwiGLU : Function<SwiGLU> {
 struct RopeHeads : Function<RopeHeads> {  // [B, T, H, D] -> [B, H, T, D]
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& cos, const Tensor& sin) {
     const int64_t B = x.size(0), T = x.size(1), H = x.size(2), D = x.size(3);
+    check_device(cos, x, "rope_heads: cos");
+    check_device(sin, x, "rope_heads: sin");
     const Tensor xc = x.contiguous(), y = at::empty({B, H, T, D}, x.options());
     Launch at(x);
     check(otx_rope_heads_fwd(xc.data_ptr(), cos.data_ptr<float>(), sin.data_ptr<float>(), y.data_ptr(), (int)B, (int)T,
