@@ -38,6 +38,15 @@ void check_device(const Tensor& t, const Tensor& like, const char* what) {
               ": Expected all tensors to be on the same device");
 }
 
+// A saved tensor as the backward reads it. A saved-tensor hook may hand back anything, and
+// the kernels take only its address: its size, type and device have to be what was saved.
+Tensor saved_as(const Tensor& t, at::IntArrayRef sizes, at::ScalarType type, const Tensor& grad, const char* what) {
+  TORCH_CHECK_VALUE(t.defined() && t.sizes() == sizes && t.scalar_type() == type && t.device() == grad.device(), what,
+                    " came back from the saved tensors as ", t.toString(), t.defined() ? t.sizes() : at::IntArrayRef(),
+                    ", not as the ", type, " ", sizes, " on ", grad.device(), " that the backward needs");
+  return t.contiguous();
+}
+
 // The stream that work on t's device is queued on, with that device made current.
 struct Launch {
   c10::DeviceGuard guard;
@@ -83,12 +92,15 @@ struct Linear : Function<Linear> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &w = saved[1];
-    const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+    const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
+    const int64_t K = shape.back(), N = grads[0].size(-1), M = grads[0].numel() / N;
     const Tensor dy = grads[0].reshape({M, N}).contiguous();
+    const Tensor x = saved_as(saved[0], {M, K}, at::kBFloat16, dy, "linear: the input");
+    TORCH_CHECK_VALUE(saved[1].numel() == N * K, "linear: the weight came back as ", saved[1].sizes());
+    const Tensor w = saved_as(saved[1], saved[1].sizes(), at::kBFloat16, dy, "linear: the weight");
     Tensor dx, dw;
     if (ctx->needs_input_grad(0))  // dx[m][k] = sum_n dy[m][n] w[n][k]
-      dx = gemm(dy, N, 1, w, 1, K, M, K, N).view(ctx->saved_data["shape"].toIntVector());
+      dx = gemm(dy, N, 1, w, 1, K, M, K, N).view(shape);
     if (ctx->needs_input_grad(1))  // dw[n][k] = sum_m dy[m][n] x[m][k]
       dw = gemm(dy, 1, N, x, 1, K, N, K, M);
     return {dx, dw};
@@ -116,9 +128,12 @@ struct RMSNorm : Function<RMSNorm> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &w = saved[1], &rstd = saved[2];
-    const int64_t D = x.size(-1), rows = x.numel() / D;
     const Tensor dy = grads[0].contiguous();
+    const int64_t D = dy.size(-1), rows = dy.numel() / D;
+    const Tensor x = saved_as(saved[0], dy.sizes(), dy.scalar_type(), dy, "rms_norm: the input");
+    TORCH_CHECK_VALUE(saved[1].numel() == D, "rms_norm: the weight came back as ", saved[1].sizes());
+    const Tensor w = saved_as(saved[1], saved[1].sizes(), dy.scalar_type(), dy, "rms_norm: the weight");
+    const Tensor rstd = saved_as(saved[2], {rows}, at::kFloat, dy, "rms_norm: 1 / rms");
     const Tensor dx = at::empty_like(x), dw = at::empty({D}, x.options().dtype(at::kFloat));
     {
       Launch at(x);
@@ -141,7 +156,8 @@ struct SiLU : Function<SiLU> {
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const Tensor x = ctx->get_saved_variables()[0], dy = grads[0].contiguous(), dx = at::empty_like(x);
+    const Tensor dy = grads[0].contiguous(), dx = at::empty_like(dy);
+    const Tensor x = saved_as(ctx->get_saved_variables()[0], dy.sizes(), dy.scalar_type(), dy, "silu: the input");
     Launch at(x);
     check(otx_silu_bwd(x.data_ptr(), dy.data_ptr(), dx.data_ptr(), x.numel(), dtype_code(x), at.stream),
           "otx_silu_bwd");
@@ -164,8 +180,12 @@ struct SwiGLU : Function<SwiGLU> {
     return h;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const Tensor gu = ctx->get_saved_variables()[0], dh = grads[0].contiguous(), dgu = at::empty_like(gu);
-    const int64_t F = gu.size(-1) / 2;
+    const Tensor dh = grads[0].contiguous();
+    const int64_t F = dh.size(-1);
+    std::vector<int64_t> shape = dh.sizes().vec();
+    shape.back() = 2 * F;
+    const Tensor gu = saved_as(ctx->get_saved_variables()[0], shape, dh.scalar_type(), dh, "swiglu: the input");
+    const Tensor dgu = at::empty_like(gu);
     Launch at(gu);
     check(otx_swiglu_bwd(gu.data_ptr(), dh.data_ptr(), dgu.data_ptr(), gu.numel() / (2 * F), (int)F, dtype_code(gu),
                          at.stream),
@@ -191,10 +211,12 @@ struct RopeHeads : Function<RopeHeads> {  // [B, T, H, D] -> [B, H, T, D]
     const auto saved = ctx->get_saved_variables();
     const Tensor dy = grads[0].contiguous();
     const int64_t B = dy.size(0), H = dy.size(1), T = dy.size(2), D = dy.size(3);
+    const Tensor cos = saved_as(saved[0], {T, D / 2}, at::kFloat, dy, "rope_heads: cos");
+    const Tensor sin = saved_as(saved[1], {T, D / 2}, at::kFloat, dy, "rope_heads: sin");
     const Tensor dx = at::empty({B, T, H, D}, dy.options());
     Launch at(dy);
-    check(otx_rope_heads_bwd(dy.data_ptr(), saved[0].data_ptr<float>(), saved[1].data_ptr<float>(), dx.data_ptr(),
-                             (int)B, (int)T, (int)H, (int)D, dtype_code(dy), at.stream),
+    check(otx_rope_heads_bwd(dy.data_ptr(), cos.data_ptr<float>(), sin.data_ptr<float>(), dx.data_ptr(), (int)B, (int)T,
+                             (int)H, (int)D, dtype_code(dy), at.stream),
           "otx_rope_heads_bwd");
     return {dx, Tensor(), Tensor()};
   }
@@ -234,10 +256,11 @@ struct Embedding : Function<Embedding> {
     return out.view(shape);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const Tensor flat = ctx->get_saved_variables()[0];
-    const int64_t V = ctx->saved_data["V"].toInt(), D = ctx->saved_data["D"].toInt(), n = flat.numel();
-    TORCH_CHECK(grads[0].device() == flat.device(), "grad_output is on ", grads[0].device(), " but the ids are on ",
-                flat.device());
+    const Tensor ids = ctx->get_saved_variables()[0];
+    const int64_t V = ctx->saved_data["V"].toInt(), D = ctx->saved_data["D"].toInt(), n = grads[0].numel() / D;
+    TORCH_CHECK(grads[0].device() == ids.device(), "grad_output is on ", grads[0].device(), " but the ids are on ",
+                ids.device());
+    const Tensor flat = saved_as(ids, {n}, at::kLong, grads[0], "embedding: the ids");
     const Tensor g = grads[0].reshape({-1, D}).to((at::ScalarType)ctx->saved_data["dtype"].toInt()).contiguous();
     const Tensor gw = at::empty({V, D}, g.options());
     Launch at(g);
@@ -269,13 +292,17 @@ struct Loss : Function<Loss> {  // logits [N, V], labels [N] -> (ce, z)
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor x = saved[0].contiguous(), lab = saved[1].contiguous();
+    TORCH_CHECK_VALUE(saved[0].dim() == 2, "loss: the logits came back from the saved tensors as ", saved[0].sizes());
+    const int64_t N = saved[0].size(0);
+    dtype_code(saved[0]);
+    const Tensor x = saved_as(saved[0], saved[0].sizes(), saved[0].scalar_type(), grads[0], "loss: the logits");
+    const Tensor lab = saved_as(saved[1], {N}, at::kLong, x, "loss: the labels");
+    const Tensor stats = saved_as(saved[2], {5, N}, at::kFloat, x, "loss: the row statistics");
     const Tensor g = at::stack({grads[0].reshape({}).to(at::kFloat), grads[1].reshape({}).to(at::kFloat)});
     const Tensor dx = at::empty_like(x);
     Launch at(x);
-    check(otx_ce_zloss_bwd(x.data_ptr(), lab.data_ptr<int64_t>(), saved[2].data_ptr<float>(), g.data_ptr<float>(),
-                           x.size(0), (int)x.size(1), dtype_code(x), ctx->saved_data["coeff"].toDouble(), dx.data_ptr(),
-                           at.stream),
+    check(otx_ce_zloss_bwd(x.data_ptr(), lab.data_ptr<int64_t>(), stats.data_ptr<float>(), g.data_ptr<float>(), N,
+                           (int)x.size(1), dtype_code(x), ctx->saved_data["coeff"].toDouble(), dx.data_ptr(), at.stream),
           "otx_ce_zloss_bwd");
     return {dx, Tensor(), Tensor()};
   }
@@ -321,24 +348,30 @@ struct Attention : Function<Attention> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor q = saved[0].contiguous(), k = saved[1].contiguous(), v = saved[2].contiguous(),
-                 o = saved[3].contiguous(), lse = saved[4].contiguous(), dout = grads[0].contiguous();
-    const int B = (int)q.size(0), H = (int)q.size(1), Hkv = (int)k.size(1), S = (int)q.size(2), D = (int)q.size(3);
+    const Tensor dout = grads[0].contiguous();
+    const auto type = dout.scalar_type();
+    for (int i = 0; i < 3; i++)
+      TORCH_CHECK_VALUE(saved[i].is_contiguous(), "q, k and v must come back from the saved tensors contiguous");
+    TORCH_CHECK_VALUE(saved[1].dim() == 4 && saved[1].size(1) > 0 && dout.size(1) % saved[1].size(1) == 0,
+                      "attention: k came back from the saved tensors as ", saved[1].sizes());
+    const int B = (int)dout.size(0), H = (int)dout.size(1), Hkv = (int)saved[1].size(1), S = (int)dout.size(2),
+              D = (int)dout.size(3);
+    const Tensor q = saved_as(saved[0], {B, H, S, D}, type, dout, "attention: q");
+    const Tensor k = saved_as(saved[1], {B, Hkv, S, D}, type, dout, "attention: k");
+    const Tensor v = saved_as(saved[2], {B, Hkv, S, D}, type, dout, "attention: v");
+    const Tensor o = saved_as(saved[3], {B, H, S, D}, type, dout, "attention: o");
+    const Tensor lse = saved_as(saved[4], {B, H, S}, at::kFloat, dout, "attention: the logsumexp");
     const int w = (int)ctx->saved_data["window"].toInt(), dt = dtype_code(q);
-    for (const Tensor& t : {k, v, o, dout})
-      TORCH_CHECK_VALUE(t.device() == q.device() && t.scalar_type() == q.scalar_type(),
-                        "saved tensors and grad_output must match q in dtype and device");
-    TORCH_CHECK_VALUE(dout.sizes() == q.sizes() && o.sizes() == q.sizes(), "o and grad_output must match q in shape");
-    TORCH_CHECK_VALUE(lse.device() == q.device() && lse.scalar_type() == at::kFloat && lse.numel() == (int64_t)B * H * S,
-                      "lse must be float32 [B, H, T] on q's device");
     const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     Launch at(q);
     const size_t nbytes = otx_attn_bwd_workspace_bytes(B, H, Hkv, S, D, w);
     const Workspace ws(q, nbytes);
-    if (saved.size() > 5) {
-      const Tensor sc = saved[5].contiguous();
-      TORCH_CHECK_VALUE(sc.device() == q.device() && sc.scalar_type() == at::kFloat,
-                        "score_cache must be a float32 tensor on q's device");
+    // no storage behind a checkpoint's placeholder (stride 0): never read
+    const bool cached = saved.size() > 5 && saved[5].numel() > 0 && saved[5].stride(0) != 0;
+    if (cached) {
+      const Tensor& sc = saved[5];
+      TORCH_CHECK_VALUE(sc.device() == q.device() && sc.scalar_type() == at::kFloat && sc.is_contiguous(),
+                        "score_cache must be a contiguous float32 tensor on q's device");
       check(otx_attn_bwd_sc(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(),
                             dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), sc.data_ptr<float>(),
                             (size_t)sc.numel() * 4, B, H, Hkv, S, D, w, dt, ws.ptr, nbytes, 0, 7, at.stream),

@@ -95,3 +95,48 @@ def test_saved_input_changed_in_place_is_refused(name):
         x.add_(1.0)
     with pytest.raises(RuntimeError, match="inplace"):
         torch.autograd.grad(y.sum(), [x])
+
+
+@pytest.mark.parametrize("name", [n for n in NAMES if n != "heads"])
+def test_a_saved_tensor_that_comes_back_changed_is_refused(name):
+    """A saved-tensor hook may hand back anything, and the kernels see only addresses: every saved tensor that comes back
+    shorter, longer or in another type is a ValueError, and one of other strides is either that or read correctly."""
+    call, inputs, nsaved = _cases()[name]
+    ref = torch.autograd.grad(call(*inputs).sum(), inputs)
+
+    def backward(which, change):
+        count = iter(range(nsaved))
+
+        def unpack(packed):
+            i, t = packed
+            return change(t) if i == which else t
+
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (next(count), t.detach()), unpack):
+            y = call(*inputs)
+        return torch.autograd.grad(y.sum(), inputs)
+
+    other = {torch.bfloat16: torch.float32, torch.float32: torch.bfloat16, torch.int64: torch.int32}
+    changes = {
+        "shorter": lambda t: t[: t.shape[0] - 1].contiguous(),
+        "narrower": lambda t: t[..., : t.shape[-1] - 1].contiguous(),
+        "another type": lambda t: t.to(other[t.dtype]),
+    }
+    for which in range(nsaved):
+        for what, change in changes.items():
+            if (name, which, what) == ("loss", 0, "another type"):
+                continue  # the loss takes logits of either type
+            print(f"autograd node {name}: saved tensor {which} {what}", flush=True)
+            with pytest.raises((ValueError, RuntimeError)) as err:
+                backward(which, change)
+            # the loss's logits of another row count or width are refused as a gradient of the wrong shape
+            assert isinstance(err.value, ValueError) or (name, which) == ("loss", 0), err.value
+        strided = lambda t: t.transpose(-1, -2).contiguous().transpose(-1, -2) if t.dim() > 1 else t[:, None].expand(
+            -1, 2).contiguous()[:, 0]
+        try:
+            got = backward(which, strided)
+        except ValueError as err:
+            assert name.startswith("attention") and "contiguous" in str(err)
+        else:
+            for a, b in zip(got, ref):
+                assert torch.equal(_bits(a), _bits(b)), f"saved tensor {which} with other strides"
+    torch.cuda.synchronize()
