@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from .. import _lib
+from . import _nodes
 
 __all__ = ["Embedding", "embedding"]
 
@@ -32,7 +32,7 @@ def embedding(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         # RuntimeError, as torch.nn.Embedding raises for the same mismatch.
         raise RuntimeError(f"ids are on {ids.device} but weight is on {weight.device}: "
                            "Expected all tensors to be on the same device")
-    return _lib.autograd().embedding(ids, weight)
+    return _nodes.call("embedding", ids, weight)
 
 
 class Embedding(nn.Module):

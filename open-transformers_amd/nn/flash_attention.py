@@ -25,6 +25,7 @@ import threading
 import torch
 
 from .. import _lib
+from . import _nodes
 
 __all__ = [
     "causal_flash_attention",
@@ -327,11 +328,17 @@ class _CausalFlashAttention(torch.autograd.Function):
         return dq, dk, dv, None, None
 
 
+def _python_node(mode):
+    """Whether a call takes the Python node: under activation checkpointing's modes,
+    which record, replay or leave out what the forward saves, and while
+    torch.jit.trace records (it cannot see a native node's launch)."""
+    return mode == _SC_PLACEHOLDER or getattr(_ckpt, "state", None) is not None or _nodes.tracing()
+
+
 def _native_attention(q, k, v, window, int8pv, mode):
-    """The native node, for every call but those under activation checkpointing's
-    modes, which record, replay or leave out what the forward saves (the Python
-    nodes above).  It saves the same tensors in the same order as they do, so it
-    serves as the recompute of a first forward that they ran."""
+    """The native node, for every other call.  It saves the same tensors in the same
+    order as the Python nodes above, so it serves as the recompute of a first forward
+    that they ran."""
     sc = None
     if mode == _SC_KEEP:
         B, H, S, _ = q.shape
@@ -347,7 +354,7 @@ def causal_flash_attention(
         raise ValueError("causal_flash_attention is deterministic: dropout must be 0.0")
     _check_inputs(q, k, v, window)
     mode = _score_cache_mode(q, k, v)
-    if mode == _SC_PLACEHOLDER or getattr(_ckpt, "state", None) is not None:
+    if _python_node(mode):
         return _CausalFlashAttention.apply(q, k, v, window, mode)
     return _native_attention(q, k, v, window, False, mode)
 
@@ -430,6 +437,6 @@ def int8pv_causal_flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Ten
     if q.dtype != torch.bfloat16:
         raise ValueError(f"int8pv_causal_flash_attention takes bfloat16 inputs, got {q.dtype}")
     mode = _score_cache_mode(q, k, v)
-    if mode == _SC_PLACEHOLDER or getattr(_ckpt, "state", None) is not None:
+    if _python_node(mode):
         return _Int8PVFlashAttention.apply(q, k, v, window, mode)
     return _native_attention(q, k, v, window, True, mode)

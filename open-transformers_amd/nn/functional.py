@@ -21,6 +21,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from . import _nodes
 
 __all__ = ["linear", "rms_norm", "silu", "swiglu", "rope_heads", "heads", "merge_heads"]
 
@@ -55,7 +56,7 @@ def gemm_bf16(a: torch.Tensor, a_strides: tuple[int, int], b: torch.Tensor, b_st
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w^T (no bias), bf16 operands, serial binary32 fold, bf16 result."""
     _need_gpu(x, w)
-    return _lib.autograd().linear(x, w)
+    return _nodes.call("linear", x, w)
 
 
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -63,7 +64,7 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     _need_gpu(x, w)
     if x.dtype not in _DT:
         raise ValueError(f"dtype {x.dtype} not supported")
-    return _lib.autograd().rms_norm(x, w, float(eps))
+    return _nodes.call("rms_norm", x, w, float(eps))
 
 
 def silu(x: torch.Tensor) -> torch.Tensor:
@@ -71,7 +72,7 @@ def silu(x: torch.Tensor) -> torch.Tensor:
     _need_gpu(x)
     if x.dtype not in _DT:
         raise ValueError(f"dtype {x.dtype} not supported")
-    return _lib.autograd().silu(x)
+    return _nodes.call("silu", x)
 
 
 def swiglu(gu: torch.Tensor) -> torch.Tensor:
@@ -82,7 +83,7 @@ def swiglu(gu: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"dtype {gu.dtype} not supported")
     if gu.shape[-1] % 16:
         raise ValueError(f"swiglu: last dimension {gu.shape[-1]} is not a multiple of 16")
-    return _lib.autograd().swiglu(gu)
+    return _nodes.call("swiglu", gu)
 
 
 def rope_heads(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
@@ -97,7 +98,7 @@ def rope_heads(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     for name, t in (("cos", cos), ("sin", sin)):
         if t.dtype != torch.float32 or tuple(t.shape) != (T, D // 2):
             raise ValueError(f"rope_heads: {name} must be binary32 [{T}, {D // 2}], got {t.dtype} {tuple(t.shape)}")
-    return _lib.autograd().rope_heads(x, cos.contiguous(), sin.contiguous())
+    return _nodes.call("rope_heads", x, cos.contiguous(), sin.contiguous())
 
 
 def heads(x: torch.Tensor) -> torch.Tensor:
@@ -106,7 +107,7 @@ def heads(x: torch.Tensor) -> torch.Tensor:
     if x.dtype not in _DT or x.dim() != 4 or x.shape[-1] % 8:
         raise ValueError(f"heads takes a bf16/binary32 [B, T, H, D] tensor with D a multiple of 8, got {x.dtype} "
                          f"{tuple(x.shape)}")
-    return _lib.autograd().swap_heads(x)
+    return _nodes.call("swap_heads", x)
 
 
 def merge_heads(o: torch.Tensor) -> torch.Tensor:
@@ -116,4 +117,4 @@ def merge_heads(o: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"merge_heads takes a bf16/binary32 [B, H, T, D] tensor with D a multiple of 8, got "
                          f"{o.dtype} {tuple(o.shape)}")
     B, H, T, D = o.shape
-    return _lib.autograd().swap_heads(o).view(B, T, H * D)
+    return _nodes.call("swap_heads", o).view(B, T, H * D)

@@ -16,6 +16,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from . import _nodes
 
 __all__ = ["fused_ce_z_loss", "ce_zloss_forward", "ce_zloss_backward"]
 
@@ -70,4 +71,4 @@ def fused_ce_z_loss(logits: torch.Tensor, labels: torch.Tensor, coeff: float, *,
     if labels.dim() != 1:
         labels = labels.reshape(-1)
     _check(logits, labels)
-    return _lib.autograd().loss(logits, labels, float(coeff))
+    return _nodes.call("loss", logits, labels, float(coeff))

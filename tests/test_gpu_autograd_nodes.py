@@ -97,6 +97,22 @@ def test_saved_input_changed_in_place_is_refused(name):
         torch.autograd.grad(y.sum(), [x])
 
 
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("name", NAMES)
+def test_a_trace_replays_the_operator(name, grad):
+    """torch.jit.trace, recorded with inputs that do and do not require gradients: the traced call on other values gives
+    the operator's bytes and gradients."""
+    call, inputs, _ = _cases()[name]
+    print(f"autograd node {name}: traced", flush=True)
+    traced = torch.jit.trace(call, tuple(t.detach().requires_grad_(grad) for t in inputs), check_trace=False)
+    args = [(t.detach() * 0.5).requires_grad_() for t in inputs]
+    y, ref = traced(*args), call(*args)
+    assert torch.equal(_bits(y.detach()), _bits(ref.detach()))
+    dy = torch.randn(y.shape, device=DEV).to(y.dtype)
+    for a, b in zip(torch.autograd.grad(y, args, dy), torch.autograd.grad(ref, args, dy)):
+        assert torch.equal(_bits(a), _bits(b))
+
+
 @pytest.mark.parametrize("name", [n for n in NAMES if n != "heads"])
 def test_a_saved_tensor_that_comes_back_changed_is_refused(name):
     """A saved-tensor hook may hand back anything, and the kernels see only addresses: every saved tensor that comes back
