@@ -102,16 +102,20 @@ def load() -> ctypes.CDLL:
 
 def autograd():
     """The native autograd nodes (csrc/otx_autograd.cpp), imported once; raises
-    RuntimeError if they have not been built."""
+    RuntimeError if they have not been built, or not against the C ABI of the library
+    that is loaded."""
     global _AUTOGRAD
     if _AUTOGRAD is None:
-        load()
         path = PKG_DIR / AUTOGRAD_LIB
+        rebuild = "run `python -c 'import __graft_entry__ as g; g.build()'` first"
+        abi = native_build_info().get("abi_blake2b")
         if not path.exists():
-            raise RuntimeError(f"{path} is missing: run `python -c 'import __graft_entry__ as g; g.build()'` first")
+            raise RuntimeError(f"{path} is missing: {rebuild}")
         spec = importlib.util.spec_from_file_location("_otx_autograd", path)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
+        if getattr(mod, "abi_blake2b", None) != abi:
+            raise RuntimeError(f"{path} was built against another C ABI than {lib_path()}: {rebuild}")
         _AUTOGRAD = mod
     return _AUTOGRAD
 

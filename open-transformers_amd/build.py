@@ -67,6 +67,15 @@ def sources_digest() -> str:
     return h.hexdigest()
 
 
+def abi_digest() -> str:
+    """blake2b-16 (hex) over the C ABI's headers: what the library and the autograd
+    nodes, which are built one after the other, have to agree on."""
+    h = hashlib.blake2b(digest_size=16)
+    for p in sorted(INCLUDE.glob("*.h")):
+        h.update(p.name.encode() + b"\0" + p.read_bytes() + b"\0")
+    return h.hexdigest()
+
+
 def tree_stamp() -> dict:
     """{"commit": 12-hex HEAD or "unknown", "dirty": bool or None} of the checkout
     holding this package; dirty means a stamped path differs from HEAD or holds
@@ -124,7 +133,7 @@ def link(out: pathlib.Path, stamp: dict | None = None, digest: str | None = None
     stamp_obj = out.parent / (out.stem + ".stamp.o")
     cxx = shutil.which("g++") or "g++"
     _run([cxx, *STAMP_FLAGS, f'-DOTX_STAMP_COMMIT="{stamp["commit"]}"', f'-DOTX_STAMP_DIRTY="{dirty}"',
-          f'-DOTX_STAMP_SOURCES="{digest}"', "-c", str(CSRC / STAMP_SOURCE), "-o", str(stamp_obj)])
+          f'-DOTX_STAMP_SOURCES="{digest}"', f'-DOTX_STAMP_ABI="{abi_digest()}"', "-c", str(CSRC / STAMP_SOURCE), "-o", str(stamp_obj)])
     tmp = out.with_suffix(".so.tmp")
     try:
         _run([hipcc_path(), "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objs), str(stamp_obj), "-o", str(tmp)])
@@ -169,6 +178,22 @@ def build(verbose: bool = False) -> pathlib.Path:
 
 
 AUTOGRAD_LIB = "_otx_autograd.so"
+AUTOGRAD_SOURCE = "otx_autograd.cpp"
+AUTOGRAD_FLAGS = ["-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                  "-DTORCH_API_INCLUDE_EXTENSION_H"]
+AUTOGRAD_LIBS = ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+
+
+def autograd_digest() -> str:
+    """sources_digest() of the autograd nodes: their source, the C ABI's headers, the
+    flags and torch's version."""
+    import torch
+
+    h = hashlib.blake2b(digest_size=16)
+    for p in [CSRC / AUTOGRAD_SOURCE] + sorted(INCLUDE.glob("*.h")):
+        h.update(p.name.encode() + b"\0" + p.read_bytes() + b"\0")
+    h.update(" ".join(AUTOGRAD_FLAGS + AUTOGRAD_LIBS + [torch.__version__]).encode())
+    return h.hexdigest()
 
 
 def build_autograd() -> pathlib.Path:
@@ -182,11 +207,10 @@ def build_autograd() -> pathlib.Path:
     tmp = out.with_suffix(".so.tmp")
     cxx = shutil.which("g++") or "g++"
     includes = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"]]
-    _run([cxx, "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-          "-DTORCH_API_INCLUDE_EXTENSION_H", f"-I{INCLUDE}", *(f"-isystem{p}" for p in includes),
-          str(CSRC / "otx_autograd.cpp"), "-o", str(tmp), f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN",
-          *(f"-L{p}" for p in cpp_extension.library_paths("cuda")), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch",
-          "-ltorch_python"])
+    _run([cxx, *AUTOGRAD_FLAGS, f'-DOTX_STAMP_SOURCES="{autograd_digest()}"', f'-DOTX_STAMP_ABI="{abi_digest()}"',
+          f"-I{INCLUDE}", *(f"-isystem{p}" for p in includes), str(CSRC / AUTOGRAD_SOURCE), "-o", str(tmp),
+          f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN",
+          *(f"-L{p}" for p in cpp_extension.library_paths("cuda")), *AUTOGRAD_LIBS])
     os.replace(tmp, out)
     return out
 

@@ -405,6 +405,8 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const std::o
 }  // namespace
 
 PYBIND11_MODULE(_otx_autograd, m) {
+  m.attr("sources_blake2b") = OTX_STAMP_SOURCES;
+  m.attr("abi_blake2b") = OTX_STAMP_ABI;
   m.def("linear", torch::wrap_pybind_function(linear));
   m.def("rms_norm", torch::wrap_pybind_function(rms_norm));
   m.def("silu", torch::wrap_pybind_function(silu));

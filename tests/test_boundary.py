@@ -73,6 +73,19 @@ def test_build_info_reports_the_stamp_of_the_loaded_library():
     assert info["sources_blake2b"] == build.sources_digest()
 
 
+def test_autograd_nodes_carry_the_stamp_of_this_tree(monkeypatch):
+    """The nodes were built from this tree's source, against the header of the loaded library; a library of another C ABI
+    is refused."""
+    from open_transformers_amd import build
+
+    assert _lib.autograd().sources_blake2b == build.autograd_digest()
+    assert _lib.autograd().abi_blake2b == _lib.native_build_info()["abi_blake2b"] == build.abi_digest()
+    monkeypatch.setattr(_lib, "_AUTOGRAD", None)
+    monkeypatch.setattr(_lib, "native_build_info", lambda: {"abi_blake2b": "0" * 32})
+    with pytest.raises(RuntimeError, match="C ABI"):
+        _lib.autograd()
+
+
 def test_rebuilt_library_is_stamped_with_head(tmp_path):
     # Relink the library from the built objects with a fresh stamp (no kernel
     # recompilation) and read the stamp back from the new file.
