@@ -50,9 +50,16 @@ extern "C" {
 int otx_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B, int H, int Hkv, int S, int D,
                  int window, int dtype, void* stream);
 
-/* Same as otx_attn_fwd with an explicit launch variant (0 = default; 1 and 2 use
- * other workgroup shapes and grid orders).  Every variant produces identical bits;
- * the variants exist so that launch-configuration invariance can be tested. */
+/* Same as otx_attn_fwd with an explicit launch variant.  Every variant produces
+ * identical bits; the variants exist so that launch-configuration invariance can
+ * be tested, and any kernel on any shape:
+ *   0  the default: the tile kernels (four waves per 32-row block) for grids of
+ *      few blocks, otherwise one wave per block and four waves per workgroup
+ *   1  two waves per workgroup, the other grid order
+ *   2  one wave per workgroup
+ *   3  variant 0 without the tile kernels: what it launches on large grids
+ * binary32 forwards and dK/dV have tile kernels only; there the variants differ in
+ * the rows per workgroup. */
 int otx_attn_fwd_ex(const void* q, const void* k, const void* v, void* o, float* lse, int B, int H, int Hkv, int S,
                     int D, int window, int dtype, int variant, void* stream);
 
@@ -68,11 +75,12 @@ int otx_attn_bwd(const void* q, const void* k, const void* v, const void* o, con
                  void* dq, void* dk, void* dv, int B, int H, int Hkv, int S, int D, int window, int dtype,
                  void* workspace, size_t workspace_bytes, void* stream);
 
-/* otx_attn_bwd with an explicit launch variant (see otx_attn_fwd_ex).  For bf16
- * inputs the dK/dV launch of variant 0 picks one of two kernel forms by shape
- * (two key blocks per workgroup when the four-key-block grid would fill the
- * device only once) and variant 2 picks the other form, so that comparing
- * variants 0 and 2 compares both forms on every shape. */
+/* otx_attn_bwd with an explicit launch variant (see otx_attn_fwd_ex).  bf16 dK/dV
+ * has three forms: the tile kernel; four key blocks per workgroup; and, with the
+ * score cache (otx_attn_bwd_sc), two key blocks per workgroup.  Variant 0 picks by
+ * shape, variant 3 picks between the last two, and variant 2 takes the one of them
+ * that variant 3 does not, so that variants 0, 2 and 3 with the cache run all three
+ * on shapes of few blocks. */
 int otx_attn_bwd_ex(const void* q, const void* k, const void* v, const void* o, const float* lse, const void* dout,
                     void* dq, void* dk, void* dv, int B, int H, int Hkv, int S, int D, int window, int dtype,
                     void* workspace, size_t workspace_bytes, int variant, void* stream);

@@ -14,11 +14,12 @@
 //          P = exp(RN(s*sigma) - LSE) and dS = RN(P * RN(dP - Dsum)), writes
 //          its dS row segment to the workspace and feeds P / dS (broadcast to
 //          both half-waves) into the dV^T and dK^T chains over queries.
-//          A second bf16 form (attn_dkdv_bf16_kb2_kernel) gives two key blocks
-//          to a workgroup of four waves and splits each tile into a dP/softmax
-//          phase per (query block, key block) pair and a dV/dK fold phase; the
-//          launcher takes it when the one-wave-per-key-block grid would fill
-//          the device only once (its long chunks would then set the time).
+//          A second form (attn_dkdv_bf16_kb2_kernel: bf16, score cache) gives two
+//          key blocks to a workgroup of four waves and splits each tile into a
+//          dP/softmax phase per (query block, key block) pair and a dV/dK fold
+//          phase; the launcher takes it when the one-wave-per-key-block grid would
+//          fill the device only once (its long chunks would then set the time)
+//          and under a window.
 //   dq   : one wave per 32-query block; dQ^T chain over the processed keys
 //          reading the stored dS tiles, scaled by sigma at the end.
 // The dkdv of binary32 inputs, and dkdv and dq of grids too small for one wave
@@ -474,14 +475,14 @@ __global__ __launch_bounds__(64 * NWK, 1) void attn_dkdv_bf16_kernel(
   }
 }
 
-// bf16 dK/dV kernel with two key blocks per workgroup of four waves.  Each
-// 64-query tile of a head runs in two phases separated by a barrier:
+// bf16 dK/dV kernel with two key blocks per workgroup of four waves, on the score
+// cache (without it the tile kernel of attn_tile.hip serves the grids that this one
+// would).  Each 64-query tile of a head runs in two phases separated by a barrier:
 //   A: wave w takes one (query block, key block) pair, qa + (w & 1) against
-//      kt0 + (w >> 1): its dP (and, without the score cache, its scores) are
-//      one v_mfma_f32_16x16x1_4b_f32 chain over d (one fma per output and step,
-//      the contract's serial fold), then P = exp(RN(s - LSE)) and
-//      dS = RN(P * RN(dP - Dsum)) lane-locally; P and dS go to LDS (and dS to
-//      the workspace for the dQ kernel).  With the score cache the chain's V
+//      kt0 + (w >> 1): its dP is one v_mfma_f32_16x16x1_4b_f32 chain over d (one
+//      fma per output and step, the contract's serial fold), then
+//      P = exp(RN(s - LSE)) and dS = RN(P * RN(dP - Dsum)) lane-locally; P and dS
+//      go to LDS (and dS to the workspace for the dQ kernel).  The chain's V
 //      operand is held in registers for most of d (it is the same for every
 //      tile), since four d16 reads per two 16x16 products saturate the LDS,
 //      and each remaining read serves a pair of d (CBSZ / ABID and BLGP
@@ -495,12 +496,12 @@ __global__ __launch_bounds__(64 * NWK, 1) void attn_dkdv_bf16_kernel(
 // split of work between waves differs.  With half the key blocks per
 // workgroup the grid has twice the workgroups, so the causal triangle's long
 // chunks no longer set the time of a grid that fills the device only once.
-template <int D, bool SC>
+template <int D>
 __global__ __launch_bounds__(256, 1) void attn_dkdv_bf16_kb2_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const uint16_t* __restrict__ dO, const float* __restrict__ lse, const float* __restrict__ dsum,
-    uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, float* __restrict__ ws_ds, int B, int H, int Hkv, int S,
-    int window, float sigma, int order, const float* __restrict__ scache) {
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ v, const uint16_t* __restrict__ dO,
+    const float* __restrict__ lse, const float* __restrict__ dsum, uint16_t* __restrict__ dk,
+    uint16_t* __restrict__ dv, float* __restrict__ ws_ds, int B, int H, int Hkv, int S, int window, float sigma,
+    int order, const float* __restrict__ scache) {
   constexpr int KB = 2;                      // key blocks per workgroup
   constexpr int NI = D / 64;                 // dV / dK chains per accumulator kind
   constexpr int CH = D / 8;                  // 16-byte chunks per global row
@@ -509,11 +510,11 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_bf16_kb2_kernel(
   constexpr int UK = RPB / 16;               // 16-byte units per padded row
   constexpr int QT_BYTES = 64 * RPB;         // one 64-row tile of Q (or dO)
   constexpr int SLOT = 2 * QT_BYTES + 2 * 64 * 4;  // Q, dO, LSE, Dsum
-  constexpr int KV_BYTES = KB * 32 * RPB;    // K (or V) rows of the workgroup
+  constexpr int KV_BYTES = KB * 32 * RPB;    // V rows of the workgroup
   constexpr int XPB = 36 * 4;                // row pitch of an exchanged 32x32 tile (bytes)
   constexpr int XT_BYTES = 32 * XPB;
   constexpr int X_BYTES = 2 * KB * 2 * XT_BYTES;  // P and dS of the four pairs
-  constexpr int IN_BYTES = 2 * SLOT + (SC ? 1 : 2) * KV_BYTES + X_BYTES;
+  constexpr int IN_BYTES = 2 * SLOT + KV_BYTES + X_BYTES;
   constexpr int OPE = D + 8;                 // bf16 pitch of the epilogue staging (reuses the buffer)
   constexpr int OS_BYTES = KB * 2 * 32 * OPE * 2;
   constexpr int SMEM = IN_BYTES > OS_BYTES ? IN_BYTES : OS_BYTES;
@@ -523,7 +524,6 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_bf16_kb2_kernel(
   unsigned char* smem = lds + OTX_EXP_LE0_TAB_N * 8;
   unsigned char* Xs = smem + 2 * SLOT;
   uint16_t* Vs = reinterpret_cast<uint16_t*>(Xs + X_BYTES);
-  uint16_t* Ks = Vs + KB * 32 * KPH;         // without the score cache only
   auto slot = [&](int sl) { return smem + sl * SLOT; };
 
   const int nkt = S / OTX_BLK;
@@ -545,20 +545,17 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_bf16_kb2_kernel(
   const int ktl = (kt0 + KB < nkt ? kt0 + KB : nkt) - 1;
   const long tiles_per_head = otx_tile_offset(nkt, window);
 
-  // K and V rows of the workgroup's key blocks (V only with the score cache),
-  // copied straight into LDS in padded rows (copy unit x is row x / UK, slot
-  // x % UK; the pad slot and rows past S copy an in-bounds chunk that is never
-  // read).  The loop's first wait and barrier make them visible.
+  // V rows of the workgroup's key blocks, copied straight into LDS in padded rows
+  // (copy unit x is row x / UK, slot x % UK; the pad slot and rows past S copy an
+  // in-bounds chunk that is never read).
   {
-    static_assert((KB * 32 * UK) % 64 == 0, "the K/V copy units must fill whole copy instructions");
+    static_assert((KB * 32 * UK) % 64 == 0, "the V copy units must fill whole copy instructions");
     const size_t row0 = (size_t)bg * S + (size_t)kt0 * OTX_BLK;
-    const unsigned char* kg = reinterpret_cast<const unsigned char*>(k + row0 * D);
     const unsigned char* vg = reinterpret_cast<const unsigned char*>(v + row0 * D);
     const int rows = S - kt0 * OTX_BLK < KB * OTX_BLK ? S - kt0 * OTX_BLK : KB * OTX_BLK;
     for (int i = wave; i < KB * 32 * UK / 64; i += 4) {
       const int x = 64 * i + L, row = x / UK, su = x % UK;
       const int off = row < rows ? row * (2 * D) + 16 * (su < CH ? su : 0) : 0;
-      if constexpr (!SC) otx_dma16(kg + off, reinterpret_cast<unsigned char*>(Ks) + 64 * i * 16);
       otx_dma16(vg + off, reinterpret_cast<unsigned char*>(Vs) + 64 * i * 16);
     }
   }
@@ -569,7 +566,6 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_bf16_kb2_kernel(
   // lane L: A rows of the 16x16 chains are queries qsub, B columns keys ksub
   const int qsub = (L >> 5) * 16 + (L & 15), ksub = ((L >> 4) & 1) * 16 + (L & 15);
   const uint32_t va_addr = otx_lds_addr(Vs + (akb * 32 + ksub) * KPH);
-  const uint32_t ka_addr = otx_lds_addr(Ks + (akb * 32 + ksub) * KPH);
   // ---- phase B roles: key block kb, dV (role 0) or dK (role 1) ----
   const int bkb = wave >> 1, role = wave & 1, kb = kt0 + bkb;
   const int kb_qhi = kb < nkt ? otx_qblock_hi(kb, window, nkt) : -1;
@@ -629,23 +625,21 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_bf16_kb2_kernel(
 
   if (n_it > 0) issue(0, 0);
   otx_load_exp_table(tab);
-  // With the score cache, phase A's B operand (V row ksub of key block akb) is
+  // Phase A's B operand (V row ksub of key block akb) is
   // the same for every tile.  Its first VR elements are read into registers
   // once, which takes the V reads off the chain's first VR / 2 groups (four
   // d16 reads per two 16x16 products keep the LDS saturated).  7/8 of the row
   // fit beside the exp's registers when the exp runs in chunks of 4.
-  constexpr int VR = SC ? 7 * D / 8 : 1;
+  constexpr int VR = 7 * D / 8;
   float vreg[VR];
-  if constexpr (SC) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this lane's copies of V (and of tile 0) have landed
-    __syncthreads();                                   // every V copy is visible
-    const uint16_t* vr = Vs + (akb * 32 + ksub) * KPH;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this lane's copies of V (and of tile 0) have landed
+  __syncthreads();                                   // every V copy is visible
+  const uint16_t* vr = Vs + (akb * 32 + ksub) * KPH;
 #pragma unroll
-    for (int d = 0; d < VR; d++) vreg[d] = __uint_as_float((uint32_t)vr[d] << 16);
-  }
+  for (int d = 0; d < VR; d++) vreg[d] = __uint_as_float((uint32_t)vr[d] << 16);
   for (int it = 0; it < n_it; ++it) {
     const int sl = it & 1;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this lane's copies of tile it (and of K, V) have landed
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this lane's copies of tile it have landed
     __syncthreads();  // tile it is visible; slot sl ^ 1 and the exchange tiles are no longer read
     if (it + 1 < n_it) issue(it + 1, sl ^ 1);
     const int r = it / nu, u = u_begin + it % nu;
@@ -667,94 +661,60 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_bf16_kb2_kernel(
       const int qw_u = __builtin_amdgcn_readfirstlane(qw), ka_u = __builtin_amdgcn_readfirstlane(ka);
       const long tile = (long)bh * tiles_per_head + otx_tile_offset(qw_u, window) + (ka_u - otx_kblock_lo(qw_u, window));
       float s[16];
-      if constexpr (SC) {
-        // the forward's cached scores of this pair, stored [key][query]
-        const float* src = scache + (tile << 10);
+      // the forward's cached scores of this pair, stored [key][query]
+      const float* src = scache + (tile << 10);
 #pragma unroll
-        for (int qs = 0; qs < 2; qs++)
+      for (int qs = 0; qs < 2; qs++)
 #pragma unroll
-          for (int ks = 0; ks < 2; ks++) {
-            const float4 t4 = *reinterpret_cast<const float4*>(src + (ks * 16 + (L & 15)) * 32 + qs * 16 +
-                                                               4 * (L >> 4));
-            s[qs * 8 + ks * 4 + 0] = t4.x;
-            s[qs * 8 + ks * 4 + 1] = t4.y;
-            s[qs * 8 + ks * 4 + 2] = t4.z;
-            s[qs * 8 + ks * 4 + 3] = t4.w;
-          }
-      }
-      f32x16 pacc = f32x16{}, sacc = f32x16{};
+        for (int ks = 0; ks < 2; ks++) {
+          const float4 t4 = *reinterpret_cast<const float4*>(src + (ks * 16 + (L & 15)) * 32 + qs * 16 +
+                                                             4 * (L >> 4));
+          s[qs * 8 + ks * 4 + 0] = t4.x;
+          s[qs * 8 + ks * 4 + 1] = t4.y;
+          s[qs * 8 + ks * 4 + 2] = t4.z;
+          s[qs * 8 + ks * 4 + 3] = t4.w;
+        }
+      f32x16 pacc = f32x16{};
       const uint32_t drow = dt_a + (aq * 32 + qsub) * RPB;
-      if constexpr (SC) {
-        // dP = dO V^T, one chain over d; read group G = d 2G, 2G + 1, three groups ahead.  Blocks 2j and
-        // 2j + 1 of the 16x16 instruction share their A rows (the same 16 queries): one d16 read serves the
-        // pair of d (blocks 2j read element 2G, blocks 2j + 1 element 2G + 1), and each product takes its
-        // element from one block of the two by the CBSZ / ABID broadcast.  Likewise blocks j and j + 2 share
-        // their B columns (the same 16 keys): past the first VR elements one read of V serves the pair (the
-        // lower half-wave reads 2G, the upper 2G + 1), broadcast by BLGP.  (Measured: this kernel 0 to -0.9 %,
-        // bytes equal.)
-        const uint32_t drow_p = drow + 2 * ((L >> 4) & 1), va_p = va_addr + 2 * (L >> 5);
-        constexpr int NG = D / 2, NGR = VR / 2;
-        auto nrd = [](int Gd) { return Gd < NGR ? 1 : 2; };  // reads of group Gd
-        auto rd = [&](auto gc) {
-          constexpr int Gd = decltype(gc)::value, BK = Gd % 4;
-          otx_lds_bf16<4 * Gd>(opr[BK][0], drow_p);
-          if constexpr (Gd >= NGR) otx_lds_bf16<4 * Gd>(opr[BK][1], va_p);
-        };
-        rd(std::integral_constant<int, 0>{});
-        rd(std::integral_constant<int, 1>{});
-        rd(std::integral_constant<int, 2>{});
-        OtxUnroll<0, NG>::run([&](auto gc) {
-          constexpr int Gd = decltype(gc)::value, BK = Gd % 4;
-          if constexpr (Gd + 3 < NG) {
-            rd(std::integral_constant<int, Gd + 3>{});
-            otx_lds_wait<nrd(Gd + 1) + nrd(Gd + 2) + nrd(Gd + 3)>(opr[BK]);
-          } else if constexpr (Gd + 2 < NG) {
-            otx_lds_wait<nrd(Gd + 1) + nrd(Gd + 2)>(opr[BK]);
-          } else if constexpr (Gd + 1 < NG) {
-            otx_lds_wait<nrd(Gd + 1)>(opr[BK]);
-          } else {
-            otx_lds_wait<0>(opr[BK]);
-          }
-          if constexpr (Gd < NGR) {
-            pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], vreg[2 * Gd], pacc, 1, 0, 0);
-            pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], vreg[2 * Gd + 1], pacc, 1, 1, 0);
-          } else {
-            pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], opr[BK][1], pacc, 1, 0, 1);
-            pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], opr[BK][1], pacc, 1, 1, 2);
-          }
-          asm volatile("" : "+a"(pacc));  // bank BK is consumed before it is read again
-        });
-      } else {
-        // S = Q K^T and dP = dO V^T, two interleaved chains over d; group G = one d
-        const uint32_t qrow = qt_a + (aq * 32 + qsub) * RPB;
-        auto rd = [&](auto gc) {
-          constexpr int Gd = decltype(gc)::value, BK = Gd % 4;
-          otx_lds_bf16<2 * Gd>(opr[BK][0], qrow);
-          otx_lds_bf16<2 * Gd>(opr[BK][1], ka_addr);
-          otx_lds_bf16<2 * Gd>(opr[BK][2], drow);
-          otx_lds_bf16<2 * Gd>(opr[BK][3], va_addr);
-        };
-        rd(std::integral_constant<int, 0>{});
-        rd(std::integral_constant<int, 1>{});
-        rd(std::integral_constant<int, 2>{});
-        OtxUnroll<0, D>::run([&](auto gc) {
-          constexpr int Gd = decltype(gc)::value, BK = Gd % 4;
-          if constexpr (Gd + 3 < D) {
-            rd(std::integral_constant<int, Gd + 3>{});
-            otx_lds_wait<12>(opr[BK]);
-          } else {
-            otx_lds_wait<4 * (D - 1 - Gd)>(opr[BK]);
-          }
-          sacc = otx_mfma16(opr[BK][0], opr[BK][1], sacc);
-          pacc = otx_mfma16(opr[BK][2], opr[BK][3], pacc);
-          // Both products of this group stay ahead of the next group's reads, so
-          // bank BK is consumed before it is read again and never copied while
-          // its loads are in flight.
-          asm volatile("" : "+a"(sacc), "+a"(pacc));
-        });
-#pragma unroll
-        for (int x = 0; x < 16; x++) s[x] = sacc[x] * sigma;  // s = RN(dot * sigma), the contract's score
-      }
+      // dP = dO V^T, one chain over d; read group G = d 2G, 2G + 1, three groups ahead.  Blocks 2j and
+      // 2j + 1 of the 16x16 instruction share their A rows (the same 16 queries): one d16 read serves the
+      // pair of d (blocks 2j read element 2G, blocks 2j + 1 element 2G + 1), and each product takes its
+      // element from one block of the two by the CBSZ / ABID broadcast.  Likewise blocks j and j + 2 share
+      // their B columns (the same 16 keys): past the first VR elements one read of V serves the pair (the
+      // lower half-wave reads 2G, the upper 2G + 1), broadcast by BLGP.  (Measured: this kernel 0 to -0.9 %,
+      // bytes equal.)
+      const uint32_t drow_p = drow + 2 * ((L >> 4) & 1), va_p = va_addr + 2 * (L >> 5);
+      constexpr int NG = D / 2, NGR = VR / 2;
+      auto nrd = [](int Gd) { return Gd < NGR ? 1 : 2; };  // reads of group Gd
+      auto rd = [&](auto gc) {
+        constexpr int Gd = decltype(gc)::value, BK = Gd % 4;
+        otx_lds_bf16<4 * Gd>(opr[BK][0], drow_p);
+        if constexpr (Gd >= NGR) otx_lds_bf16<4 * Gd>(opr[BK][1], va_p);
+      };
+      rd(std::integral_constant<int, 0>{});
+      rd(std::integral_constant<int, 1>{});
+      rd(std::integral_constant<int, 2>{});
+      OtxUnroll<0, NG>::run([&](auto gc) {
+        constexpr int Gd = decltype(gc)::value, BK = Gd % 4;
+        if constexpr (Gd + 3 < NG) {
+          rd(std::integral_constant<int, Gd + 3>{});
+          otx_lds_wait<nrd(Gd + 1) + nrd(Gd + 2) + nrd(Gd + 3)>(opr[BK]);
+        } else if constexpr (Gd + 2 < NG) {
+          otx_lds_wait<nrd(Gd + 1) + nrd(Gd + 2)>(opr[BK]);
+        } else if constexpr (Gd + 1 < NG) {
+          otx_lds_wait<nrd(Gd + 1)>(opr[BK]);
+        } else {
+          otx_lds_wait<0>(opr[BK]);
+        }
+        if constexpr (Gd < NGR) {
+          pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], vreg[2 * Gd], pacc, 1, 0, 0);
+          pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], vreg[2 * Gd + 1], pacc, 1, 1, 0);
+        } else {
+          pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], opr[BK][1], pacc, 1, 0, 1);
+          pacc = __builtin_amdgcn_mfma_f32_16x16x1f32(opr[BK][0], opr[BK][1], pacc, 1, 1, 2);
+        }
+        asm volatile("" : "+a"(pacc));  // bank BK is consumed before it is read again
+      });
       // lane L, register x: query qw*32 + qi(x), key ka*32 + kj(x)
       float lq[16], dsq[16];
 #pragma unroll
@@ -1067,8 +1027,8 @@ hipError_t launch_dq_tile(int dtype, int D, int n16, const void* k, const float*
 template <typename T, int D>
 static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void* v, const void* o, const float* lse,
                                const void* dO, void* dq, void* dk, void* dv, float* dsum, float* ds, int B, int H,
-                               int Hkv, int S, int window, float sigma, int order, int stages, const float* scache,
-                               hipStream_t st) {
+                               int Hkv, int S, int window, float sigma, int order, bool tile, int stages,
+                               const float* scache, hipStream_t st) {
   const long rows = (long)B * H * S;
   hipError_t e = hipSuccess;
   if (stages & 1) {
@@ -1101,7 +1061,7 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
   // 181; nkb 2048, window 256: 216 -> 171; nkb 4096: 1158 against 1234).  Sixteen keys per workgroup rather
   // than 32 up to two key blocks per CU (nkb 512: 95 against 106 us; nkb 1024: 165 against 139), half a block
   // under a window (nkb 128: 20 against 29; nkb 256: 29.2 against 29.1; nkb 512: 51 against 46).
-  const bool tile_dkdv = sizeof(T) == 4 || (nw == 4 && nkb <= (scache != nullptr ? 2 : 8) * cus);
+  const bool tile_dkdv = sizeof(T) == 4 || (tile && nkb <= (scache != nullptr ? 2 : 8) * cus);
   if (!(stages & 2)) {
   } else if (tile_dkdv) {
     const int n16 = nw == 4 ? (2 * nkb <= (window > 0 ? 1 : 4) * cus ? 1 : 2) : nw;
@@ -1114,29 +1074,30 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
                      dim3(64 * NW), 0, st, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,         \
                      (const uint16_t*)dO, lse, dsum, (uint16_t*)dk, (uint16_t*)dv, ds, B, H, Hkv, S, window,   \
                      sigma, order, scache)
-#define OTX_LAUNCH_DKDV_KB2(SC)                                                                              \
-  hipLaunchKernelGGL((attn_dkdv_bf16_kb2_kernel<D, SC>), dim3((unsigned)(((nt + 1) / 2) * B * Hkv)), dim3(256), \
-                     0, st, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dO, lse,  \
-                     dsum, (uint16_t*)dk, (uint16_t*)dv, ds, B, H, Hkv, S, window, sigma, order, scache)
     // Kernel choice (every choice gives the same bits).  Four key blocks per
     // workgroup, one wave each, costs least per key block under a full causal
-    // mask; when that grid fills the device's workgroup slots (one per CU) at
-    // most once, the longest chunks set the time, and two key blocks per
-    // workgroup (phases A/B, twice the workgroups) balance it.  Under a sliding
-    // window with the score cache the two-key-block form wins at any grid size:
-    // its query range per workgroup is two blocks narrower, so fewer tiles have
-    // idle waves at the band's edges.  nw 4 (the default variant) takes that
-    // choice, nw 1 the other one, nw 2 two key blocks with one wave each.
-    const bool one_round = (long)((nt + 3) / 4) * B * Hkv <= otx_cu_count();
-    const bool prefer_kb2 = one_round || (window > 0 && scache != nullptr);
-    const bool kb2 = nw == 4 ? prefer_kb2 : (nw == 1 ? !prefer_kb2 : false);
+    // mask.  With the score cache, when that grid fills the device's workgroup
+    // slots (one per CU) at most once, the longest chunks set the time, and two key
+    // blocks per workgroup (phases A/B, twice the workgroups) balance it; under a
+    // sliding window the two-key-block form wins at any grid size: its query range
+    // per workgroup is two blocks narrower, so fewer tiles have idle waves at the
+    // band's edges.  nw 4 takes that choice, nw 1 the other one, nw 2 two key blocks
+    // with one wave each.
     if (scache != nullptr) {
-      if (kb2) OTX_LAUNCH_DKDV_KB2(true); else if (nw == 2) OTX_LAUNCH_DKDV_BF16(2, true); else OTX_LAUNCH_DKDV_BF16(4, true);
+      const bool one_round = (long)((nt + 3) / 4) * B * Hkv <= otx_cu_count();
+      const bool prefer_kb2 = one_round || window > 0;
+      if (nw == 4 ? prefer_kb2 : nw == 1 && !prefer_kb2)
+        hipLaunchKernelGGL((attn_dkdv_bf16_kb2_kernel<D>), dim3((unsigned)(((nt + 1) / 2) * B * Hkv)), dim3(256), 0, st,
+                           (const uint16_t*)q, (const uint16_t*)v, (const uint16_t*)dO, lse, dsum, (uint16_t*)dk,
+                           (uint16_t*)dv, ds, B, H, Hkv, S, window, sigma, order, scache);
+      else if (nw == 2)
+        OTX_LAUNCH_DKDV_BF16(2, true);
+      else
+        OTX_LAUNCH_DKDV_BF16(4, true);
     } else {
-      if (kb2) OTX_LAUNCH_DKDV_KB2(false); else if (nw == 2) OTX_LAUNCH_DKDV_BF16(2, false); else OTX_LAUNCH_DKDV_BF16(4, false);
+      if (nw == 2) OTX_LAUNCH_DKDV_BF16(2, false); else OTX_LAUNCH_DKDV_BF16(4, false);
     }
 #undef OTX_LAUNCH_DKDV_BF16
-#undef OTX_LAUNCH_DKDV_KB2
   }
   e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -1147,7 +1108,7 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
   // 27); D 64, nqb 512: 39 -> 26, nqb 1024: 40 against 44.  binary32, D 128, nqb 1024: 85 -> 69, 2048: 113
   // against 117; window 256, nqb 512: 32 -> 19, 1024: 30 against 34.
   const long dq_lim = sizeof(T) == 4 ? (window > 0 ? 2 : 4) : D == 64 ? 2 : (window > 0 ? 4 : 8);
-  if ((stages & 4) && nw == 4 && nqb <= dq_lim * cus)
+  if ((stages & 4) && tile && nqb <= dq_lim * cus)
     return launch_dq_tile(sizeof(T) == 2, D, nqb <= 2 * cus ? 1 : 2, k, ds, dq, B, H, Hkv, S, window, sigma, order, st);
   if (stages & 4) {
     switch (nw) {
@@ -1160,23 +1121,24 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
   return hipGetLastError();
 }
 
+// tile: whether the tile kernels may be chosen (binary32 dK/dV has no other form).
 // scache (bf16 only, may be null): the forward's score cache, read by dK/dV instead of recomputing Q K^T.
 hipError_t launch_bwd(int dtype, int D, int nw, const void* q, const void* k, const void* v, const void* o,
                       const float* lse, const void* dO, void* dq, void* dk, void* dv, float* dsum, float* ds, int B,
-                      int H, int Hkv, int S, int window, float sigma, int order, int stages, const float* scache,
-                      hipStream_t st) {
+                      int H, int Hkv, int S, int window, float sigma, int order, bool tile, int stages,
+                      const float* scache, hipStream_t st) {
   if (dtype == 1) {
     if (D == 128)
       return launch_bwd_t<uint16_t, 128>(nw, q, k, v, o, lse, dO, dq, dk, dv, dsum, ds, B, H, Hkv, S, window, sigma,
-                                         order, stages, scache, st);
+                                         order, tile, stages, scache, st);
     return launch_bwd_t<uint16_t, 64>(nw, q, k, v, o, lse, dO, dq, dk, dv, dsum, ds, B, H, Hkv, S, window, sigma,
-                                      order, stages, scache, st);
+                                      order, tile, stages, scache, st);
   }
   if (D == 128)
-    return launch_bwd_t<float, 128>(nw, q, k, v, o, lse, dO, dq, dk, dv, dsum, ds, B, H, Hkv, S, window, sigma, order, stages,
-                                    scache, st);
-  return launch_bwd_t<float, 64>(nw, q, k, v, o, lse, dO, dq, dk, dv, dsum, ds, B, H, Hkv, S, window, sigma, order, stages,
-                                 scache, st);
+    return launch_bwd_t<float, 128>(nw, q, k, v, o, lse, dO, dq, dk, dv, dsum, ds, B, H, Hkv, S, window, sigma, order,
+                                    tile, stages, scache, st);
+  return launch_bwd_t<float, 64>(nw, q, k, v, o, lse, dO, dq, dk, dv, dsum, ds, B, H, Hkv, S, window, sigma, order,
+                                 tile, stages, scache, st);
 }
 
 }  // namespace otx

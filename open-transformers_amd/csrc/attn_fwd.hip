@@ -587,9 +587,9 @@ static hipError_t launch_fwd_t(const void* q, const void* k, const void* v, void
                                const int8_t* qvt = nullptr, const float* vstep = nullptr, float* scache = nullptr) {
   const int nqt = S / OTX_BLK;
   const int nchunk = (nqt + NWQ - 1) / NWQ;
-  // Head-grouped workgroups (see the kernel) for GQA in the default launch
-  // order; the other launch variants keep one head per workgroup, so the
-  // parity tests compare both mappings byte for byte.
+  // Head-grouped workgroups (see the kernel) for GQA in launch variants 0 and 3;
+  // variants 1 and 2 keep one head per workgroup, so that the parity tests compare
+  // both mappings byte for byte.
   const int G = H / Hkv;
   const int hg = (NWQ > 1 && G % NWQ == 0 && order == 0) ? 1 : 0;
   const long nu = hg ? nqt : nchunk, bu = hg ? (long)B * Hkv * (G / NWQ) : (long)B * H;
@@ -603,9 +603,9 @@ static hipError_t launch_fwd_t(const void* q, const void* k, const void* v, void
 
 // Whether a forward takes attn_fwd_tile_kernel and with how many 16-query tiles
 // per workgroup (0: the one-wave-per-block kernel); every choice gives the same
-// bits.  nb: the query blocks of all heads.  In the default launch the tile
-// kernel serves up to four blocks per CU under a full causal mask and two under
-// a window, where the one-wave-per-block kernel has at most one wave per SIMD and
+// bits.  tile: whether the launch allows the tile kernel; nb: the query blocks of
+// all heads.  It serves up to four blocks per CU under a full causal mask and two
+// under a window, where the one-wave-per-block kernel has at most one wave per SIMD and
 // waits for the longest rows.  256 CUs, bf16, D 128: 16 heads x 1024 (nb 512)
 // 166 -> 76 us, int8-PV 134 -> 69; 16 x 2048 (nb 1024) 322 -> 226, int8-PV, four
 // heads a group, 255 -> 184; window 256, nb 512: 67 -> 39, int8-PV 59 -> 39.
@@ -617,9 +617,9 @@ static hipError_t launch_fwd_t(const void* q, const void* k, const void* v, void
 // 39).  binary32 always takes the tile kernel: it replaced a form with one wave
 // per block and per SIMD (4 heads x 256, D 64: 36 -> 14 us; 16 heads x 2 x 4096,
 // D 128: 1781 -> 1531).
-static int fwd_tile_rows16(int nwq, long nb, int window) {
+static int fwd_tile_rows16(bool tile, long nb, int window) {
   const long cus = otx_cu_count();
-  if (nwq != 4 || nb > (window > 0 ? 2 : 4) * cus) return 0;
+  if (!tile || nb > (window > 0 ? 2 : 4) * cus) return 0;
   return nb <= (window > 0 ? 1 : 2) * cus ? 1 : 2;
 }
 
@@ -629,15 +629,15 @@ hipError_t launch_fwd_tile_i8(int D, int n16, const void* q, const void* k, void
 
 template <int D>
 static hipError_t launch_fwd_i8_d(int nwq, const void* q, const void* k, const void* v, void* o, float* lse, int B,
-                                  int H, int Hkv, int S, int window, float sigma, int order, int8_t* qvt,
-                                  float* vstep, float* scache, hipStream_t st) {
+                                  int H, int Hkv, int S, int window, float sigma, int order, bool tile,
+                                  int8_t* qvt, float* vstep, float* scache, hipStream_t st) {
   const long nblk = (long)B * Hkv * (S / OTX_BLK);
   constexpr int BPW = 256 / D;
   hipLaunchKernelGGL((attn_quant_v_kernel<D>), dim3((unsigned)((nblk + BPW - 1) / BPW)), dim3(256), 0, st,
                      (const uint16_t*)v, qvt, vstep, nblk);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (const int n16 = fwd_tile_rows16(nwq, (long)(S / OTX_BLK) * B * H, window))
+  if (const int n16 = fwd_tile_rows16(tile, (long)(S / OTX_BLK) * B * H, window))
     return launch_fwd_tile_i8(D, n16, q, k, o, lse, B, H, Hkv, S, window, sigma, order, qvt, vstep, scache, st);
   switch (nwq) {
     case 4: return launch_fwd_t<D, 4, true>(q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, st, qvt, vstep, scache);
@@ -648,11 +648,11 @@ static hipError_t launch_fwd_i8_d(int nwq, const void* q, const void* k, const v
 
 // int8-PV forward (bf16 inputs): quantizes V into qvt / vstep, then runs the forward.
 hipError_t launch_fwd_int8pv(int D, int nwq, const void* q, const void* k, const void* v, void* o, float* lse, int B,
-                             int H, int Hkv, int S, int window, float sigma, int order, int8_t* qvt, float* vstep,
-                             float* scache, hipStream_t st) {
+                             int H, int Hkv, int S, int window, float sigma, int order, bool tile, int8_t* qvt,
+                             float* vstep, float* scache, hipStream_t st) {
   if (D == 128)
-    return launch_fwd_i8_d<128>(nwq, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, qvt, vstep, scache, st);
-  return launch_fwd_i8_d<64>(nwq, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, qvt, vstep, scache, st);
+    return launch_fwd_i8_d<128>(nwq, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, tile, qvt, vstep, scache, st);
+  return launch_fwd_i8_d<64>(nwq, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, tile, qvt, vstep, scache, st);
 }
 
 template <int D>
@@ -672,12 +672,12 @@ hipError_t launch_fwd_tile(int dtype, int D, int n16, const void* q, const void*
 
 // scache (bf16 only, may be null): also write the score cache.
 hipError_t launch_fwd(int dtype, int D, int nwq, const void* q, const void* k, const void* v, void* o, float* lse,
-                      int B, int H, int Hkv, int S, int window, float sigma, int order, float* scache,
+                      int B, int H, int Hkv, int S, int window, float sigma, int order, bool tile, float* scache,
                       hipStream_t st) {
   const long nb = (long)(S / OTX_BLK) * B * H;
   const bool bf16 = dtype == 1;
   if (!bf16 && scache != nullptr) return hipErrorInvalidValue;  // the score cache is a bf16-path feature
-  int n16 = fwd_tile_rows16(nwq, nb, window);
+  int n16 = fwd_tile_rows16(tile, nb, window);
   if (!bf16 && n16 == 0) n16 = nwq == 1 ? 1 : 2;  // binary32 has no other form
   if (n16)
     return launch_fwd_tile(dtype, D, n16, q, k, v, o, lse, B, H, Hkv, S, window, sigma, order, scache, st);

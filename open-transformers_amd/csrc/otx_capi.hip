@@ -14,15 +14,15 @@
 
 namespace otx {
 hipError_t launch_fwd(int dtype, int D, int nwq, const void* q, const void* k, const void* v, void* o, float* lse,
-                      int B, int H, int Hkv, int S, int window, float sigma, int order, float* scache,
+                      int B, int H, int Hkv, int S, int window, float sigma, int order, bool tile, float* scache,
                       hipStream_t st);
 hipError_t launch_fwd_int8pv(int D, int nwq, const void* q, const void* k, const void* v, void* o, float* lse, int B,
-                             int H, int Hkv, int S, int window, float sigma, int order, int8_t* qvt, float* vstep,
-                             float* scache, hipStream_t st);
+                             int H, int Hkv, int S, int window, float sigma, int order, bool tile, int8_t* qvt,
+                             float* vstep, float* scache, hipStream_t st);
 hipError_t launch_bwd(int dtype, int D, int nw, const void* q, const void* k, const void* v, const void* o,
                       const float* lse, const void* dO, void* dq, void* dk, void* dv, float* dsum, float* ds, int B,
-                      int H, int Hkv, int S, int window, float sigma, int order, int stages, const float* scache,
-                      hipStream_t st);
+                      int H, int Hkv, int S, int window, float sigma, int order, bool tile, int stages,
+                      const float* scache, hipStream_t st);
 hipError_t launch_gemm(const void* A, long a_i, long a_r, const void* B, long b_j, long b_r, void* C, long ldc, int M,
                        int N, int R, bool out_f32, int variant, hipStream_t st);
 hipError_t launch_rmsnorm_fwd(int dtype, const void* x, const void* w, void* y, float* rstd, long rows, int D,
@@ -69,11 +69,14 @@ static int check_shape(int B, int H, int Hkv, int S, int D, int window, int dtyp
   return OTX_OK;
 }
 
-static void launch_variant(int variant, int* nw, int* order) {
+// Waves per workgroup, grid order, and whether the tile kernels (attn_tile.hip) may be chosen.
+static void launch_variant(int variant, int* nw, int* order, bool* tile) {
+  *tile = false;
   switch (variant) {
     case 1: *nw = 2; *order = 1; break;
     case 2: *nw = 1; *order = 0; break;
-    default: *nw = 4; *order = 0; break;
+    case 3: *nw = 4; *order = 0; break;
+    default: *nw = 4; *order = 0; *tile = true; break;
   }
 }
 
@@ -101,9 +104,10 @@ int otx_attn_fwd_ex(const void* q, const void* k, const void* v, void* o, float*
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
     return fail(OTX_EINVAL, "q, k, v and o must be 16-byte aligned");
   int nw, order;
-  launch_variant(variant, &nw, &order);
+  bool tile;
+  launch_variant(variant, &nw, &order, &tile);
   hipError_t e = otx::launch_fwd(dtype, D, nw, q, k, v, o, lse, B, H, Hkv, S, window, otx_softmax_scale(D), order,
-                                 nullptr, (hipStream_t)stream);
+                                 tile, nullptr, (hipStream_t)stream);
   if (e != hipSuccess) return fail(OTX_EHIP, "forward launch failed: %s", hipGetErrorString(e));
   return OTX_OK;
 }
@@ -137,9 +141,10 @@ int otx_attn_fwd_int8pv_ex(const void* q, const void* k, const void* v, void* o,
   int8_t* qvt = (int8_t*)workspace;
   float* vstep = (float*)((char*)workspace + int8pv_qv_bytes(B, Hkv, S, D));
   int nw, order;
-  launch_variant(variant, &nw, &order);
+  bool tile;
+  launch_variant(variant, &nw, &order, &tile);
   hipError_t e = otx::launch_fwd_int8pv(D, nw, q, k, v, o, lse, B, H, Hkv, S, window, otx_softmax_scale(D), order,
-                                        qvt, vstep, nullptr, (hipStream_t)stream);
+                                        tile, qvt, vstep, nullptr, (hipStream_t)stream);
   if (e != hipSuccess) return fail(OTX_EHIP, "int8-PV forward launch failed: %s", hipGetErrorString(e));
   return OTX_OK;
 }
@@ -208,9 +213,10 @@ int otx_attn_fwd_int8pv_noalloc(const void* q, const void* k, const void* v, voi
   int8_t* qvt = (int8_t*)base;
   float* vstep = (float*)((char*)base + int8pv_qv_bytes(B, Hkv, S, D));
   int nw, order;
-  launch_variant(variant, &nw, &order);
+  bool tile;
+  launch_variant(variant, &nw, &order, &tile);
   hipError_t e = otx::launch_fwd_int8pv(D, nw, q, k, v, o, lse, B, H, Hkv, S, window, otx_softmax_scale(D), order,
-                                        qvt, vstep, nullptr, (hipStream_t)stream);
+                                        tile, qvt, vstep, nullptr, (hipStream_t)stream);
   if (e != hipSuccess) return fail(OTX_EHIP, "int8-PV forward launch failed: %s", hipGetErrorString(e));
   return OTX_OK;
 }
@@ -233,9 +239,10 @@ int otx_attn_bwd_stages(const void* q, const void* k, const void* v, const void*
   float* dsum = (float*)workspace;
   float* ds = (float*)((char*)workspace + ((rows * sizeof(float) + 255) / 256) * 256);
   int nw, order;
-  launch_variant(variant, &nw, &order);
+  bool tile;
+  launch_variant(variant, &nw, &order, &tile);
   hipError_t e = otx::launch_bwd(dtype, D, nw, q, k, v, o, lse, dout, dq, dk, dv, dsum, ds, B, H, Hkv, S, window,
-                                 otx_softmax_scale(D), order, stages, nullptr, (hipStream_t)stream);
+                                 otx_softmax_scale(D), order, tile, stages, nullptr, (hipStream_t)stream);
   if (e != hipSuccess) return fail(OTX_EHIP, "backward launch failed: %s", hipGetErrorString(e));
   return OTX_OK;
 }
@@ -281,9 +288,10 @@ int otx_attn_fwd_sc(const void* q, const void* k, const void* v, void* o, float*
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
     return fail(OTX_EINVAL, "q, k, v and o must be 16-byte aligned");
   int nw, order;
-  launch_variant(variant, &nw, &order);
+  bool tile;
+  launch_variant(variant, &nw, &order, &tile);
   hipError_t e = otx::launch_fwd(dtype, D, nw, q, k, v, o, lse, B, H, Hkv, S, window, otx_softmax_scale(D), order,
-                                 scache, (hipStream_t)stream);
+                                 tile, scache, (hipStream_t)stream);
   if (e != hipSuccess) return fail(OTX_EHIP, "forward launch failed: %s", hipGetErrorString(e));
   return OTX_OK;
 }
@@ -303,9 +311,10 @@ int otx_attn_fwd_int8pv_sc(const void* q, const void* k, const void* v, void* o,
   int8_t* qvt = (int8_t*)workspace;
   float* vstep = (float*)((char*)workspace + int8pv_qv_bytes(B, Hkv, S, D));
   int nw, order;
-  launch_variant(variant, &nw, &order);
+  bool tile;
+  launch_variant(variant, &nw, &order, &tile);
   hipError_t e = otx::launch_fwd_int8pv(D, nw, q, k, v, o, lse, B, H, Hkv, S, window, otx_softmax_scale(D), order,
-                                        qvt, vstep, scache, (hipStream_t)stream);
+                                        tile, qvt, vstep, scache, (hipStream_t)stream);
   if (e != hipSuccess) return fail(OTX_EHIP, "int8-PV forward launch failed: %s", hipGetErrorString(e));
   return OTX_OK;
 }
@@ -330,9 +339,10 @@ int otx_attn_bwd_sc(const void* q, const void* k, const void* v, const void* o, 
   float* dsum = (float*)workspace;
   float* ds = (float*)((char*)workspace + ((rows * sizeof(float) + 255) / 256) * 256);
   int nw, order;
-  launch_variant(variant, &nw, &order);
+  bool tile;
+  launch_variant(variant, &nw, &order, &tile);
   hipError_t e = otx::launch_bwd(dtype, D, nw, q, k, v, o, lse, dout, dq, dk, dv, dsum, ds, B, H, Hkv, S, window,
-                                 otx_softmax_scale(D), order, stages, scache, (hipStream_t)stream);
+                                 otx_softmax_scale(D), order, tile, stages, scache, (hipStream_t)stream);
   if (e != hipSuccess) return fail(OTX_EHIP, "backward launch failed: %s", hipGetErrorString(e));
   return OTX_OK;
 }

@@ -39,9 +39,6 @@ __device__ __forceinline__ f32x32 otx_mfma_bhalf(float a, float b, f32x32 c) {
 // of block L/16, row L%16 and B of block L/16, column L%16; result register r
 // (0..15) of lane L holds block r/4, row 4*(L/16) + r%4, column L%16.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ f32x16 otx_mfma16(float a, float b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
-}
 
 // (x, y) <- (x.lo | y.lo, x.hi | y.hi)   [lo = lanes 0..31, hi = lanes 32..63]
 __device__ __forceinline__ void otx_swap_halves(float& x, float& y) {

@@ -110,8 +110,8 @@ def _check_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window: int
 def flash_attention_forward(
     q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window: int = 0, variant: int = 0
 ) -> tuple[torch.Tensor, torch.Tensor]:
-    """Forward pass returning (O, LSE).  ``variant`` selects a launch shape
-    (0 default, 1, 2); all variants give identical bits."""
+    """Forward pass returning (O, LSE).  ``variant`` selects a launch shape (0 default,
+    1, 2, 3; see otx_attn_fwd_ex in include/otx_attn.h); all variants give identical bits."""
     B, H, Hkv, S, D = _check_inputs(q, k, v, window)
     o = torch.empty_like(q)
     lse = torch.empty((B, H, S), dtype=torch.float32, device=q.device)

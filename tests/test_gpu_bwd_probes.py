@@ -1,8 +1,9 @@
 """The backward's closed-form probes (tests/bwd_probes.py) on the GPU.
 
 Each probe runs through the C ABI with bf16 and binary32 inputs, in launch
-variants 0 and 2 (for bf16 these take the two dK/dV kernel forms), with and
-without the score cache (bf16).  The closed-form bits must hold, dS_00 read
+variants 0, 2 and 3 (for bf16 these take the tile kernels, the four-key-block
+dK/dV and, with the score cache, the two-key-block dK/dV that large grids
+launch), with and without the score cache (bf16).  The closed-form bits must hold, dS_00 read
 back from the backward workspace must equal the contract's, and every output
 byte must equal the oracle's.
 """
@@ -63,7 +64,7 @@ def test_backward_probes_on_gpu(bf16):
     for name, p, check in bp.all_probes(bf16):
         ref = dict(zip(("dq", "dk", "dv"),
                        orc.attn_bwd(p["q"], p["k"], p["v"], p["o"], p["lse"], p["do"], window=0, out_bf16=bf16)))
-        for variant in (0, 2):
+        for variant in (0, 2, 3):
             for sc in ((False, True) if bf16 else (False,)):
                 print(f"probe {name} {'bf16' if bf16 else 'binary32'} variant {variant} score cache {sc}", flush=True)
                 got = _gpu_bwd(p, bf16, variant, sc)
@@ -79,7 +80,7 @@ def test_backward_with_lse_below_the_scores(bf16):
     otx_expf instead of the table-driven path, and every output byte must still
     equal the oracle's for the same LSE.  Every third query row has its LSE
     lowered by 2 (arguments up to about +2), the others keep the forward's; GQA
-    (H 4, Hkv 2), both dK/dV forms (variants 0 and 2), score cache on and off."""
+    (H 4, Hkv 2), every dK/dV form (variants 0, 2 and 3), score cache on and off."""
     rng = np.random.default_rng(7)
     B, H, Hkv, S, D = 1, 4, 2, 128, 128
 
@@ -96,7 +97,7 @@ def test_backward_with_lse_below_the_scores(bf16):
     p["lse"] = lse
     ref = dict(zip(("dq", "dk", "dv"),
                    orc.attn_bwd(p["q"], p["k"], p["v"], p["o"], p["lse"], p["do"], window=0, out_bf16=bf16)))
-    for variant in (0, 2):
+    for variant in (0, 2, 3):
         for sc in ((False, True) if bf16 else (False,)):
             print(f"lowered LSE {'bf16' if bf16 else 'binary32'} variant {variant} score cache {sc}", flush=True)
             got = _gpu_bwd(p, bf16, variant, sc)

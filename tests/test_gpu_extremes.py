@@ -77,14 +77,17 @@ def test_extreme_inputs_match_oracle(case):
         inp[nm] = synthetic.round_to_bf16(x) if bf16 else x
     with np.errstate(all="ignore"):
         ref = oracle_fwd_bwd(inp, window, bf16)
-    got = gpu_fwd_bwd(inp, window, bf16, variant=c["variant"], score_cache=bf16 and c["cache"])
-    for nm in ("o", "lse", "dq", "dk", "dv"):
-        eq(got[nm], ref[nm], nm)
+    variants = (c["variant"], 3) if bf16 else (c["variant"],)
+    for variant in variants:
+        got = gpu_fwd_bwd(inp, window, bf16, variant=variant, score_cache=bf16 and c["cache"])
+        for nm in ("o", "lse", "dq", "dk", "dv"):
+            eq(got[nm], ref[nm], f"{nm} (variant {variant})")
     if bf16 and c["D"] == 128 and c["int8"]:
         with np.errstate(all="ignore"):
             ro, rl = orc.attn_fwd_int8pv(inp["q"], inp["k"], inp["v"], window=window)
         t = {nm: torch.from_numpy(inp[nm]).to(torch.bfloat16).cuda() for nm in ("q", "k", "v")}
-        o8, l8 = fa.int8pv_flash_attention_forward(t["q"], t["k"], t["v"], window=window, variant=c["variant"])
-        torch.cuda.synchronize()
-        eq(o8.float().cpu().numpy(), ro, "int8-PV O")
-        eq(l8.cpu().numpy(), rl, "int8-PV LSE")
+        for variant in variants:
+            o8, l8 = fa.int8pv_flash_attention_forward(t["q"], t["k"], t["v"], window=window, variant=variant)
+            torch.cuda.synchronize()
+            eq(o8.float().cpu().numpy(), ro, f"int8-PV O (variant {variant})")
+            eq(l8.cpu().numpy(), rl, f"int8-PV LSE (variant {variant})")

@@ -1,7 +1,7 @@
 """The forward's closed-form probes (tests/fwd_probes.py) on the GPU.
 
 Each probe runs through the C ABI at D 64 and 128 with bf16 and binary32
-inputs, in launch variants 0 and 2, with and without the score cache (bf16).
+inputs, in launch variants 0, 2 and 3, with and without the score cache (bf16).
 The probed row's LSE and O columns must equal the contract's hand-derived
 bits (the deviations' bits differ, as the CPU pins show), and every O and LSE
 byte must equal the oracle's.  The int8-PV forward runs the same probes: its
@@ -46,7 +46,7 @@ def _gpu_fwd(p, window, bf16, variant, score_cache, int8pv=False):
 def test_forward_probes_on_gpu(D, bf16):
     for name, p, window in fp.all_probes(D):
         ro, rlse = orc.attn_fwd(p["q"], p["k"], p["v"], window=window, out_bf16=bf16)
-        for variant in (0, 2):
+        for variant in (0, 2, 3):
             for sc in ((False, True) if bf16 else (False,)):
                 print(f"forward probe {name} D={D} {'bf16' if bf16 else 'binary32'} variant {variant} "
                       f"score cache {sc}", flush=True)
@@ -62,7 +62,7 @@ def test_forward_probes_int8pv_lse(D):
         _, rlse = orc.attn_fwd(p["q"], p["k"], p["v"], window=window, out_bf16=True)
         ro8, rlse8 = orc.attn_fwd_int8pv(p["q"], p["k"], p["v"], window=window, out_bf16=True)
         assert_bits_equal(rlse8, rlse, f"probe {name}: oracle int8-PV LSE vs binary32 LSE")
-        for variant in (0, 2):
+        for variant in (0, 2, 3):
             for sc in (False, True):
                 print(f"int8-PV forward probe {name} D={D} variant {variant} score cache {sc}", flush=True)
                 got = _gpu_fwd(p, window, True, variant, sc, int8pv=True)

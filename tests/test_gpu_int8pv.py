@@ -80,7 +80,7 @@ def test_int8pv_fwd_bwd_bitexact(B, H, Hkv, S, D, window, seed):
     inp = make(B, H, Hkv, S, D, seed=seed)
     ro, rl = orc.attn_fwd_int8pv(inp["q"], inp["k"], inp["v"], window=window)
     q, k, v = (_gpu(inp[n]) for n in ("q", "k", "v"))
-    for variant in (0, 1, 2):
+    for variant in (0, 1, 2, 3):
         o, lse = fa.int8pv_flash_attention_forward(q, k, v, window=window, variant=variant)
         torch.cuda.synchronize()
         assert_bits_equal(_host(o), ro, f"O (variant {variant})")
@@ -88,7 +88,7 @@ def test_int8pv_fwd_bwd_bitexact(B, H, Hkv, S, D, window, seed):
     _, lse32 = fa.flash_attention_forward(q, k, v, window=window)
     assert_bits_equal(_host(lse32), rl, "LSE of the binary32 forward")
     # the score cache of the int8-PV forward is the binary32 forward's (same scores)
-    for variant in (0, 1, 2):
+    for variant in (0, 1, 2, 3):
         o8, l8, sc8 = fa.int8pv_flash_attention_forward_sc(q, k, v, window=window, variant=variant)
         _, _, sc32 = fa.flash_attention_forward_sc(q, k, v, window=window, variant=variant)
         torch.cuda.synchronize()
@@ -117,7 +117,7 @@ def test_int8pv_subnormal_outputs():
     ro, rl = orc.attn_fwd_int8pv(inp["q"], inp["k"], inp["v"], window=0)
     assert (np.abs(ro) < np.float32(2.0 ** -126)).mean() > 0.9
     q, k, v = (_gpu(inp[n]) for n in ("q", "k", "v"))
-    for variant in (0, 1, 2):
+    for variant in (0, 1, 2, 3):
         o, lse = fa.int8pv_flash_attention_forward(q, k, v, window=0, variant=variant)
         torch.cuda.synchronize()
         assert_bits_equal(_host(o), ro, f"O (variant {variant})")
@@ -147,7 +147,7 @@ def test_int8pv_tiny_block_maxima():
     assert tiny > 50
     ro, rl = orc.attn_fwd_int8pv(inp["q"], inp["k"], inp["v"], window=0)
     q, k, v = (_gpu(inp[n]) for n in ("q", "k", "v"))
-    for variant in (0, 1, 2):
+    for variant in (0, 1, 2, 3):
         o, lse = fa.int8pv_flash_attention_forward(q, k, v, window=0, variant=variant)
         torch.cuda.synchronize()
         assert_bits_equal(_host(o), ro, f"O (variant {variant})")
@@ -164,10 +164,11 @@ def test_int8pv_nan_in_k():
     ro, rl = orc.attn_fwd_int8pv(inp["q"], inp["k"], inp["v"], window=0)
     assert np.isnan(rl).sum() == 88
     q, k, v = (_gpu(inp[n]) for n in ("q", "k", "v"))
-    o, lse = fa.int8pv_flash_attention_forward(q, k, v, window=0)
-    torch.cuda.synchronize()
-    assert_bits_equal_nan_class(_host(o), ro, "O")
-    assert_bits_equal_nan_class(_host(lse), rl, "LSE")
+    for variant in (0, 2, 3):
+        o, lse = fa.int8pv_flash_attention_forward(q, k, v, window=0, variant=variant)
+        torch.cuda.synchronize()
+        assert_bits_equal_nan_class(_host(o), ro, f"O (variant {variant})")
+        assert_bits_equal_nan_class(_host(lse), rl, f"LSE (variant {variant})")
 
 
 def test_int8pv_open1b_shape_all_heads():

@@ -64,7 +64,8 @@ def test_c4_batch_and_launch_invariance():
     base = {}
     for B in (1, 2, 8, 16):
         inp = make(B, 16, 16, 1024, 128, dtype="bf16", seed=44)
-        for variant, sc in (((0, False), (1, False), (2, False), (0, True), (1, True), (2, True)) if B in (1, 16)
+        for variant, sc in (((0, False), (1, False), (2, False), (3, False), (0, True), (1, True), (2, True),
+                             (3, True)) if B in (1, 16)
                             else ((0, False), (0, True))):
             got = gpu_fwd_bwd(inp, 0, True, variant=variant, score_cache=sc)
             for n in NAMES:

@@ -3,7 +3,7 @@ the GPU, through the C ABI.
 
 RMSNorm forward / backward and SiLU forward / backward run with bf16 and with
 binary32 data (the binary32 outputs show the deviations that bf16 rounds
-away); the int8-PV forward runs at D 64 and 128 in launch variants 0 and 2,
+away); the int8-PV forward runs at D 64 and 128 in launch variants 0, 2 and 3,
 with and without the score cache.  The probed elements must hold the
 contract's hand-derived bits, and every output byte must equal the oracle's.
 """
@@ -106,7 +106,7 @@ def test_int8pv_probes(D):
     for name, p in lp.int8pv_probes(D):
         ro, rlse = orc.attn_fwd_int8pv(p["q"], p["k"], p["v"], window=p["_window"], out_bf16=True)
         q, k, v = (_gpu(p[n], True) for n in ("q", "k", "v"))
-        for variant in (0, 2):
+        for variant in (0, 2, 3):
             for sc in (False, True):
                 print(f"int8-PV probe {name} D={D} variant {variant} score cache {sc}", flush=True)
                 f = fa.int8pv_flash_attention_forward_sc if sc else fa.int8pv_flash_attention_forward

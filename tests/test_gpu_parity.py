@@ -39,7 +39,7 @@ def test_fwd_bwd_bitexact(B, H, Hkv, S, D, window, dtype, seed, qk_scale):
     inp = make(B, H, Hkv, S, D, dtype=dtype, seed=seed, qk_scale=qk_scale)
     bf16 = dtype == "bf16"
     ref = oracle_fwd_bwd(inp, window, bf16)
-    for variant in (0, 1, 2):
+    for variant in (0, 1, 2, 3):
         for sc in ((False, True) if bf16 else (False,)):
             got = gpu_fwd_bwd(inp, window, bf16, variant=variant, score_cache=sc)
             for name in ("o", "lse", "dq", "dk", "dv"):
@@ -66,11 +66,11 @@ def test_long_sequence_bitexact(S, window):
     """Long sequences with a GQA group of four (the head-grouped forward and dQ
     workgroups): tile indices, score-cache and dS-tile addresses and the 32-bit
     lane offsets at 16K (full causal, 131,328 tiles per head) and 32K tokens
-    (window 512), launch variants 0 and 2, score cache off and on."""
+    (window 512), launch variants 0, 2 and 3, score cache off and on."""
     print(f"long sequence S={S} window={window}", flush=True)
     inp = make(1, 4, 1, S, 128, dtype="bf16", seed=21 + window)
     ref = oracle_fwd_bwd(inp, window, True)
-    for variant in (0, 2):
+    for variant in (0, 2, 3):
         for sc in (False, True):
             got = gpu_fwd_bwd(inp, window, True, variant=variant, score_cache=sc)
             for name in ("o", "lse", "dq", "dk", "dv"):
@@ -90,7 +90,7 @@ def test_subnormal_outputs_bitexact():
     ref = oracle_fwd_bwd(inp, 0, True)
     tiny = np.abs(ref["o"]) < np.float32(2.0 ** -126)
     assert tiny.mean() > 0.9, "the case must put the outputs below the normal range"
-    for variant in (0, 1, 2):
+    for variant in (0, 1, 2, 3):
         for sc in (False, True):
             got = gpu_fwd_bwd(inp, 0, True, variant=variant, score_cache=sc)
             for name in ("o", "lse", "dq", "dk", "dv"):
@@ -117,10 +117,11 @@ def test_nonfinite_inputs_propagate_like_the_oracle(what, val, dtype):
     bf16 = dtype == "bf16"
     ref = oracle_fwd_bwd(inp, 0, bf16)
     assert np.isnan(ref["o"]).any() or np.isnan(ref["dq"]).any()
-    for sc in ((False, True) if bf16 else (False,)):
-        got = gpu_fwd_bwd(inp, 0, bf16, score_cache=sc)
-        for name in ("o", "lse", "dq", "dk", "dv"):
-            assert_bits_equal_nan_class(got[name], ref[name], f"{name} (score cache {sc})")
+    for variant in ((0, 2, 3) if bf16 else (0,)):
+        for sc in ((False, True) if bf16 else (False,)):
+            got = gpu_fwd_bwd(inp, 0, bf16, variant=variant, score_cache=sc)
+            for name in ("o", "lse", "dq", "dk", "dv"):
+                assert_bits_equal_nan_class(got[name], ref[name], f"{name} (variant {variant}, score cache {sc})")
 
 
 def test_overflowing_accumulation_and_wide_windows():
@@ -131,14 +132,33 @@ def test_overflowing_accumulation_and_wide_windows():
     inp = make(1, 2, 2, 128, 128, dtype="bf16", seed=32)
     for w in (128, 160, 512):
         ref = oracle_fwd_bwd(inp, w, True)
-        for sc in (False, True):
-            got = gpu_fwd_bwd(inp, w, True, score_cache=sc)
+        for variant, sc in ((0, False), (0, True), (3, False), (3, True)):
+            got = gpu_fwd_bwd(inp, w, True, variant=variant, score_cache=sc)
             for name in ("o", "lse", "dq", "dk", "dv"):
-                assert_bits_equal(got[name], ref[name], f"{name} (window {w}, score cache {sc})")
+                assert_bits_equal(got[name], ref[name], f"{name} (window {w}, variant {variant}, score cache {sc})")
     inp["v"] = synthetic.round_to_bf16(np.sign(inp["v"]) * np.float32(3.0e38))
     ref = oracle_fwd_bwd(inp, 0, True)
-    for sc in (False, True):
-        got = gpu_fwd_bwd(inp, 0, True, score_cache=sc)
+    for variant, sc in ((0, False), (0, True), (3, False), (3, True)):
+        got = gpu_fwd_bwd(inp, 0, True, variant=variant, score_cache=sc)
         for name in ("o", "lse", "dq", "dk", "dv"):
-            assert_bits_equal_nan_class(got[name], ref[name], f"{name} (V +-3e38, score cache {sc})")
+            assert_bits_equal_nan_class(got[name], ref[name], f"{name} (V +-3e38, variant {variant}, score cache {sc})")
+
+
+@pytest.mark.parametrize("window", [0, 512])
+def test_nonfinite_inputs_on_the_kernels_of_large_grids(window):
+    """Non-finite elements in a grid of 4096 query blocks (four heads a group, the score cache and no cache), where the
+    default launch takes the one-wave-per-block kernels with head-grouped and paired workgroups: byte for byte, and NaN
+    for NaN, what variant 2 gives, whose kernels the cases above compare with the oracle."""
+    print(f"non-finite on large grids, window {window}", flush=True)
+    inp = make(4, 16, 4, 2048, 128, dtype="bf16", seed=33)
+    inp["q"][0, 3, 700, 5], inp["q"][2, 8, 2047, 0] = np.nan, np.inf
+    inp["k"][1, 1, 900, 7], inp["k"][3, 2, 31, 127] = np.nan, -np.inf
+    inp["v"][1, 3, 1300, 64], inp["v"][2, 0, 3, 1] = np.inf, np.nan
+    inp["do"][0, 15, 1000, 9], inp["do"][3, 0, 2000, 3] = -np.inf, np.nan
+    for sc in (False, True):
+        ref = gpu_fwd_bwd(inp, window, True, variant=2, score_cache=sc)
+        got = gpu_fwd_bwd(inp, window, True, score_cache=sc)
+        for name in ("o", "lse", "dq", "dk", "dv"):
+            assert np.isnan(ref[name]).any() and np.isfinite(ref[name]).any()
+            assert_bits_equal_nan_class(got[name], ref[name], f"{name} (window {window}, score cache {sc})")
 

@@ -21,11 +21,15 @@ REPS = 120
 
 CASES = [
     # B, H, Hkv, S, D, window, seed, variant, score cache
-    pytest.param(1, 2, 2, 128, 64, 0, 6, 0, False, id="d64-two-kb"),
+    pytest.param(1, 2, 2, 128, 64, 0, 6, 0, False, id="d64-tile"),
     pytest.param(1, 2, 2, 128, 64, 0, 6, 2, False, id="d64-four-kb"),
-    pytest.param(1, 2, 2, 128, 64, 0, 6, 0, True, id="d64-two-kb-cache"),
-    pytest.param(1, 2, 2, 128, 128, 0, 2, 0, False, id="d128-two-kb"),
-    pytest.param(2, 4, 2, 160, 128, 64, 3, 0, True, id="gqa-win64-cache"),
+    pytest.param(1, 2, 2, 128, 64, 0, 6, 0, True, id="d64-tile-cache"),
+    pytest.param(1, 2, 2, 128, 128, 0, 2, 0, False, id="d128-tile"),
+    pytest.param(2, 4, 2, 160, 128, 64, 3, 0, True, id="gqa-win64-tile-cache"),
+    pytest.param(1, 2, 2, 128, 64, 0, 6, 3, True, id="d64-two-kb-cache"),
+    pytest.param(1, 2, 2, 128, 128, 0, 2, 3, True, id="d128-two-kb-cache"),
+    pytest.param(1, 2, 2, 128, 128, 0, 2, 3, False, id="d128-four-kb"),
+    pytest.param(2, 8, 2, 160, 128, 64, 3, 3, True, id="gqa4-win64-two-kb-cache"),
     pytest.param(1, 4, 1, 96, 64, 32, 4, 1, False, id="mqa-win32-two-waves"),
 ]
 
