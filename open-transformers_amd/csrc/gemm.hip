@@ -16,8 +16,8 @@
 //
 // Tiling: a workgroup of 4 waves owns a 128 x 128 block of C, each wave a
 // 64 x 64 quarter (two MFMAs per r: i-blocks {0,1} x j-block 0, then x
-// j-block 1), or, in the narrow form, a 128 x 64 block with 64 x 32 per wave
-// (one MFMA per r), or, in the small forms, a 64 x 64 or 32 x 32 block with
+// j-block 1), or, in the narrow form (both operands i-contiguous), a 128 x 64 block
+// with 64 x 32 per wave (one MFMA per r), or, in the small forms, a 64 x 64 or 32 x 32 block with
 // 32 x 32 or 16 x 16 per wave, on v_mfma_f32_16x16x4_f32 (four serial fmas per
 // output; see there).  The wide and narrow forms (gemm_bf16_v2_kernel)
 // advance r in chunks of 32 kept in LDS as bf16 in two slots, one barrier per chunk:
@@ -458,7 +458,8 @@ static hipError_t launch_gemm_t(const void* A, long a_i, long a_r, const void* B
                                 long ldc, int M, int N, int R, bool out_f32, int form, hipStream_t st) {
   if (form == 3) return launch_gemm_k4<ARC, BRC, 1>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
   if (form == 2) return launch_gemm_k4<ARC, BRC, 2>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
-  if (form == 1) return launch_gemm_w<ARC, BRC, 32>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
+  if constexpr (!ARC && !BRC)
+    if (form == 1) return launch_gemm_w<ARC, BRC, 32>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
   return launch_gemm_w<ARC, BRC, 64>(A, a_i, a_r, B, b_j, b_r, C, ldc, M, N, R, out_f32, st);
 }
 
@@ -469,7 +470,7 @@ static hipError_t launch_gemm_t(const void* A, long a_i, long a_r, const void* B
 // 4 us of launch taken off) is, for m = 1, 2 and more:
 //                        y = x w^T          dx = dy w          dw = dy^T x
 //   wide               1.24 1.17 1.12     1.19 1.14 1.10     1.09 1.10 1.085
-//   narrow             1.43 1.26 1.16     1.40 1.27 1.18     1.19 1.11 1.10
+//   narrow            (1.43 1.26 1.16)   (1.40 1.27 1.18)    1.19 1.11 1.10
 //   64 x 64            1.25 1.17 1.15     1.25 1.17 1.18     1.25 1.17 1.18
 //   32 x 32            1.41 throughout
 // (few waves per SIMD expose a wide tile's waits; an r-contiguous operand costs the wide and
@@ -478,20 +479,23 @@ static hipError_t launch_gemm_t(const void* A, long a_i, long a_r, const void* B
 // tiles; 1024 x 1024 over 1024 27 -> 21 us and 1280 x 5632 over 2048 267 -> 229 us, 64 x 64;
 // 8192 x 11264 over 2048 stays with the wide form's 2.71 ms.  The narrow form is left to
 // products with both operands i-contiguous (11264 x 2048 over 8192, 5.5 wide tiles per CU:
-// 2.66 ms against 2.84 and 2.86); elsewhere the 64 x 64 form is as fast or faster.
-// variant 1, 2 and 3 force the wide, the narrow and the 64 x 64 form.
+// 2.66 ms against 2.84 and 2.86); elsewhere the 64 x 64 form was as fast or faster (the figures
+// in brackets), and the narrow form is not built.
+// variant 1, 2, 3 and 4 force the wide, the narrow (where it exists), the 64 x 64 and the
+// 32 x 32 form.
 static int gemm_form(int M, int N, bool arc, bool brc, int variant) {
-  if (variant >= 1) return variant - 1;
-  const long t = (long)(M / GT) * (N / GT), n = otx_cu_count();
   const int lay = arc && brc ? 0 : arc || brc ? 1 : 2;
-  static const long over[3][3][3] = {{{1240, 1170, 1120}, {1190, 1140, 1100}, {1090, 1100, 1085}},
-                                     {{1430, 1260, 1160}, {1400, 1270, 1180}, {1190, 1110, 1100}},
-                                     {{1250, 1170, 1150}, {1250, 1170, 1180}, {1250, 1170, 1180}}};
+  if (variant >= 1 && (variant != 2 || lay == 2)) return variant - 1;
+  const long t = (long)(M / GT) * (N / GT), n = otx_cu_count();
+  static const long wide[3][3] = {{1240, 1170, 1120}, {1190, 1140, 1100}, {1090, 1100, 1085}};
+  static const long narrow[3] = {1190, 1110, 1100};
+  static const long small[3][3] = {{1250, 1170, 1150}, {1250, 1170, 1180}, {1250, 1170, 1180}};
   long best = 1410 * ((16 * t + n - 1) / n);  // in 1/16000 of a wide tile's matrix instructions
   int form = 3;
   for (int f = 2; f >= 0; f--) {
     if (f == 1 && lay != 2) continue;
-    const long m = ((t << f) + n - 1) / n, cost = m * (16 >> f) * over[f][lay][m < 3 ? m - 1 : 2];
+    const long* over = f == 2 ? small[lay] : f == 1 ? narrow : wide[lay];
+    const long m = ((t << f) + n - 1) / n, cost = m * (16 >> f) * over[m < 3 ? m - 1 : 2];
     if (cost <= best) {
       best = cost;
       form = f;

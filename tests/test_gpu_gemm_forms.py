@@ -1,5 +1,5 @@
-"""The small GEMM forms (v_mfma_f32_16x16x4_f32: four serial fmas per output and instruction) against the serial-fold
-oracle where they can go wrong: every remainder of R by the stage length of either form (64 and 128), one to more
+"""The GEMM forms (the small ones on v_mfma_f32_16x16x4_f32: four serial fmas per instruction) against the serial-fold
+oracle where they can go wrong: every remainder of R by the stage length of the small forms (64 and 128), one to more
 stages than the LDS slots, both operand layouts of each side, padded row pitches, and operands whose fold order and
 rounding show in every output (cancellations over 2^24, subnormals, signed zeros, infinities)."""
 
@@ -44,7 +44,7 @@ def _dev(a, r_contiguous, pad):
 @pytest.mark.parametrize("R", [32, 64, 96, 128, 160, 224, 352, 512, 544, 1120])
 @pytest.mark.parametrize("kind", ["cancel", "tiny", "inf"])
 def test_small_forms_match_the_serial_fold(R, kind):
-    print(f"gemm small forms R{R} {kind}", flush=True)
+    print(f"gemm forms R{R} {kind}", flush=True)
     rng = np.random.default_rng(R)
     a, b = _operand(rng, M, R, kind), _operand(rng, N, R, kind)
     with np.errstate(all="ignore"):
@@ -53,9 +53,26 @@ def test_small_forms_match_the_serial_fold(R, kind):
         for brc in (True, False):
             ta, sa = _dev(a, arc, 8)
             tb, sb = _dev(b, brc, 16)
-            for variant in (0, 3):
+            for variant in range(5):
                 y = F.gemm_bf16(ta, sa, tb, sb, M, N, R, variant=variant)
                 y32 = F.gemm_bf16(ta, sa, tb, sb, M, N, R, out_dtype=torch.float32, variant=variant)
                 torch.cuda.synchronize()
                 eq(y.float().cpu().numpy(), ref, f"bf16 result, layouts {arc} {brc}, variant {variant}")
                 eq(y32.cpu().numpy(), ref32, f"binary32 result, layouts {arc} {brc}, variant {variant}")
+
+
+@pytest.mark.parametrize("shape", [(128, 256, 512), (1024, 1024, 96), (1280, 5632, 64), (2048, 4096, 64)])
+def test_every_form_gives_the_chosen_ones_bytes(shape):
+    """Products of few to many tiles (the library's choice goes from 32 x 32 to the wide tiles), every forced form and
+    layout against the choice."""
+    m, n, r = shape
+    print(f"gemm forms {shape}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    a, b = (torch.randn(rows, r, device=DEV, generator=g).bfloat16() for rows in (m, n))
+    ref = F.gemm_bf16(a, (r, 1), b, (r, 1), m, n, r)
+    at, bt = a.t().contiguous(), b.t().contiguous()
+    for ta, sa in ((a, (r, 1)), (at, (1, m))):
+        for tb, sb in ((b, (r, 1)), (bt, (1, n))):
+            for variant in range(5):
+                y = F.gemm_bf16(ta, sa, tb, sb, m, n, r, variant=variant)
+                assert torch.equal(y.view(torch.int16), ref.view(torch.int16)), (sa, sb, variant)

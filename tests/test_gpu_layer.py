@@ -62,7 +62,7 @@ def test_gemm_three_forms(M, N, R):
     assert_bits_equal(host(dw), orc.gemm(dy.T, x.T), "dw = dy^T x")
 
 
-@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4])
 def test_gemm_padded_strides(variant):
     """Operands that are views into larger buffers: a row pitch past the logical
     width (still a multiple of 8 elements) and a start 8 elements into the buffer,

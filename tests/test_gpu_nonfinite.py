@@ -108,7 +108,7 @@ def test_gemm_nonfinite_and_overflowing_rows():
     a, b = bf(rng.standard_normal((M, R))), bf(rng.standard_normal((N, R)))
     a[3, 5], b[7, 9], a[10, :] = np.nan, np.inf, 3e38
     a, b = bf(a), bf(b)
-    for v in (0, 1, 2, 3):
+    for v in range(5):
         c = F.gemm_bf16(gpu(a), (R, 1), gpu(b), (R, 1), M, N, R, variant=v)
         torch.cuda.synchronize()
         eq(host(c), orc.gemm(a, b), f"gemm form {v}")
@@ -129,7 +129,7 @@ def test_gemm_step_whose_product_alone_overflows():
     a, b = bf(a), bf(b)
     ref = orc.gemm(a, b, out_bf16=False)
     assert np.isfinite(ref[0, 0]) and abs(float(a[0, 1]) * float(b[0, 1])) > 3.5e38  # the case is reached
-    for v in (1, 2, 3):
+    for v in (1, 2, 3, 4):
         c = F.gemm_bf16(gpu(a), (R, 1), gpu(b), (R, 1), M, N, R, out_dtype=torch.float32, variant=v)
         torch.cuda.synchronize()
         assert_bits_equal(host(c), ref, f"form {v}")
