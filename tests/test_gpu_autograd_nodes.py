@@ -1,12 +1,16 @@
 """The native autograd nodes as autograd sees them: saved-tensor hooks reach every saved tensor, a saved input changed
 in place is refused, a gradient that nobody asks for is not computed, an unused output counts as a zero gradient, and
-non-contiguous and expanded upstream gradients give the bytes of contiguous ones."""
+non-contiguous and expanded upstream gradients give the bytes of contiguous ones; other streams and threads, traces, and
+the transforms that have no rule for a node and refuse it."""
 
 from __future__ import annotations
+
+import threading
 
 import pytest
 import torch
 
+from open_transformers_amd.nn import flash_attention as fa
 from open_transformers_amd.nn import functional as F
 from open_transformers_amd.nn.embedding import embedding
 from open_transformers_amd.nn.flash_attention import causal_flash_attention, int8pv_causal_flash_attention
@@ -156,3 +160,82 @@ def test_a_saved_tensor_that_comes_back_changed_is_refused(name):
             for a, b in zip(got, ref):
                 assert torch.equal(_bits(a), _bits(b)), f"saved tensor {which} with other strides"
     torch.cuda.synchronize()
+
+
+def _forward_backward(call, inputs, dy):
+    args = [t.detach().requires_grad_() for t in inputs]
+    y = call(*args)
+    return [y.detach(), *torch.autograd.grad(y, args, dy)]
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_side_streams_and_threads(name):
+    """Forward and backward on another stream, and on two threads with a stream each at once, the memory that the nodes
+    take being used again at once by their own next calls: the bytes of the default stream."""
+    print(f"autograd node {name}: streams and threads", flush=True)
+    call, inputs, _ = _cases()[name]
+    y = call(*inputs)
+    dy = torch.randn(y.shape, device=DEV).to(y.dtype)
+    ref = _forward_backward(call, inputs, dy)
+    torch.cuda.synchronize()
+    got = [[], []]
+
+    def work(out):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(8):
+                out.append([t.clone() for t in _forward_backward(call, inputs, dy)])
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(out,)) for out in got]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for out in got:
+        assert len(out) == 8
+        for run in out:
+            for a, b in zip(run, ref):
+                assert torch.equal(_bits(a), _bits(b))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_transforms_without_a_rule_refuse(name):
+    call, inputs, _ = _cases()[name]
+    args = tuple(t.detach() for t in inputs)
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.vmap(call)(*[torch.stack([a, a]) for a in args])
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.grad(lambda *a: call(*a).sum())(*args)
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError, match="jvp"):
+        call(*[torch.autograd.forward_ad.make_dual(a, a) for a in args])
+
+
+@pytest.mark.parametrize("cache", [False, True])
+@pytest.mark.parametrize("int8pv", [False, True])
+def test_both_attention_nodes_save_the_same_tensors(int8pv, cache):
+    """A checkpoint's first forward may run the Python node and its recompute the native one: the same tensors, in the
+    same order, and the same result."""
+    _, inputs, _ = _cases()["attention"]
+    python = fa._Int8PVFlashAttention if int8pv else fa._CausalFlashAttention
+    native = int8pv_causal_flash_attention if int8pv else causal_flash_attention
+    saved = ([], [])
+
+    def packing(out):
+        def pack(t):
+            out.append(t.detach().clone())
+            return t
+
+        return torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t)
+
+    before = fa.set_score_cache(cache)
+    try:
+        with packing(saved[0]):
+            a = python.apply(*inputs, 32, fa._score_cache_mode(*inputs))
+        with packing(saved[1]):
+            b = native(*inputs, window=32)
+    finally:
+        fa.set_score_cache(before)
+    assert len(saved[0]) == len(saved[1]) == (6 if cache else 5)
+    for x, y in zip((a.detach(), *saved[0]), (b.detach(), *saved[1])):
+        assert x.shape == y.shape and x.dtype == y.dtype and torch.equal(_bits(x), _bits(y))
