@@ -31,10 +31,16 @@
 // LDS once per row (the same operations, so the same bytes), and a logit then
 // costs one LDS read and two or three vector instructions.  Groups of 2048 (or
 // 512) logits that hold a value outside the window (zeros, tiny values, infinities,
-// NaN) are evaluated directly.  Below CE_TABLE_MIN_V logits the table costs what it
-// saves; rows that are not 16-byte aligned and binary32 rows take the general form.
-// Measured at 8192 x 128256 bf16: forward and backward 2000 -> 1389 us (the kernels
-// 1040 -> 600 and 960 -> 766 us; the backward's 4.2 GB at 5.5 TB/s).  The general forward
+// NaN) are evaluated directly.  Rows that are not 16-byte aligned and binary32 rows take
+// the general form, and so do rows below CE_TABLE_MIN_V logits, which pay a table of the
+// same size for less: forward and backward of 8192 rows, table against general form, V
+// 4096 153 against 112 us, 8192 166 / 154, 12288 201 / 232, 16384 231 / 295, 32768 394 /
+// 670, 128256 1421 / 2325.
+// Measured at 8192 x 128256 bf16, forward and backward on one box, before the table form
+// and now: logits N(0, 2^2) 1959 -> 1426 us (589 + 837; the backward's 4.2 GB at 5.0 TB/s);
+// the last 256 of each row -inf 1965 -> 1427; half of each row -inf, in one run 2046 ->
+// 1503, every second logit 1980 -> 1880; zeros 3976 -> 1778; N(0, 1e-3^2), a value outside
+// the window in most groups, 1911 -> 1963 (943 + 968 -> 834 + 1129).  The general forward
 // against one lane per chunk in memory: 4096 x 50257 bf16 637 -> 300 us, 2000 x 5003 bf16
 // 99 -> 34 us, 4096 x 128256 binary32 940 -> 761 us.
 #include "otx_common.h"

@@ -50,6 +50,8 @@ def ce_zloss_forward(logits: torch.Tensor, labels: torch.Tensor, coeff: float):
 
 
 def ce_zloss_backward(logits, labels, stats, grad_ce, grad_z, coeff: float) -> torch.Tensor:
+    """Gradient of ``ce * grad_ce + z * grad_z`` from the forward's ``stats`` (or the caller's own: the stored
+    maximum may lie on either side of the logits)."""
     N, V = _check(logits, labels)
     logits, labels = logits.contiguous(), labels.contiguous()
     g = torch.stack([grad_ce.reshape(()).float(), grad_z.reshape(()).float()]).contiguous()
