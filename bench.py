@@ -770,7 +770,7 @@ def bench_loss(args, torch, dev) -> int:
                    "N": N, "V": V, "coeff": coeff, "bytes_per_step": step_bytes},
         "bit_exact_vs_oracle": verified,
         "phase_ms": {"fwd": round(fwd_ms, 4), "bwd": round(bwd_ms, 4)},
-        "roofline": {"bound": "hbm", "kernel": "ce_bwd_kernel", "achieved": round(bwd_gbs, 1), "peak": 8000.0,
+        "roofline": {"bound": "hbm", "kernel": "ce_bwd_table_kernel", "achieved": round(bwd_gbs, 1), "peak": 8000.0,
                      "unit": "GB/s", "frac": round(bwd_gbs / 8000.0, 4), "traffic": None},
         "cpu_baseline": cpu,
     }

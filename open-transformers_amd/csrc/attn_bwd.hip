@@ -1058,7 +1058,9 @@ static hipError_t launch_bwd_t(int nw, const void* q, const void* k, const void*
   // key blocks are at most two per CU (with the score cache, 16 heads x 1024, D 128: 118 -> 95 us; 16 heads,
   // 4 KV heads x 2048: 886 -> 492; at nkb 1024, 32 heads x 1024: 137 against 139, D 64: 87 against 89), or
   // eight when the scores are recomputed, where the other forms have more to do in one wave (nkb 1024: 188 ->
-  // 181; nkb 2048, window 256: 216 -> 171; nkb 4096: 1158 against 1234).  Sixteen keys per workgroup rather
+  // 181; nkb 2048, window 256: 216 -> 171; nkb 4096: 1158 against 1234).  With the cache and a window the
+  // forms are close beyond that line (four heads a group, D 128, two-key-block form against tile: window 512,
+  // nkb 1024 509 / 550 us, 2048 1016 / 1046, 4096 2006 / 1951; window 256, 306 / 311 and 579 / 571).  Sixteen keys per workgroup rather
   // than 32 up to two key blocks per CU (nkb 512: 95 against 106 us; nkb 1024: 165 against 139), half a block
   // under a window (nkb 128: 20 against 29; nkb 256: 29.2 against 29.1; nkb 512: 51 against 46).
   const bool tile_dkdv = sizeof(T) == 4 || (tile && nkb <= (scache != nullptr ? 2 : 8) * cus);
