@@ -47,7 +47,9 @@ def test_gpu_tile_small(shape, form):
 # block counts over all heads on either side of a limit: (B, H, Hkv, S, D, window)
 LIMITS = [(1, 16, 8, 512, 128, 64), (1, 16, 8, 544, 128, 64), (1, 16, 16, 1024, 64, 0), (1, 16, 16, 1056, 64, 0),
           (1, 16, 16, 1024, 128, 96), (1, 16, 16, 1056, 128, 96), (1, 32, 32, 1024, 128, 0), (1, 32, 32, 1056, 128, 0),
-          (2, 32, 16, 1024, 64, 64), (2, 32, 32, 1024, 128, 64), (2, 33, 33, 1024, 128, 64), (1, 32, 2, 1024, 128, 256)]
+          (2, 32, 16, 1024, 64, 64), (2, 32, 32, 1024, 128, 64), (2, 33, 33, 1024, 128, 64), (1, 32, 2, 1024, 128, 256),
+          # past every limit, an odd number of blocks: the one-wave kernels' paired and head-grouped workgroups
+          (4, 16, 16, 2080, 128, 0), (4, 16, 4, 2080, 128, 0), (4, 16, 4, 2080, 128, 512)]
 
 
 @pytest.mark.parametrize("shape", LIMITS, ids=[f"l{i}" for i in range(len(LIMITS))])
