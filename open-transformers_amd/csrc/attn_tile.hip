@@ -132,7 +132,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_tile_kernel(
   __shared__ float Sp[2][16 * NQ];             // and their steps
 
   const int nqt = S / OTX_BLK, units = nqt * UPB, BH = B * H;
-  const int bid = blockIdx.x;
+  const int bid = blockIdx.x + gridDim.x * blockIdx.y;
+  if (bid >= units * BH) return;  // a grid of several rows (see fwd_tile_grid) may end in spare workgroups
   int unit, bh;
   if (order == 0) {  // longest key ranges first, heads fastest
     unit = units - 1 - bid / BH;
@@ -743,13 +744,21 @@ __global__ __launch_bounds__(256, 2) void attn_dq_tile_kernel(const T* __restric
   }
 }
 
+// A launch holds fewer than 2^32 threads along x. binary32 forwards have no other kernel, and a card's memory holds
+// more workgroups than that (2^23 blocks of 32 rows, D 64, two workgroups each: 69 GB of Q): they go along y too.
+static dim3 fwd_tile_grid(long wgs) {
+  constexpr long most = (1L << 24) - 1;
+  const long y = (wgs + most - 1) / most;
+  return dim3((unsigned)((wgs + y - 1) / y), (unsigned)y);
+}
+
 template <typename T, int D>
 static hipError_t launch_fwd_tile_d(int nq, const void* q, const void* k, const void* v, void* o, float* lse, int B,
                                     int H, int Hkv, int S, int window, float sigma, int order, float* scache,
                                     hipStream_t st) {
-  const unsigned grid = (unsigned)((long)(S / OTX_BLK) * (2 / nq) * B * H);
+  const dim3 grid = fwd_tile_grid((long)(S / OTX_BLK) * (2 / nq) * B * H);
 #define OTX_FWD_TILE(NQ)                                                                                        \
-  hipLaunchKernelGGL((attn_fwd_tile_kernel<T, D, NQ>), dim3(grid), dim3(256), 0, st, (const T*)q, (const T*)k, \
+  hipLaunchKernelGGL((attn_fwd_tile_kernel<T, D, NQ>), grid, dim3(256), 0, st, (const T*)q, (const T*)k, \
                      (const T*)v, (T*)o, lse, B, H, Hkv, S, window, sigma, order, scache, nullptr, nullptr)
   if (nq == 1) OTX_FWD_TILE(1); else OTX_FWD_TILE(2);
 #undef OTX_FWD_TILE
@@ -761,9 +770,9 @@ template <int D>
 static hipError_t launch_fwd_tile_i8_d(int nq, const void* q, const void* k, void* o, float* lse, int B, int H, int Hkv,
                                        int S, int window, float sigma, int order, const int8_t* qvt,
                                        const float* vstep, float* scache, hipStream_t st) {
-  const unsigned grid = (unsigned)((long)(S / OTX_BLK) * (2 / nq) * B * H);
+  const dim3 grid = fwd_tile_grid((long)(S / OTX_BLK) * (2 / nq) * B * H);
 #define OTX_FWD_TILE(NQ)                                                                                    \
-  hipLaunchKernelGGL((attn_fwd_tile_kernel<uint16_t, D, NQ, true>), dim3(grid), dim3(256), 0, st,           \
+  hipLaunchKernelGGL((attn_fwd_tile_kernel<uint16_t, D, NQ, true>), grid, dim3(256), 0, st,           \
                      (const uint16_t*)q, (const uint16_t*)k, nullptr, (uint16_t*)o, lse, B, H, Hkv, S, window, \
                      sigma, order, scache, qvt, vstep)
   if (nq == 1) OTX_FWD_TILE(1); else OTX_FWD_TILE(2);

@@ -108,3 +108,26 @@ def test_gpu_tile_choice_int8pv(shape):
         part = [t[i:i + 1, s].float().cpu().numpy() for t, s in ((q, qs), (k, slice(kv, kv + 1)), (v, slice(kv, kv + 1)))]
         for t, want, n in zip(ref, orc.attn_fwd_int8pv(*part, window=window), NAMES):
             assert_bits_equal(t[i:i + 1, qs].float().cpu().numpy(), want, f"{n} of head group {kv}")
+
+
+def test_more_workgroups_than_a_launch_row_holds():
+    """A binary32 forward of 2^23 + 1 blocks in the sixteen-query form: 2^24 + 2 workgroups of 256 threads, more than one
+    launch holds along x.  Heads from both rows of the grid against a call of those heads alone (they share one KV head)."""
+    H = (1 << 23) + 1
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 160 << 30:
+        pytest.skip("needs 160 GiB of free device memory")
+    print(f"binary32 forward of {H} heads", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    few = [0, 1, 12345, H // 2, H - 2, H - 1]
+    qf, k, v = (torch.randn(1, n, 32, 64, device="cuda", generator=g) for n in (len(few), 1, 1))
+    q = torch.zeros(1, H, 32, 64, device="cuda")
+    q[:, few] = qf
+    o, lse = fa.flash_attention_forward(q, k, v, variant=2)
+    want_o, want_lse = fa.flash_attention_forward(qf, k, v, variant=2)
+    got_o, got_lse = o[:, few], lse[:, few]
+    same = torch.equal(got_o, want_o) and torch.equal(got_lse, want_lse)
+    plain = torch.equal(o[:, 7], o[:, H - 5]) and torch.equal(lse[:, 7], lse[:, H - 5])  # heads of zero queries
+    del q, o, lse
+    torch.cuda.empty_cache()
+    assert same and plain
